@@ -52,9 +52,7 @@ sys.path.insert(0, ROOT)
 METRIC = "GB/s+gates/s at 32q FP64; swap-tests/s batched; Trotter solve time at F≥1-1e-4"
 HBM_PEAK_GBS = 8000.0
 FP32_MATRIX_PEAK_TFLOPS = 157.3
-# FP32 FMA on the VALU without packed instructions: half of the published
-# 157.3 TFLOP/s vector peak, which counts packed FP32 (not used here)
-FP32_VALU_PEAK_TFLOPS = 78.6
+FP64_MATRIX_PEAK_TFLOPS = 78.6
 
 
 def profiled_traffic(name, kernel, qubits=None):
@@ -598,11 +596,10 @@ def run_swap_tests(qe, points, centroids, iterations, warmup, seed):
     ev_ms = qe.qmxTimerEndMs()
     timed_same = bool(np.array_equal(plan.assignments(), final64[0]))
     timed_err = float(np.max(np.abs(2 * plan.p0() - 2 * final64[1])))
-    # the swap-test tile kernel alone: MFMA blocks per launch / device time
+    # the swap-test kernel alone: matrix-core products per launch / device time
     blocks = int(qe.lib.qmxSwapPlanMfmaBlocks(plan.plan))
     tile_ms = float(qe.lib.qmxSwapPlanTimeTiles(plan.plan, 5))
-    tflops = blocks * 4096 / (tile_ms / 1e3) / 1e12
-    valu_tflops = blocks * 2048 / (tile_ms / 1e3) / 1e12
+    tflops = blocks * 2048 / (tile_ms / 1e3) / 1e12
     evals = K.swap_test_amplitude_evaluations(data)
     res = {"swap_tests_per_s": round(tests * iterations / wall, 1), "unit": "swap-tests/s",
            "workload": f"{points} points x {centroids} centroids, q in 4..10 (registers 2q+1 = 9..21 qubits), "
@@ -614,22 +611,21 @@ def run_swap_tests(qe, points, centroids, iterations, warmup, seed):
            "max_distance_error_vs_exact_fp64": dist_err, "max_distance_error_fp64_plan": dist_err64,
            "timed_run_assignments_identical_to_fp64": timed_same, "timed_run_max_distance_diff_vs_fp64": timed_err,
            "autotune_timings": timings, "rows_per_tile": rows, "tiles": plan.num_tiles(),
-           "method": "closed-form evaluation of the circuit's ancilla-0 amplitudes (a_x b_y + a_y b_x)/2 over all "
-                     "4^q index pairs, from the encoded registers; the CSWAP ladder and the Hadamards are not applied "
-                     "gate by gate (the gate-level circuit is the oracle's and the cpu_reference_method's)",
-           "roofline": {"bound": "valu", "kernel": "kSwapTilesMfma (32x32x2 FP32 MFMA blocks of the amplitude matrix, "
-                                                   "squares summed on the VALU)",
-                        "achieved": round(valu_tflops, 2), "peak": FP32_VALU_PEAK_TFLOPS, "unit": "TFLOP/s",
-                        "frac": round(valu_tflops / FP32_VALU_PEAK_TFLOPS, 4),
-                        "traffic": profiled_traffic("qkmeans_swap", "kSwapTilesMfma")[0],
-                        "traffic_source": profiled_traffic("qkmeans_swap", "kSwapTilesMfma")[1],
-                        "avg_launch_ms": round(tile_ms, 4), "mfma_blocks_per_launch": blocks,
-                        "valu_flops_per_block": 2048, "mfma_tflops": round(tflops, 2),
-                        "mfma_frac": round(tflops / FP32_MATRIX_PEAK_TFLOPS, 4),
-                        "note": "registers are L2-resident (19 MB of FP32 point registers), so HBM does not bound it; "
-                                "the matrix cores form each 32x32 block of amplitudes (4096 flops) and the VALU "
-                                "squares and sums its 1024 entries (one FP32 FMA each, 2048 flops), so the VALU, "
-                                "at its non-packed FP32 rate (packed FP32 is not used), is the bound"}}
+           "method": "closed form of the circuit's P(ancilla = 0) from the encoded registers: the sum over all 4^q "
+                     "index pairs of the squared ancilla-0 amplitudes (a_x b_y + a_y b_x)/2 factors into "
+                     "(|a|^2 |b|^2 + <a,b>^2)/2, whose inner products are one FP64 matrix product; the CSWAP ladder "
+                     "and the Hadamards are not applied gate by gate (the gate-level circuit is the oracle's and the "
+                     "cpu_reference_method's)",
+           "roofline": {"bound": "mfma", "kernel": "kOverlap (inner products of 16 points x 16 centroids on "
+                                                   "v_mfma_f64_16x16x4f64, P0 and assignment)",
+                        "achieved": round(tflops, 2), "peak": FP64_MATRIX_PEAK_TFLOPS, "unit": "TFLOP/s",
+                        "frac": round(tflops / FP64_MATRIX_PEAK_TFLOPS, 4),
+                        "traffic": profiled_traffic("qkmeans_swap", "kOverlap")[0],
+                        "traffic_source": profiled_traffic("qkmeans_swap", "kOverlap")[1],
+                        "avg_launch_ms": round(tile_ms, 4), "mfma_products_per_launch": blocks,
+                        "note": "16x16x4 FP64 matrix products (2048 flops each); registers are cache-resident (19 MB "
+                                "of FP32 point registers), so HBM does not bound the launch; at these sizes a "
+                                "wave's chain of loads and products and the launch itself take most of the time"}}
     plan.close()
     p64.close()
     return res, data

@@ -220,14 +220,14 @@ typedef struct qmxSwapPlan qmxSwapPlan;
 qmxSwapPlan *qmxSwapPlanCreate(int numPoints, const int *pointQubits, const double *points, int numCentroids,
                                int maxQubits, const double *centroids, int precision);
 void qmxSwapPlanDestroy(qmxSwapPlan *plan);
-/* times candidate tile shapes per register size on the device, keeps the fastest;
- * returns the number of timings made */
+/* times candidate splits of the registers' rows over waves per register size on
+ * the device, keeps the fastest; returns the number of timings made */
 int qmxSwapPlanAutotune(qmxSwapPlan *plan);
 int qmxSwapPlanRowsPerTile(const qmxSwapPlan *plan, int qubits);
 int qmxSwapPlanNumTiles(const qmxSwapPlan *plan);
-/* 32x32 amplitude blocks an iteration forms on the matrix cores (FP32 plans; 0 for FP64) */
+/* 16x16x4 matrix-core products an iteration makes */
 long long qmxSwapPlanMfmaBlocks(const qmxSwapPlan *plan);
-/* device time of one swap-test launch (ms), averaged over `launches` (overwrites the partials) */
+/* device time of one swap-test launch (ms), averaged over `launches` (the plan's results stay) */
 double qmxSwapPlanTimeTiles(qmxSwapPlan *plan, int launches);
 void qmxSwapPlanRun(qmxSwapPlan *plan, int iterations, int useGraph);
 /* P(ancilla = 0) of the last iteration's tests, numPoints x numCentroids */

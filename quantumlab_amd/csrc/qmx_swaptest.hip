@@ -15,23 +15,21 @@
 //    left) (the reference's recursion), then each amplitude as the product of
 //    cos/sin(theta/2) along its path — the state the Ry tree prepares, in
 //    O(2^q) instead of 2^q gates of O(2^(2q+1)) each.
-//  * kSwapTiles: after H and the two encodings the register is |+>|a>|b>; the
+//  * kOverlap: after H and the two encodings the register is |+>|a>|b>; the
 //    CSWAP ladder and the final H leave ancilla-0 amplitudes
-//    (a_x b_y + a_y b_x)/2. The kernel evaluates every one of those 2^(2q)
-//    amplitudes (nothing of the 2^(2q+1)-amplitude register is stored) and
-//    reduces |amp|^2 in FP64. Work is a static list of tiles (test, first
-//    row, rows) over which a persistent grid strides — no atomics, every wave
-//    exits when the list ends; the rows per tile are chosen per q by an
-//    autotuner that times each candidate on the device.
-//  * one k-means iteration = swap tiles -> per-test P0 -> argmax assignment ->
-//    centroid means -> re-encoded centroids, captured once as a hipGraph and
+//    (a_x b_y + a_y b_x)/2, so P(anc = 0) = 1/4 sum_xy (a_x b_y + a_y b_x)^2.
+//    The registers are real, and the double sum factors exactly into
+//    (|a|^2 |b|^2 + <a, b>^2)/2: three sums of 2^q products instead of one of
+//    2^(2q) squares. The inner products of 16 points with 16 centroids are one
+//    FP64 matrix product over the registers' rows.
+//  * one k-means iteration = inner products, P0 and argmax assignment in one
+//    launch -> partial centroid sums -> centroid means, normalised and
+//    re-encoded at every size; three launches, captured once as a hipGraph and
 //    replayed.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
-#include <cstring>
 #include <limits>
-#include <type_traits>
 #include <vector>
 
 #include "qmx_device.h"
@@ -43,33 +41,40 @@ namespace {
 
 constexpr int kMinQ = 1, kMaxQ = 12;
 
+// one workgroup's points: up to 16 * (4 / split) consecutive entries of the
+// size-ordered point list, all of register size q; `split` waves share a
+// register's rows
 struct Tile {
-    int test;   // point * numCentroids + centroid
-    int x0;     // first row
-    int nx;     // rows
-    int pad;
+    int first, count;
+    int q;
+    int split;
 };
 
 // ---- amplitude encoding -----------------------------------------------------
-// vectors: packed real FP64 inputs (length 2^q each, offsets in off[]); out:
-// the encoded states in the storage precision T (same packing). The encoding
-// is O(2^q) per vector, so it is computed in FP64 for both storage precisions
-// and each amplitude is rounded once when stored. One workgroup per vector;
-// LDS holds the magnitudes and the cos/sin factors of the 2^q - 1 angles.
+// cos and sin of half the reference's angle 2 atan2(s, c): c/h and s/h with
+// h = hypot(c, s). The quotients replace an atan2, a cosine and a sine per node
+// (the levels of the tree are a serial chain, so their latency is the kernel's
+// time: 54 us for one 1024-entry vector before). Where h is zero, not finite or
+// so small that it has lost digits, the angle itself is used.
+__device__ __forceinline__ void angleFactors(double c, double s, double &cs, double &sn) {
+    const double h = hypot(c, s);
+    if (h > 1e-280 && h < std::numeric_limits<double>::infinity()) {
+        cs = c / h;
+        sn = s / h;
+    } else {
+        const double theta = 2.0 * atan2(s, c);
+        cs = cos(theta / 2.0);
+        sn = sin(theta / 2.0);
+    }
+}
+
+// The encoding tree over mag[0 .. 2^q) (LDS, overwritten), one workgroup; cs, sn:
+// 2^q doubles each in LDS. Writes the encoded state to o (storage precision)
+// and its squared norm as stored to *norm2 (nullptr: not wanted).
 template <typename T>
-__global__ void __launch_bounds__(kBlock) kAEState(const double *__restrict__ vecs, const long long *__restrict__ off,
-                                                   const int *__restrict__ qs, T *__restrict__ out, int count) {
-    extern __shared__ unsigned char smem[];
-    const int v = blockIdx.x;
-    if (v >= count) return;
-    const int q = qs[v];
+__device__ __forceinline__ void encodeTree(double *mag, double *cs, double *sn, int q, T *__restrict__ o,
+                                           double *norm2) {
     const int D = 1 << q;
-    double *mag = reinterpret_cast<double *>(smem);  // D values
-    double *cs = mag + D;                            // D-1 cos(theta/2), level-major like the reference's list
-    double *sn = cs + D;                             // D-1 sin(theta/2)
-    const double *in = vecs + off[v];
-    for (int i = threadIdx.x; i < D; i += kBlock) mag[i] = in[i];
-    __syncthreads();
     // level l: pairs (left = k 2^(l+1), right = left + 2^l) of the running
     // magnitudes; angle index = D - 2^(q-l) + k (AmplitudeEncodeCuda.cu:126-129)
     for (int l = 0; l < q; ++l) {
@@ -78,9 +83,7 @@ __global__ void __launch_bounds__(kBlock) kAEState(const double *__restrict__ ve
         for (int k = threadIdx.x; k < pairs; k += kBlock) {
             const int left = k << (l + 1), right = left + (1 << l);
             const double c = mag[left], s = mag[right];
-            const double theta = 2.0 * atan2(s, c);
-            cs[base + k] = cos(theta / 2.0);
-            sn[base + k] = sin(theta / 2.0);
+            angleFactors(c, s, cs[base + k], sn[base + k]);
             if (pairs != 1) {
                 // magnitudes at or below the arithmetic's epsilon are zeroed, as
                 // the reference does with _QL_FLT_EPSILON (QLFloat.h:120,139: the
@@ -92,7 +95,7 @@ __global__ void __launch_bounds__(kBlock) kAEState(const double *__restrict__ ve
         __syncthreads();
     }
     // amplitude of basis state x: product over levels of cos (bit 0) / sin (bit 1)
-    T *o = out + off[v];
+    Acc acc[1];
     for (int x = threadIdx.x; x < D; x += kBlock) {
         double amp = 1.0;
         for (int l = 0; l < q; ++l) {
@@ -100,225 +103,165 @@ __global__ void __launch_bounds__(kBlock) kAEState(const double *__restrict__ ve
             amp *= ((x >> l) & 1) ? sn[idx] : cs[idx];
         }
         o[x] = (T)amp;
+        const double stored = (double)(T)amp;
+        acc[0].add(stored * stored);
     }
-}
-
-// centroid registers at every size: cent (C x 2^maxQ, FP64) truncated to 2^q
-// and L2-normalised into cin (FP64, packed per (q, c))
-__global__ void __launch_bounds__(kBlock) kCentroidInputs(const double *__restrict__ cent, int maxQ, int C, int qLo,
-                                                          int qHi, const long long *__restrict__ cOff,
-                                                          double *__restrict__ cin) {
-    const int q = qLo + blockIdx.x / C, c = blockIdx.x % C;
-    if (q > qHi) return;
-    const int D = 1 << q;
-    const double *src = cent + (size_t)c * (1 << maxQ);
-    Acc acc[1];
-    for (int i = threadIdx.x; i < D; i += kBlock) acc[0].add(src[i] * src[i]);
+    if (!norm2) return;  // the same for every thread
     double tot[1];
     blockReduce<1>(acc, tot);
-    __shared__ double norm;
-    if (threadIdx.x == 0) norm = tot[0] > 0 ? 1.0 / sqrt(tot[0]) : 0.0;
-    __syncthreads();
-    double *dst = cin + cOff[blockIdx.x];
-    for (int i = threadIdx.x; i < D; i += kBlock) dst[i] = src[i] * norm;
+    if (threadIdx.x == 0) *norm2 = tot[0];
 }
 
-// ---- swap-test tiles ------------------------------------------------------------
-// Tile (test, x0, nx): rows x in [x0, x0+nx), all columns y. A lane owns
-// CPL = clamp(D/256, 1, 4) columns per pass (registers a_y, b_y); lanes split
-// into RG = 256/TPR row groups of TPR = min(D/CPL, 256) lanes, each walking
-// its rows with a_x, b_x read from LDS (uniform within the row group). Sums
-// of 8 rows are FP32, accumulated in FP64 with compensation.
-constexpr int kMaxTileRows = 1024;
+// vectors: packed real FP64 inputs (length 2^q each, offsets in off[]); out:
+// the encoded states in the storage precision T (same packing), norm2 (may be
+// nullptr) their squared norms. The encoding is O(2^q) per vector, so it is
+// computed in FP64 for both storage precisions and each amplitude is rounded
+// once when stored. One workgroup per vector; LDS holds the magnitudes and the
+// cos/sin factors of the 2^q - 1 angles.
+template <typename T>
+__global__ void __launch_bounds__(kBlock) kAEState(const double *__restrict__ vecs, const long long *__restrict__ off,
+                                                   const int *__restrict__ qs, T *__restrict__ out,
+                                                   double *__restrict__ norm2, int count) {
+    extern __shared__ unsigned char smem[];
+    const int v = blockIdx.x;
+    if (v >= count) return;
+    const int q = qs[v];
+    const int D = 1 << q;
+    double *mag = reinterpret_cast<double *>(smem);
+    const double *in = vecs + off[v];
+    for (int i = threadIdx.x; i < D; i += kBlock) mag[i] = in[i];
+    __syncthreads();
+    encodeTree<T>(mag, mag + D, mag + 2 * D, q, out + off[v], norm2 ? norm2 + v : nullptr);
+}
+
+// ---- inner products, P0 and assignment ----------------------------------------
+// P0[p][c] = (|a|^2 |b|^2 + <a, b>^2)/2 and each point's best centroid (largest
+// P0, ties to the lowest index). A wave takes 16 points of one size and 16
+// centroids at a time on v_mfma_f64_16x16x4f64: lane l holds point l%16 and
+// centroid l%16 at row 4 (l/16) + k of each run of 16 rows, k = 0..3 in four
+// products, so a lane reads four consecutive rows at once (the order of the
+// rows in the sum is free). FP32 registers are widened first: every product and
+// sum is FP64. The result's lane l holds points l/16 + 4v, centroid l%16.
+//
+// What bounds it: the registers are read once per iteration (FP32, 4096 points
+// of 16..1024 amplitudes: 4.8 MB, from the caches) and the products take ~1 us
+// of the matrix cores, so it is the latency of a wave's serial chain of loads
+// and products; `split` waves divide a register's rows (4 from 256 rows, 2 from
+// 64) and their sums meet in LDS. Replaces 4^q amplitudes formed on the matrix
+// cores and squared on the VALU (490 us a launch at that size; bound there by
+// the squares).
+constexpr int kWaves = kBlock / 64;
+typedef double d4v __attribute__((ext_vector_type(4)));
+
+// rows i .. i+3 of a register of D rows, zeros past its end. `vec`: registers
+// start at multiples of 4 rows, so four rows are one aligned access
+template <typename T>
+__device__ __forceinline__ d4v rows4(const T *__restrict__ a, int i, int D, bool vec) {
+    typedef T V __attribute__((ext_vector_type(4)));
+    if (vec) {
+        if (i >= D) return d4v{0, 0, 0, 0};
+        // 16 B units: FP64 offsets of 4 rows are 32 B apart
+        const V v = *reinterpret_cast<const V *>(a + i);
+        return d4v{(double)v.x, (double)v.y, (double)v.z, (double)v.w};
+    }
+    d4v r;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) r[k] = i + k < D ? (double)a[i + k] : 0.0;
+    return r;
+}
 
 template <typename T>
-__global__ void __launch_bounds__(kBlock) kSwapTiles(const Tile *__restrict__ tiles, int numTiles,
-                                                     const T *__restrict__ pointAE, const long long *__restrict__ pOff,
-                                                     const int *__restrict__ pQ, const T *__restrict__ centAE,
-                                                     const long long *__restrict__ cOff, int C, int qLo,
-                                                     double *__restrict__ partial) {
-    __shared__ T lx[2][kMaxTileRows];  // a_x, b_x of the tile's rows
-    for (int w = blockIdx.x; w < numTiles; w += gridDim.x) {
-        const Tile t = tiles[w];
-        const int p = t.test / C, c = t.test % C;
-        const int q = pQ[p];
-        const int D = 1 << q;
-        const T *a = pointAE + pOff[p];
-        const T *b = centAE + cOff[(q - qLo) * C + c];
-        __syncthreads();
-        for (int i = threadIdx.x; i < t.nx; i += kBlock) {
-            lx[0][i] = a[t.x0 + i];
-            lx[1][i] = b[t.x0 + i];
-        }
-        __syncthreads();
-        const int CPL = D >= 4 * kBlock ? 4 : (D >= kBlock ? D / kBlock : 1);
-        const int TPR = D / CPL < kBlock ? D / CPL : kBlock;
-        const int RG = kBlock / TPR;
-        const int col0 = threadIdx.x % TPR, rg = threadIdx.x / TPR;
-        Acc acc[1];
-        for (int y0 = col0; y0 < D; y0 += CPL * TPR) {
-            T ay[4], by[4];
+__global__ void __launch_bounds__(kBlock) kOverlap(const Tile *__restrict__ tiles, const int *__restrict__ order,
+                                                   const T *__restrict__ pointAE, const long long *__restrict__ pOff,
+                                                   const double *__restrict__ pNorm, const T *__restrict__ centAE,
+                                                   const long long *__restrict__ cOff,
+                                                   const double *__restrict__ cNorm, int C, int qLo, int vec,
+                                                   double *__restrict__ p0, int *__restrict__ assign) {
+    __shared__ d4v part[kWaves][64];
+    const Tile t = tiles[blockIdx.x];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int col = lane & 15, kq = lane >> 4;
+    const int D = 1 << t.q;
+    const int mine = wave / t.split, share = wave % t.split;   // point group, part of the rows
+    const int count = min(16, t.count - 16 * mine);            // may be <= 0: a wave without points
+    const int nx = D / t.split < 16 ? 16 : D / t.split;        // split > 1 only from 64 rows
+    const int *ids = order + t.first + 16 * mine;
+    const int pm = col < count ? ids[col] : -1;
+    const T *a = pm >= 0 ? pointAE + pOff[pm] : pointAE;
+    // best centroid so far of points l/16 + 4v (every lane of the 16 alike)
+    double best[4];
+    int bestC[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int y = y0 + k * TPR;
-                const bool ok = k < CPL && y < D;
-                ay[k] = ok ? a[y] : (T)0;
-                by[k] = ok ? b[y] : (T)0;
-            }
-            T s8 = (T)0;
-            int inChunk = 0;
-            for (int r = rg; r < t.nx; r += RG) {
-                const T ax = lx[0][r], bx = lx[1][r];
-                T v = ax * by[0] + ay[0] * bx;
-                T s = v * v;
-                if (CPL > 1) {
-#pragma unroll
-                    for (int k = 1; k < 4; ++k) {
-                        if (k < CPL) {
-                            v = ax * by[k] + ay[k] * bx;
-                            s += v * v;
-                        }
-                    }
-                }
-                s8 += s;
-                if (++inChunk == 8) {
-                    acc[0].add((double)s8);
-                    s8 = (T)0;
-                    inChunk = 0;
-                }
-            }
-            acc[0].add((double)s8);
-        }
-        double tot[1];
-        blockReduce<1>(acc, tot);
-        if (threadIdx.x == 0) partial[w] = tot[0];
+    for (int v = 0; v < 4; ++v) {
+        best[v] = -std::numeric_limits<double>::infinity();
+        bestC[v] = 0;
     }
-}
-
-// FP32 plans: the same sums on the matrix cores, one wave per tile. A tile's
-// rows x0 .. x0+nx (nx a multiple of 32, or the whole register when D < 32)
-// against all columns, in 32 x 32 blocks of M[x][y] = a_x b_y + b_x a_y (twice
-// the ancilla-0 amplitude) from one v_mfma_f32_32x32x2f32 each:
-//   A (32 x 2): lane l holds A[l%32][l/32] = (l < 32 ? a : b)[x0 + l%32]
-//   B (2 x 32): lane l holds B[l/32][l%32] = (l < 32 ? b : a)[y0 + l%32]
-// so K = 2 is exactly the two products (and M is symmetric, so only blocks on
-// or above the diagonal are formed). Each of the 16 accumulator values per
-// lane is one element of the block; their squares are summed in FP32 per column
-// block (1, 2, 4 or 8 row blocks share one B operand) and in FP64 across blocks.
-constexpr int kMaxRowBlocks = 8;  // 256 rows per tile
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-
-// one tile of NB row blocks. M is symmetric (M[x][y] = M[y][x]), so the sum
-// over all blocks is the diagonal blocks once plus the blocks above the
-// diagonal twice: row block X only meets column blocks Y >= X.
-template <int NB>
-__device__ __forceinline__ double swapTileMfma(const float *sx, const float *sy, int x0, int D, int r) {
-    const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float av[NB];
+    for (int c0 = 0; c0 < C; c0 += 16) {
+        const int c = c0 + col;
+        const T *b = centAE + cOff[(t.q - qLo) * C + (c < C ? c : C - 1)];
+        d4v acc = {0, 0, 0, 0};
+        if (count > 0)
+            for (int s = share * nx; s < (share + 1) * nx; s += 16) {
+                const int i = s + 4 * kq;
+                const d4v x = pm >= 0 ? rows4<T>(a, i, D, vec) : d4v{0, 0, 0, 0};
+                const d4v y = rows4<T>(b, i, D, vec);
 #pragma unroll
-    for (int k = 0; k < NB; ++k) {
-        const int x = x0 + 32 * k + r;
-        av[k] = x < D ? sx[x] : 0.f;
-    }
-    double acc = 0.0;
-    float bv = x0 + r < D ? sy[x0 + r] : 0.f;
-    for (int y0 = x0; y0 < D; y0 += 32) {
-        const int yn = y0 + 32 + r;
-        const float bnext = yn < D ? sy[yn] : 0.f;  // next column block, loaded ahead
-        float s = 0.f;
-        if (y0 >= x0 + 32 * (NB - 1)) {
-            // every row block of the tile is at or left of this column block
-            floatx16 d[NB];
-#pragma unroll
-            for (int k = 0; k < NB; ++k) d[k] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[k], bv, zero, 0, 0, 0);
-#pragma unroll
-            for (int k = 0; k < NB; ++k) {
-                float sk = 0.f;
-#pragma unroll
-                for (int v = 0; v < 16; ++v) sk = fmaf(d[k][v], d[k][v], sk);
-                s += (y0 == x0 + 32 * k) ? sk : 2.f * sk;
+                for (int k = 0; k < 4; ++k) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x[k], y[k], acc, 0, 0, 0);
             }
-        } else {
-            // the tile's first column blocks: only row blocks X <= Y
+        if (t.split > 1) {  // the same for the whole workgroup
+            part[wave][lane] = acc;
+            __syncthreads();
+            if (share == 0)
+                for (int k = 1; k < t.split; ++k) acc += part[wave + k][lane];
+            __syncthreads();
+        }
+        if (share != 0 || count <= 0) continue;
+        const double bb = c < C ? cNorm[(t.q - qLo) * C + c] : 0.0;
 #pragma unroll
-            for (int k = 0; k < NB; ++k) {
-                if (y0 >= x0 + 32 * k) {
-                    const floatx16 d = __builtin_amdgcn_mfma_f32_32x32x2f32(av[k], bv, zero, 0, 0, 0);
-                    float sk = 0.f;
+        for (int v = 0; v < 4; ++v) {
+            const int row = kq + 4 * v;
+            const int p = row < count ? ids[row] : -1;
+            double val = -std::numeric_limits<double>::infinity();
+            int at = c;
+            if (p >= 0 && c < C) {
+                val = 0.5 * (pNorm[p] * bb + acc[v] * acc[v]);
+                p0[(size_t)p * C + c] = val;
+                // a P0 that is not a number is never larger than another, and as
+                // the first one it stays
+                if (!(val == val)) val = c == 0 ? std::numeric_limits<double>::infinity()
+                                                : -std::numeric_limits<double>::infinity();
+            }
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) sk = fmaf(d[v], d[v], sk);
-                    s += (y0 == x0 + 32 * k) ? sk : 2.f * sk;
+            for (int off = 1; off < 16; off <<= 1) {
+                const double ov = __shfl_xor(val, off, 64);
+                const int oc = __shfl_xor(at, off, 64);
+                if (ov > val || (ov == val && oc < at)) {
+                    val = ov;
+                    at = oc;
                 }
             }
-        }
-        acc += (double)s;
-        bv = bnext;
-    }
-    return acc;
-}
-
-__global__ void __launch_bounds__(kBlock) kSwapTilesMfma(const Tile *__restrict__ tiles, int numTiles,
-                                                         const float *__restrict__ pointAE,
-                                                         const long long *__restrict__ pOff, const int *__restrict__ pQ,
-                                                         const float *__restrict__ centAE,
-                                                         const long long *__restrict__ cOff, int C, int qLo,
-                                                         double *__restrict__ partial) {
-    const int lane = threadIdx.x & 63, r = lane & 31, hi = lane >> 5;
-    const int wavesTotal = gridDim.x * (kBlock / 64);
-    for (int w = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); w < numTiles; w += wavesTotal) {
-        const Tile t = tiles[w];
-        const int p = t.test / C, c = t.test % C;
-        const int q = pQ[p];
-        const int D = 1 << q;
-        const float *a = pointAE + pOff[p];
-        const float *b = centAE + cOff[(q - qLo) * C + c];
-        const float *sx = hi ? b : a;  // rows
-        const float *sy = hi ? a : b;  // columns
-        const int nb = (t.nx + 31) >> 5;
-        double acc;
-        switch (nb) {  // wave-uniform
-            case 1: acc = swapTileMfma<1>(sx, sy, t.x0, D, r); break;
-            case 2: acc = swapTileMfma<2>(sx, sy, t.x0, D, r); break;
-            case 4: acc = swapTileMfma<4>(sx, sy, t.x0, D, r); break;
-            default: acc = swapTileMfma<8>(sx, sy, t.x0, D, r); break;
-        }
-        for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 64);
-        if (lane == 0) partial[w] = acc;
-    }
-}
-
-// P0 of each test: (1/4) sum of its tiles' partials (tiles of a test are contiguous)
-__global__ void __launch_bounds__(kBlock) kSwapFinish(const double *__restrict__ partial, const int *__restrict__ tStart,
-                                                      const int *__restrict__ tCount, int numTests, double *__restrict__ p0) {
-    const int t = blockIdx.x * kBlock + threadIdx.x;
-    if (t >= numTests) return;
-    Acc acc;
-    const int s = tStart[t], n = tCount[t];
-    for (int i = 0; i < n; ++i) acc.add(partial[s + i]);
-    p0[t] = 0.25 * acc.value();
-}
-
-// assignment: the centroid of largest P0 (= largest overlap); ties -> lowest index
-__global__ void __launch_bounds__(kBlock) kAssign(const double *__restrict__ p0, int P, int C, int *__restrict__ assign) {
-    const int p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= P) return;
-    int best = 0;
-    double bv = p0[(size_t)p * C];
-    for (int c = 1; c < C; ++c) {
-        const double v = p0[(size_t)p * C + c];
-        if (v > bv) {
-            bv = v;
-            best = c;
+            if (val > best[v]) {
+                best[v] = val;
+                bestC[v] = at;
+            }
         }
     }
-    assign[p] = best;
+    if (share != 0 || col != 0) return;
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        if (kq + 4 * v < count) assign[ids[kq + 4 * v]] = bestC[v];
 }
 
-// centroid means over assigned points, coordinate by coordinate (points only
-// contribute their own 2^q coordinates); empty clusters keep their centroid.
-// Stage 1: one workgroup per (centroid, 256-coordinate slice, chunk of points)
-// writes the chunk's sum and count; stage 2 adds the chunks in order. FP64,
-// deterministic.
+// ---- centroid means --------------------------------------------------------------
+// means over assigned points, coordinate by coordinate (points only contribute
+// their own 2^q coordinates); empty clusters keep their centroid. Stage 1
+// (kCentroidPartial): one workgroup per (centroid, 256-coordinate slice, chunk
+// of points) writes the chunk's sum and count; stage 2 (kCentroidUpdate) adds
+// the chunks in order. FP64, deterministic.
+// The chunk's members are first listed in LDS, 256 assignments at a time, so
+// their coordinates are loads that do not wait for one another (a loop over all
+// points that loaded each member's coordinates in turn took 30 us at 4096
+// points and 16 centroids).
 constexpr int kMeanChunks = 16;
 
 __global__ void __launch_bounds__(kBlock) kCentroidPartial(const double *__restrict__ pointsV,
@@ -326,24 +269,60 @@ __global__ void __launch_bounds__(kBlock) kCentroidPartial(const double *__restr
                                                            const int *__restrict__ pQ, const int *__restrict__ assign,
                                                            int P, int C, int maxQ, double *__restrict__ sums,
                                                            int *__restrict__ counts, int *__restrict__ members) {
+    __shared__ long long listOff[kBlock];
+    __shared__ int listD[kBlock];
+    __shared__ int waveHits[kWaves], waveMembers[kWaves];
     const int dim = 1 << maxQ;
     const int slices = dim / kBlock > 0 ? dim / kBlock : 1;
     const int chunk = blockIdx.x % kMeanChunks;
     const int cs = blockIdx.x / kMeanChunks;
     const int c = cs / slices;
-    const int j = (cs % slices) * kBlock + threadIdx.x;
+    const int j0 = (cs % slices) * kBlock, j = j0 + threadIdx.x;
     const int per = (P + kMeanChunks - 1) / kMeanChunks;
     const int p0 = chunk * per, p1 = p0 + per < P ? p0 + per : P;
     if (c >= C) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     double sum = 0.0;
     int cnt = 0, mem = 0;
-    for (int p = p0; p < p1; ++p) {
-        if (assign[p] != c) continue;
-        ++mem;
-        if (j < (1 << pQ[p])) {
-            sum += pointsV[pOff[p] + j];
-            ++cnt;
+    for (int base = p0; base < p1; base += kBlock) {
+        const int p = base + threadIdx.x;
+        const bool in = p < p1 && assign[p] == c;
+        const int D = in ? 1 << pQ[p] : 0;
+        const bool hit = D > j0;  // has coordinates in this slice
+        const unsigned long long hits = __ballot(hit);
+        const unsigned long long ins = __ballot(in);
+        if (lane == 0) {
+            waveHits[wave] = __popcll(hits);
+            waveMembers[wave] = __popcll(ins);
         }
+        __syncthreads();
+        int at = __popcll(hits & ((1ull << lane) - 1ull)), total = 0;
+        for (int w = 0; w < kWaves; ++w) {
+            if (w < wave) at += waveHits[w];
+            total += waveHits[w];
+            mem += waveMembers[w];
+        }
+        if (hit) {
+            listOff[at] = pOff[p];
+            listD[at] = D;
+        }
+        __syncthreads();
+        for (int i = 0; i < total; i += 8) {
+            double v[8];
+            bool ok[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                ok[k] = i + k < total && j < listD[i + k < total ? i + k : 0];
+                v[k] = ok[k] ? pointsV[listOff[i + k] + j] : 0.0;
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (ok[k]) {
+                    sum += v[k];
+                    ++cnt;
+                }
+        }
+        __syncthreads();
     }
     if (j < dim) {
         const size_t o = ((size_t)chunk * C + c) * dim + j;
@@ -353,23 +332,57 @@ __global__ void __launch_bounds__(kBlock) kCentroidPartial(const double *__restr
     if (threadIdx.x == 0 && (cs % slices) == 0) members[chunk * C + c] = mem;
 }
 
-__global__ void __launch_bounds__(kBlock) kCentroidCombine(const double *__restrict__ sums, const int *__restrict__ counts,
-                                                           const int *__restrict__ members, int C, int maxQ,
-                                                           double *__restrict__ cent) {
-    const int dim = 1 << maxQ;
-    const int slices = dim / kBlock > 0 ? dim / kBlock : 1;
-    const int c = blockIdx.x / slices;
-    const int j = (blockIdx.x % slices) * kBlock + threadIdx.x;
-    if (c >= C || j >= dim) return;
-    double sum = 0.0;
-    int cnt = 0, mem = 0;
-    for (int k = 0; k < kMeanChunks; ++k) {
-        const size_t o = ((size_t)k * C + c) * dim + j;
-        sum += sums[o];
-        cnt += counts[o];
-        mem += members[k * C + c];
+// One workgroup per (register size q, centroid c): the new centroid's first 2^q
+// coordinates (the mean where points were assigned, else the old coordinate;
+// chunks = 0: the centroids as they are), L2-normalised and encoded at size q,
+// with the squared norm of the stored register. The workgroup of the largest
+// size also writes the new coordinates to `cent`: only coordinates that have
+// members, which the other sizes' workgroups do not read from there.
+template <typename T>
+__global__ void __launch_bounds__(kBlock) kCentroidUpdate(const double *__restrict__ sums,
+                                                          const int *__restrict__ counts,
+                                                          const int *__restrict__ members, int chunks, int maxQ, int C,
+                                                          int qLo, int qHi, const long long *__restrict__ cOff,
+                                                          double *cent, T *__restrict__ centAE,
+                                                          double *__restrict__ cNorm) {
+    extern __shared__ unsigned char smem[];
+    __shared__ double norm;
+    const int q = qLo + blockIdx.x / C, c = blockIdx.x % C;
+    const int D = 1 << q;
+    const size_t dim = (size_t)1 << maxQ;
+    double *mag = reinterpret_cast<double *>(smem);
+    double *cc = cent + (size_t)c * dim;
+    int mem = 0;
+    for (int k = 0; k < chunks; ++k) mem += members[k * C + c];
+    Acc acc[1];
+    for (int i = threadIdx.x; i < D; i += kBlock) {
+        double sum = 0.0;
+        int cnt = 0;
+        if (mem > 0) {
+#pragma unroll 4
+            for (int k = 0; k < chunks; ++k) {
+                const size_t o = ((size_t)k * C + c) * dim + i;
+                sum += sums[o];
+                cnt += counts[o];
+            }
+        }
+        double v;
+        if (cnt > 0) {
+            v = sum / cnt;
+            if (q == qHi) cc[i] = v;
+        } else {
+            v = cc[i];
+        }
+        mag[i] = v;
+        acc[0].add(v * v);
     }
-    if (mem > 0 && cnt > 0) cent[(size_t)c * dim + j] = sum / cnt;
+    double tot[1];
+    blockReduce<1>(acc, tot);
+    if (threadIdx.x == 0) norm = tot[0] > 0 ? 1.0 / sqrt(tot[0]) : 0.0;
+    __syncthreads();
+    for (int i = threadIdx.x; i < D; i += kBlock) mag[i] *= norm;
+    __syncthreads();
+    encodeTree<T>(mag, mag + D, mag + 2 * D, q, centAE + cOff[blockIdx.x], cNorm + blockIdx.x);
 }
 
 }  // namespace
@@ -380,17 +393,18 @@ struct SwapPlanImpl {
     int prec;
     int P, C, maxQ, qLo, qHi;
     std::vector<int> hQ;
+    int sizeCount[kMaxQ + 1] = {0};    // points of each register size
     std::vector<long long> hPOff, hCOff;
-    void *pointsV = nullptr, *pointAE = nullptr, *cent = nullptr, *centIn = nullptr, *centAE = nullptr;
+    void *pointsV = nullptr, *pointAE = nullptr, *cent = nullptr, *centAE = nullptr;
     long long *pOff = nullptr, *cOff = nullptr;
-    int *pQ = nullptr, *cQ = nullptr, *assign = nullptr, *tStart = nullptr, *tCount = nullptr;
-    Tile *tiles = nullptr;
-    double *partial = nullptr, *p0 = nullptr;
+    int *pQ = nullptr, *assign = nullptr;
+    int *order = nullptr;      // points by register size, largest first
+    Tile *tiles = nullptr;     // room for every choice of rowsPerTile
+    double *pNorm = nullptr, *cNorm = nullptr, *p0 = nullptr;
     double *meanSums = nullptr;
     int *meanCounts = nullptr, *meanMembers = nullptr;
     int numTiles = 0;
-    int rowsPerTile[kMaxQ + 1] = {0};
-    int grid = 0;
+    int rowsPerTile[kMaxQ + 1] = {0};  // register rows one wave sums: 2^q, or a half or quarter of it
     hipGraph_t graph = nullptr;
     hipGraphExec_t graphExec = nullptr;
     size_t aeSmem = 0;
@@ -398,84 +412,69 @@ struct SwapPlanImpl {
 
 namespace {
 
-// the swap-test sums of every tile: matrix cores for FP32 registers, FP64 on the VALU
+// results to p0 and assign (the plan's, or scratch where only the time counts)
 template <typename T>
-void launchSwapTiles(SwapPlanImpl *s) {
-    if constexpr (std::is_same<T, float>::value)
-        hipLaunchKernelGGL(kSwapTilesMfma, dim3(s->grid), dim3(kBlock), 0, hstream(), s->tiles, s->numTiles,
-                           (const float *)s->pointAE, s->pOff, s->pQ, (const float *)s->centAE, s->cOff, s->C, s->qLo,
-                           s->partial);
-    else
-        hipLaunchKernelGGL(kSwapTiles<T>, dim3(s->grid), dim3(kBlock), 0, hstream(), s->tiles, s->numTiles,
-                           (const T *)s->pointAE, s->pOff, s->pQ, (const T *)s->centAE, s->cOff, s->C, s->qLo,
-                           s->partial);
+void launchOverlap(SwapPlanImpl *s, double *p0, int *assign) {
+    hipLaunchKernelGGL(kOverlap<T>, dim3(s->numTiles), dim3(kBlock), 0, hstream(), s->tiles, s->order,
+                       (const T *)s->pointAE, s->pOff, s->pNorm, (const T *)s->centAE, s->cOff, s->cNorm, s->C, s->qLo,
+                       s->qLo >= 2 ? 1 : 0, p0, assign);
+}
+
+// the centroids at every register size: new means from the partial sums
+// (chunks = kMeanChunks) or the current centroids (chunks = 0)
+template <typename T>
+void launchCentroids(SwapPlanImpl *s, int chunks) {
+    const int numCent = (s->qHi - s->qLo + 1) * s->C;
+    hipLaunchKernelGGL(kCentroidUpdate<T>, dim3(numCent), dim3(kBlock), s->aeSmem, hstream(), s->meanSums,
+                       s->meanCounts, s->meanMembers, chunks, s->maxQ, s->C, s->qLo, s->qHi, s->cOff,
+                       (double *)s->cent, (T *)s->centAE, s->cNorm);
 }
 
 template <typename T>
 void launchIteration(SwapPlanImpl *s) {
-    const int numTests = s->P * s->C;
-    const int numCent = (s->qHi - s->qLo + 1) * s->C;
-    launchSwapTiles<T>(s);
-    hipLaunchKernelGGL(kSwapFinish, dim3((numTests + kBlock - 1) / kBlock), dim3(kBlock), 0, hstream(), s->partial,
-                       s->tStart, s->tCount, numTests, s->p0);
-    hipLaunchKernelGGL(kAssign, dim3((s->P + kBlock - 1) / kBlock), dim3(kBlock), 0, hstream(), s->p0, s->P, s->C,
-                       s->assign);
+    launchOverlap<T>(s, s->p0, s->assign);
     const int slices = std::max(1, (1 << s->maxQ) / kBlock);
     hipLaunchKernelGGL(kCentroidPartial, dim3(s->C * slices * kMeanChunks), dim3(kBlock), 0, hstream(),
                        (const double *)s->pointsV, s->pOff, s->pQ, s->assign, s->P, s->C, s->maxQ, s->meanSums,
                        s->meanCounts, s->meanMembers);
-    hipLaunchKernelGGL(kCentroidCombine, dim3(s->C * slices), dim3(kBlock), 0, hstream(), s->meanSums, s->meanCounts,
-                       s->meanMembers, s->C, s->maxQ, (double *)s->cent);
-    hipLaunchKernelGGL(kCentroidInputs, dim3(numCent), dim3(kBlock), 0, hstream(), (const double *)s->cent, s->maxQ,
-                       s->C, s->qLo, s->qHi, s->cOff, (double *)s->centIn);
-    hipLaunchKernelGGL(kAEState<T>, dim3(numCent), dim3(kBlock), s->aeSmem, hstream(), (const double *)s->centIn,
-                       s->cOff, s->cQ, (T *)s->centAE, numCent);
+    launchCentroids<T>(s, kMeanChunks);
 }
 
-// encode the current centroids at every size (used at creation)
-template <typename T>
-void encodeCentroids(SwapPlanImpl *s) {
-    const int numCent = (s->qHi - s->qLo + 1) * s->C;
-    hipLaunchKernelGGL(kCentroidInputs, dim3(numCent), dim3(kBlock), 0, hstream(), (const double *)s->cent, s->maxQ,
-                       s->C, s->qLo, s->qHi, s->cOff, (double *)s->centIn);
-    hipLaunchKernelGGL(kAEState<T>, dim3(numCent), dim3(kBlock), s->aeSmem, hstream(), (const double *)s->centIn,
-                       s->cOff, s->cQ, (T *)s->centAE, numCent);
+// waves that share a register's rows, from the rows one of them takes
+int splitOf(const SwapPlanImpl *s, int q) {
+    const int split = (1 << q) / s->rowsPerTile[q];
+    return split >= 4 ? 4 : split >= 2 ? 2 : 1;
 }
 
-// build the tile list for the current rows-per-tile choice (per q)
+// the tile list for the current rows-per-tile choice (per q), largest registers
+// first: the last workgroups to start are the short ones
 void buildTiles(SwapPlanImpl *s) {
     std::vector<Tile> tl;
-    std::vector<int> start(s->P * s->C), count(s->P * s->C);
-    // order: largest registers first so the persistent grid's tail is small tiles
-    std::vector<int> order(s->P);
-    for (int p = 0; p < s->P; ++p) order[p] = p;
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return s->hQ[x] > s->hQ[y]; });
-    for (int p : order) {
-        const int D = 1 << s->hQ[p];
-        const int rows = std::min(std::min(D, s->prec == FP32 ? 32 * kMaxRowBlocks : kMaxTileRows),
-                                  s->rowsPerTile[s->hQ[p]]);
-        for (int c = 0; c < s->C; ++c) {
-            const int test = p * s->C + c;
-            start[test] = (int)tl.size();
-            for (int x0 = 0; x0 < D; x0 += rows) tl.push_back(Tile{test, x0, std::min(rows, D - x0), 0});
-            count[test] = (int)tl.size() - start[test];
+    for (int first = 0, q = s->qHi; q >= s->qLo; --q) {
+        const int split = splitOf(s, q), per = 16 * (kWaves / split);
+        for (int left = s->sizeCount[q]; left > 0; left -= per) {
+            const int n = std::min(left, per);
+            tl.push_back(Tile{first, n, q, split});
+            first += n;
         }
     }
-    if (s->tiles) devFree(s->tiles);
-    if (s->partial) devFree(s->partial);
     s->numTiles = (int)tl.size();
-    s->tiles = static_cast<Tile *>(devAlloc(tl.size() * sizeof(Tile)));
-    s->partial = static_cast<double *>(devAlloc(tl.size() * sizeof(double)));
     hostToDevice(s->tiles, tl.data(), tl.size() * sizeof(Tile));
-    hostToDevice(s->tStart, start.data(), start.size() * sizeof(int));
-    hostToDevice(s->tCount, count.data(), count.size() * sizeof(int));
-    int cus = 256;
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, 0) == hipSuccess) cus = prop.multiProcessorCount;
-    // FP32: one tile per wave (4 per workgroup); FP64: one tile per workgroup
-    const int perGroup = s->prec == FP32 ? kBlock / 64 : 1;
-    s->grid = std::max(1, std::min((s->numTiles + perGroup - 1) / perGroup, cus * 8));
 }
+
+// outputs of launches that are only timed: the plan keeps its last results
+struct TimingScratch {
+    double *p0;
+    int *assign;
+    explicit TimingScratch(const SwapPlanImpl *s)
+        : p0(static_cast<double *>(devAlloc((size_t)s->P * s->C * sizeof(double)))),
+          assign(static_cast<int *>(devAlloc((size_t)s->P * sizeof(int)))) {}
+    TimingScratch(const TimingScratch &) = delete;
+    ~TimingScratch() {
+        devFree(p0);
+        devFree(assign);
+    }
+};
 
 void dropGraph(SwapPlanImpl *s) {
     if (s->graphExec) QMX_HIP_CHECK(hipGraphExecDestroy(s->graphExec));
@@ -599,7 +598,8 @@ void amplitudeEncode(QuregDev *q, const double *vec, int qbits) {
     hostToDevice(dIn, vec, (size_t)D * sizeof(double));
     hostToDevice(dOff, &h.off, sizeof(long long));
     hostToDevice(dQ, &h.q, sizeof(int));
-    hipLaunchKernelGGL(kAEState<double>, dim3(1), dim3(kBlock), smem, hstream(), dIn, dOff, dQ, dOut, 1);
+    hipLaunchKernelGGL(kAEState<double>, dim3(1), dim3(kBlock), smem, hstream(), dIn, dOff, dQ, dOut,
+                       (double *)nullptr, 1);
     initBlank(q);
     QMX_DISPATCH(q->prec, T, {
         hipLaunchKernelGGL(kAEWrite<T>, dim3(gridFor(D, 1)), dim3(kBlock), 0, hstream(), (Amp<T> *)q->amps, dOut, D);
@@ -637,6 +637,7 @@ qmxSwapPlan *qmxSwapPlanCreate(int numPoints, const int *pointQubits, const doub
         }
         s->qLo = std::min(s->qLo, q);
         s->qHi = std::max(s->qHi, q);
+        ++s->sizeCount[q];
     }
     s->hPOff.resize(numPoints);
     long long tot = 0;
@@ -646,17 +647,14 @@ qmxSwapPlan *qmxSwapPlanCreate(int numPoints, const int *pointQubits, const doub
     }
     const int nq = s->qHi - s->qLo + 1;
     s->hCOff.resize((size_t)nq * numCentroids);
-    std::vector<int> cq((size_t)nq * numCentroids);
     long long ctot = 0;
     for (int qi = 0; qi < nq; ++qi)
         for (int c = 0; c < numCentroids; ++c) {
             s->hCOff[(size_t)qi * numCentroids + c] = ctot;
-            cq[(size_t)qi * numCentroids + c] = s->qLo + qi;
             ctot += 1ll << (s->qLo + qi);
         }
     // encoded registers in the storage precision; inputs, centroids and the
-    // encoding arithmetic in FP64 (O(2^q) per vector, negligible next to the
-    // O(2^2q) swap-test evaluation)
+    // encoding arithmetic in FP64
     const size_t eb = precision == FP64 ? 8 : 4;
     std::vector<double> pts(points, points + tot);
     for (int p = 0; p < numPoints; ++p) {
@@ -672,15 +670,15 @@ qmxSwapPlan *qmxSwapPlanCreate(int numPoints, const int *pointQubits, const doub
     const size_t centCount = (size_t)numCentroids * (1ull << maxQubits);
     s->cent = devAlloc(centCount * 8);
     hostToDevice(s->cent, centroids, centCount * 8);
-    s->centIn = devAlloc((size_t)ctot * 8);
     s->centAE = devAlloc((size_t)ctot * eb);
     s->pOff = static_cast<long long *>(devAlloc(numPoints * sizeof(long long)));
     s->cOff = static_cast<long long *>(devAlloc(s->hCOff.size() * sizeof(long long)));
     s->pQ = static_cast<int *>(devAlloc(numPoints * sizeof(int)));
-    s->cQ = static_cast<int *>(devAlloc(cq.size() * sizeof(int)));
     s->assign = static_cast<int *>(devAlloc(numPoints * sizeof(int)));
-    s->tStart = static_cast<int *>(devAlloc((size_t)numPoints * numCentroids * sizeof(int)));
-    s->tCount = static_cast<int *>(devAlloc((size_t)numPoints * numCentroids * sizeof(int)));
+    s->order = static_cast<int *>(devAlloc(numPoints * sizeof(int)));
+    s->tiles = static_cast<Tile *>(devAlloc((size_t)(numPoints / 16 + kMaxQ + 1) * sizeof(Tile)));
+    s->pNorm = static_cast<double *>(devAlloc(numPoints * sizeof(double)));
+    s->cNorm = static_cast<double *>(devAlloc((size_t)nq * numCentroids * sizeof(double)));
     s->p0 = static_cast<double *>(devAlloc((size_t)numPoints * numCentroids * sizeof(double)));
     const size_t meanSlots = (size_t)kMeanChunks * numCentroids * (1ull << maxQubits);
     s->meanSums = static_cast<double *>(devAlloc(meanSlots * sizeof(double)));
@@ -689,27 +687,30 @@ qmxSwapPlan *qmxSwapPlanCreate(int numPoints, const int *pointQubits, const doub
     hostToDevice(s->pOff, s->hPOff.data(), numPoints * sizeof(long long));
     hostToDevice(s->cOff, s->hCOff.data(), s->hCOff.size() * sizeof(long long));
     hostToDevice(s->pQ, s->hQ.data(), numPoints * sizeof(int));
-    hostToDevice(s->cQ, cq.data(), cq.size() * sizeof(int));
+    std::vector<int> order(numPoints);
+    for (int p = 0; p < numPoints; ++p) order[p] = p;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return s->hQ[x] > s->hQ[y]; });
+    hostToDevice(s->order, order.data(), numPoints * sizeof(int));
     s->aeSmem = (size_t)3 * (1u << s->qHi) * sizeof(double);
     // 11- and 12-qubit registers need more than the 64 KiB default of dynamic LDS
     bool ldsOk = true;
     QMX_DISPATCH(precision, T, {
         if (s->aeSmem > 65536)
-            ldsOk = allowDynamicLds(reinterpret_cast<const void *>(kAEState<T>), s->aeSmem, "qmxSwapPlanCreate");
+            ldsOk = allowDynamicLds(reinterpret_cast<const void *>(kAEState<T>), s->aeSmem, "qmxSwapPlanCreate") &&
+                    allowDynamicLds(reinterpret_cast<const void *>(kCentroidUpdate<T>), s->aeSmem, "qmxSwapPlanCreate");
     });
     if (!ldsOk) {
         qmxSwapPlanDestroy(plan);
         return nullptr;
     }
-    // default tile rows: FP32 (one wave per tile) 64 rows, or the register
-    // when smaller; FP64 (one workgroup per tile) ~16K amplitudes a tile
-    for (int q = 0; q <= kMaxQ; ++q)
-        s->rowsPerTile[q] = precision == FP32 ? std::min(1 << q, 64)
-                                              : std::max(1, std::min(16384 >> q, std::min(1 << q, kMaxTileRows)));
+    // default rows per wave: a register's rows split over four waves from 256
+    // rows, over two from 64 (see kOverlap); smaller ones are one wave's
+    for (int q = 0; q <= kMaxQ; ++q) s->rowsPerTile[q] = (1 << q) / (q >= 8 ? 4 : q >= 6 ? 2 : 1);
     QMX_DISPATCH(precision, T, {
         hipLaunchKernelGGL(kAEState<T>, dim3(numPoints), dim3(kBlock), s->aeSmem, hstream(),
-                           (const double *)s->pointsV, s->pOff, s->pQ, (T *)s->pointAE, numPoints);
-        encodeCentroids<T>(s);
+                           (const double *)s->pointsV, s->pOff, s->pQ, (T *)s->pointAE,
+                           s->pNorm, numPoints);
+        launchCentroids<T>(s, 0);
     });
     checkLaunch("qmxSwapPlanCreate");
     buildTiles(s);
@@ -722,58 +723,39 @@ void qmxSwapPlanDestroy(qmxSwapPlan *plan) {
     if (!plan) return;
     SwapPlanImpl *s = &plan->impl;
     dropGraph(s);
-    for (void *p : {s->pointsV, s->pointAE, s->cent, s->centIn, s->centAE, (void *)s->pOff, (void *)s->cOff,
-                    (void *)s->pQ, (void *)s->cQ, (void *)s->assign, (void *)s->tStart, (void *)s->tCount,
-                    (void *)s->tiles, (void *)s->partial, (void *)s->p0, (void *)s->meanSums,
-                    (void *)s->meanCounts, (void *)s->meanMembers})
+    for (void *p : {s->pointsV, s->pointAE, s->cent, s->centAE, (void *)s->pOff, (void *)s->cOff, (void *)s->pQ,
+                    (void *)s->assign, (void *)s->order, (void *)s->tiles, (void *)s->pNorm, (void *)s->cNorm,
+                    (void *)s->p0, (void *)s->meanSums, (void *)s->meanCounts, (void *)s->meanMembers})
         devFree(p);
     delete plan;
 }
 
-// time candidate rows-per-tile for each register size on the device and keep
-// the fastest; returns the number of (size, candidate) timings made
+// time candidate rows-per-tile for each register size on the device (the rows
+// whole, halved or quartered over a workgroup's waves) and keep the fastest;
+// returns the number of (size, candidate) timings made
 int qmxSwapPlanAutotune(qmxSwapPlan *plan) {
     using namespace qmx;
     SwapPlanImpl *s = &plan->impl;
     dropGraph(s);
-    // FP32 tiles are row blocks of 32 on the matrix cores; FP64 tiles any rows
-    const std::vector<int> cands = s->prec == FP32 ? std::vector<int>{32, 64, 128, 256}
-                                                   : std::vector<int>{1, 4, 16, 64, 256, 1024, 4096};
+    TimingScratch scratch(s);
     int timings = 0;
     for (int q = s->qLo; q <= s->qHi; ++q) {
-        bool present = false;
-        for (int x : s->hQ) present |= (x == q);
-        if (!present) continue;
-        const int D = 1 << q;
+        if (!s->sizeCount[q]) continue;
         double best = 1e30;
         int bestRows = s->rowsPerTile[q];
-        int lastRows = -1;
-        for (int rowsCand : cands) {
-            int rows = rowsCand;
-            if (s->prec == FP32) {
-                if (D < 32) rows = D;           // a register smaller than one block: one tile
-                else if (rows > D) continue;
-            } else if (rows > D || rows > kMaxTileRows || (long long)rows * D > (1ll << 22) ||
-                       ((long long)rows * D < 256 && rows != D)) {
-                continue;
-            }
-            if (rows == lastRows) continue;
-            lastRows = rows;
-            // retime the whole tile list with this size's rows changed
-            int saved[kMaxQ + 1];
-            std::memcpy(saved, s->rowsPerTile, sizeof saved);
-            s->rowsPerTile[q] = rows;
+        for (int split = 1; split <= kWaves; split *= 2) {
+            if (split > 1 && (1 << q) / split < 16) break;  // a product step takes 16 rows
+            s->rowsPerTile[q] = (1 << q) / split;
             buildTiles(s);
             timerBegin();
-            QMX_DISPATCH(s->prec, T, { launchSwapTiles<T>(s); });
+            QMX_DISPATCH(s->prec, T, { launchOverlap<T>(s, scratch.p0, scratch.assign); });
             checkLaunch("autotune");
             const double ms = timerEndMs();
             ++timings;
             if (ms < best) {
                 best = ms;
-                bestRows = rows;
+                bestRows = s->rowsPerTile[q];
             }
-            std::memcpy(s->rowsPerTile, saved, sizeof saved);
         }
         s->rowsPerTile[q] = bestRows;
     }
@@ -788,35 +770,27 @@ int qmxSwapPlanRowsPerTile(const qmxSwapPlan *plan, int q) {
 
 int qmxSwapPlanNumTiles(const qmxSwapPlan *plan) { return plan->impl.numTiles; }
 
-// 32 x 32 amplitude blocks one iteration forms on the matrix cores (FP32
-// plans: blocks on or above the diagonal of every test, padded to a block for
-// registers under 32 amplitudes); 0 for FP64 plans
+// 16 x 16 x 4 matrix-core products one iteration makes
 long long qmxSwapPlanMfmaBlocks(const qmxSwapPlan *plan) {
     using namespace qmx;
     const SwapPlanImpl *s = &plan->impl;
-    if (s->prec != FP32) return 0;
-    long long blocks = 0;
-    for (int p = 0; p < s->P; ++p) {
-        const int D = 1 << s->hQ[p];
-        const int rows = std::min(std::min(D, 32 * kMaxRowBlocks), s->rowsPerTile[s->hQ[p]]);
-        const int nyb = (D + 31) / 32;
-        for (int x0 = 0; x0 < D; x0 += rows) {
-            const int xb0 = x0 / 32, nb = (std::min(rows, D - x0) + 31) / 32;
-            for (int k = 0; k < nb; ++k) blocks += nyb - (xb0 + k);
-        }
-    }
-    return blocks * s->C;
+    long long products = 0;
+    for (int q = s->qLo; q <= s->qHi; ++q)
+        products += (long long)((s->sizeCount[q] + 15) / 16) * (std::max(16, 1 << q) / 4);
+    return products * ((s->C + 15) / 16);
 }
 
-// device time of one launch of the swap-test tiles (ms, HIP events on the
+// device time of one swap-test launch (inner products, P0, assignment; ms, HIP events on the
 // library stream), averaged over `launches`
 double qmxSwapPlanTimeTiles(qmxSwapPlan *plan, int launches) {
     using namespace qmx;
     SwapPlanImpl *s = &plan->impl;
     if (launches < 1) return 0.0;
+    TimingScratch scratch(s);
     deviceSync();
     timerBegin();
-    for (int i = 0; i < launches; ++i) QMX_DISPATCH(s->prec, T, { launchSwapTiles<T>(s); });
+    for (int i = 0; i < launches; ++i)
+        QMX_DISPATCH(s->prec, T, { launchOverlap<T>(s, scratch.p0, scratch.assign); });
     checkLaunch("qmxSwapPlanTimeTiles");
     return timerEndMs() / launches;
 }
@@ -859,13 +833,13 @@ void qmxSwapPlanCentroids(qmxSwapPlan *plan, double *out) {
 }
 
 // replace the centroids (numCentroids x 2^maxQubits doubles) and re-encode
-// them; the point registers, tiles, autotuned shapes and a captured graph stay
+// them; the point registers, tiles, tuned shapes and a captured graph stay
 void qmxSwapPlanSetCentroids(qmxSwapPlan *plan, const double *centroids) {
     using namespace qmx;
     SwapPlanImpl *s = &plan->impl;
     deviceSync();
     hostToDevice(s->cent, centroids, (size_t)s->C * (1ull << s->maxQ) * sizeof(double));
-    QMX_DISPATCH(s->prec, T, { encodeCentroids<T>(s); });
+    QMX_DISPATCH(s->prec, T, { launchCentroids<T>(s, 0); });
     checkLaunch("qmxSwapPlanSetCentroids");
     deviceSync();
 }

@@ -213,3 +213,39 @@ def test_closed_form_cpu_port_matches_inner_products(cpuref):
     fn(len(qs), qa.ctypes.data_as(C.POINTER(C.c_int)), A.ctypes.data_as(dp), off.ctypes.data_as(lp),
        B.ctypes.data_as(dp), off.ctypes.data_as(lp), out.ctypes.data_as(dp))
     assert np.max(np.abs(out - np.array(want))) < 1e-13
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("P,C,q_lo,q_hi,max_q", [(1, 1, 1, 1, 1), (15, 3, 1, 4, 6), (17, 16, 2, 5, 5), (33, 17, 6, 8, 8),
+                                                 (70, 33, 4, 10, 12), (40, 5, 11, 12, 12)])
+@pytest.mark.parametrize("precision", [QMX_PREC_FP64, QMX_PREC_FP32])
+def test_iteration_at_tile_edges(gpu, P, C, q_lo, q_hi, max_q, precision):
+    """One iteration where tiles are ragged: fewer than 16 points or centroids of
+    a size, registers below one 16-row step, rows over one, two and four waves,
+    centroids longer than every point, and every tuned split."""
+    rng = np.random.default_rng([P, C, q_hi])
+    qs = rng.integers(q_lo, q_hi + 1, size=P).astype(np.int32)
+    sizes = 1 << qs.astype(np.int64)
+    off = np.concatenate([[0], np.cumsum(sizes)[:-1]]).astype(np.int64)
+    init = rng.standard_normal((C, 1 << max_q))
+    data = K.Dataset(rng.standard_normal(int(sizes.sum())), off, qs, np.zeros(P, np.int32), init, init, max_q)
+    unit = [data.point(p) / np.linalg.norm(data.point(p)) for p in range(P)]
+    want = np.array([[0.5 + 0.5 * (unit[p] @ c[:len(unit[p])]) ** 2 / (c[:len(unit[p])] @ c[:len(unit[p])])
+                      for c in init] for p in range(P)])
+    # FP64: sums of 2^q products; FP32: registers rounded once (relative 2^-24 an
+    # amplitude, so at most 2^-23 on an overlap and twice that on its square)
+    tol = 1e-13 if precision == QMX_PREC_FP64 else 2.0 ** -22
+    for tuned in (False, True):
+        plan = K.SwapPlan(gpu, data, precision)
+        if tuned:
+            assert plan.autotune() > 0
+        plan.run(1, graph=tuned)
+        got, assign, cents = plan.p0(), plan.assignments(), plan.centroids()
+        plan.close()
+        assert np.max(np.abs(got - want)) < tol
+        assert np.array_equal(assign, np.argmax(got, axis=1))
+        for c in range(C):
+            members = [unit[p] for p in range(P) if assign[p] == c]
+            for j in range(1 << max_q):
+                vals = [m[j] for m in members if len(m) > j]
+                assert abs(cents[c, j] - (np.mean(vals) if vals else init[c, j])) < 1e-13
