@@ -526,12 +526,24 @@ void tileFormBuild(const float *hm, const Fused5TileSpec &sp, void *out) {
     }
 }
 
+// Tiles per workgroup: `most` where that still leaves `perCU` workgroups on every
+// CU, else the largest power of two that does. FP64 workgroups are worth splitting
+// until two sit on each CU: a 17-qubit register has 64 tiles, 8 workgroups of 8
+// took 22.3 us, 64 of one 6.5 us; at 20 qubits (512 tiles) 24.8 and 12.2 us. FP32
+// workgroups pay more for their prologue and only split below one a CU: 1024
+// tiles took 11.1 us by four and 11.7 us by one.
+long long tilesPerGroup(long long numTiles, int most, int perCU) {
+    long long per = most;
+    while (per > 1 && numTiles < per * perCU * numCUs()) per /= 2;
+    return per;
+}
+
 void launchFused5Tile(QuregDev *q, const Fused5Spec &spec, const void *form) {
     Fused5TileSpec sp = tileSpecOf(spec.targetsSorted);
     sp.numTiles = q->numAmps / kTileAmps;
-    sp.tilesPerGroup = kTilesPerGroup;
+    sp.tilesPerGroup = tilesPerGroup(sp.numTiles, kTilesPerGroup, 1);
     // a multiple of 8 workgroups (xcdBlock's XCD order); the extra ones exit
-    const long long g = ((sp.numTiles + kTilesPerGroup - 1) / kTilesPerGroup + 7) / 8 * 8;
+    const long long g = ((sp.numTiles + sp.tilesPerGroup - 1) / sp.tilesPerGroup + 7) / 8 * 8;
     hipLaunchKernelGGL(kFused5Tile, dim3((unsigned)g), dim3(kBlock), 0, hstream(), (Amp<float> *)q->amps, sp,
                        static_cast<const f4v *>(form));
     checkLaunch("fused5Apply");
@@ -672,8 +684,8 @@ void fused5ApplyOnce64(QuregDev *q, const int *targs, const Cplx *u) {
     stageCommit(sg, bytes, st);
     Fused5TileSpec64 sp = tileSpecOf64(spec.targetsSorted);
     sp.numTiles = q->numAmps / kTileAmps;
-    sp.tilesPerGroup = kTilesPerGroup64;
-    const long long g = ((sp.numTiles + kTilesPerGroup64 - 1) / kTilesPerGroup64 + 7) / 8 * 8;
+    sp.tilesPerGroup = tilesPerGroup(sp.numTiles, kTilesPerGroup64, 2);
+    const long long g = ((sp.numTiles + sp.tilesPerGroup - 1) / sp.tilesPerGroup + 7) / 8 * 8;
     hipLaunchKernelGGL(kFused5Tile64, dim3((unsigned)g), dim3(kBlock), 0, st, (Amp<double> *)q->amps, sp,
                        static_cast<const d2v *>(sg.dev));
     checkLaunch("fused5ApplyOnce64");

@@ -235,14 +235,33 @@ __global__ void __launch_bounds__(kBlock) kOutcomeHist(const Amp<T> *__restrict_
     }
 }
 
-// per outcome, the chunks' partials in chunk order
+// Per outcome, the sum of its chunks' partials, one wave each: lane l takes
+// partials l, l + 64, ... (four loads in flight) and the lanes merge by a
+// butterfly, so the order is fixed. Few outcomes leave few sums of many chunks
+// (2^16 units: 64 outcomes, 1024 chunks), and a thread that walked them one by
+// one took 241 us after a 5 us histogram (17 qubits FP64); a wave each takes 7 us.
 __global__ void __launch_bounds__(kBlock) kOutcomeFinish(const double *__restrict__ part, int chunkLog,
                                                          long long numOut, double *out) {
-    const long long o = (long long)blockIdx.x * kBlock + threadIdx.x;
+    constexpr int U = 4;
+    const int lane = threadIdx.x & 63;
+    const long long o = flatBlockLinear() * (kBlock / 64) + (threadIdx.x >> 6);
     if (o >= numOut) return;
+    const long long n = 1ll << chunkLog;
+    const double *p = part + (o << chunkLog);
     Acc acc;
-    for (long long c = 0; c < (1ll << chunkLog); ++c) acc.add(part[(o << chunkLog) + c]);
-    out[o] = acc.value();
+    for (long long c0 = lane; c0 < n; c0 += 64 * U) {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = c0 + 64 * u < n ? p[c0 + 64 * u] : 0.0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc.add(v[u]);
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        const double os = __shfl_xor(acc.s, off, 64), oc = __shfl_xor(acc.c, off, 64);
+        acc.merge(os, oc);
+    }
+    if (lane == 0) out[o] = acc.value();
 }
 
 template <int NV>
@@ -428,8 +447,8 @@ const double *probOfAllOutcomesDevice(const QuregDev *q, const int *qubits, int 
     });
     checkLaunch("probOfAllOutcomes");
     if (pl.chunkLog) {
-        hipLaunchKernelGGL(kOutcomeFinish, dim3((unsigned)((numOut + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                           hstream(), part, pl.chunkLog, numOut, res);
+        hipLaunchKernelGGL(kOutcomeFinish, gridFor(numOut * 64, 1), dim3(kBlock), 0, hstream(), part, pl.chunkLog,
+                           numOut, res);
         checkLaunch("probOfAllOutcomes finish");
     }
     return res;
