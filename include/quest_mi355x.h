@@ -129,7 +129,8 @@ long long qmxLoadStateCSV(Qureg qureg, const char *path);
  * (QL/Circuit/QLGate.cpp:652-803, driven by QL/Simulator/QLSimulator*.cpp):
  * unfused, each operation is the QuEST call that loop makes; fused (state
  * vectors), the unitaries between collapses run as dense blocks of at most k
- * qubits, one sweep per block. */
+ * qubits, several blocks to a sweep where k is 5. State vectors of at most 12
+ * qubits take either form gate by gate, in one launch. */
 typedef struct qmxCircuit qmxCircuit;
 
 /* QuantumLab's basic operations: the codes of EBasicOperation
@@ -191,6 +192,14 @@ int qmxCircuitNumBlocks(const qmxCircuit *c);
  * matrix index) and its 2^k x 2^k matrix (row-major; any pointer may be NULL),
  * returning k; 0 for a collapse; -1 past the end. */
 int qmxCircuitStep(const qmxCircuit *c, int step, int *targs, qreal *re, qreal *im);
+/* How a circuit fused into blocks of 5 runs on registers of more than 12 qubits:
+ * sweep `sweep` (one read and write of a register of this storage precision)
+ * applies its blocks of 4 or 5 qubits one after another; a gate that shares its
+ * sweep with no other is one block of its own qubits (targets and controls). Gives
+ * block `block`'s qubits and matrix as qmxCircuitStep does and returns its qubit
+ * count; 0 past the sweep's last block, -1 past the last sweep or where no sweeps
+ * are planned. Collapses run between sweeps and are not listed. */
+int qmxCircuitSweepBlock(qmxCircuit *c, int precision, int sweep, int block, int *targs, qreal *re, qreal *im);
 /* Apply to a register of the circuit's width; returns the product of the
  * collapse probabilities (1 without collapses). fused != 0 on a state vector
  * uses the fused blocks (after qmxCircuitFuse), otherwise each operation is the

@@ -15,20 +15,19 @@
 // operation that is neither noise nor a collapse is followed by the density
 // simulator's after-gate noise (QLSimulatorDensityMatrix.cpp:88-153).
 //
-// Applied fused (state vectors), the planner below has grouped the unitaries
-// between collapses into dense blocks of at most k qubits; each block is one
-// sweep (qmx::applyMatrixN, or the FP32 MFMA kernel for 5-qubit blocks)
-// instead of one sweep per gate, and each collapse is a barrier no block
-// crosses. On density registers, fused application is the unfused sequence:
-// the library already composes every operation on at most two qubits into
-// superoperator sweeps there.
+// Applied fused (state vectors), the unitaries between collapses run as dense
+// blocks, and each collapse is a barrier no block crosses. Blocks of at most 5
+// qubits on registers of more than 12 qubits share sweeps (qmx_plan.cpp plans
+// them, qmx_sweep.hip builds and applies them: many gates to a read and write of
+// the register); other block sizes take one sweep a block (qmx::applyMatrixN).
+// State vectors of at most 12 qubits take every list, fused or not, gate by gate
+// in one workgroup's LDS, one launch for the list. On density registers, fused
+// application is the unfused sequence: the library already composes every
+// operation on at most two qubits into superoperator sweeps there.
 //
-// Planner (greedy, dependency-aware): for a gate on qubit set Q, let B be the
-// last block after the latest barrier that touches Q. The gate may join B, or
-// any later block (those touch none of Q, so the gate commutes past them),
-// provided the union of qubits stays <= k. Among those it joins the one with
-// the largest overlap, else opens a new block at the end. Block matrices are
-// products of the expanded gate matrices, formed on the host in FP64.
+// The block planner below (qmxCircuitFuse's steps) is greedy and dependency-aware:
+// see fuseSegment. Block matrices are products of the expanded gate matrices,
+// formed on the host in FP64.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -39,10 +38,12 @@
 
 #include "QuEST.h"
 #include "qmx_internal.h"
+#include "qmx_sweep.h"
 #include "quest_mi355x.h"
 #include "quest_validation.h"
 
 using qmx::Cplx;
+using qmx::FlatGate;
 
 namespace {
 
@@ -90,7 +91,6 @@ struct Block {
     std::vector<int> gates;     // indices into the operation list, in order
     std::vector<int> targs;     // ascending qubits (targs[0] = LSB of the block matrix)
     std::vector<Cplx> u;        // dense block matrix, row-major
-    void *prepared5 = nullptr;  // device-resident form for the FP32 MFMA kernel
     int barrierOp = -1;         // >= 0: this step is the collapse ops[barrierOp]
 };
 
@@ -170,43 +170,89 @@ void setCompact(Gate &g, int target, uint64_t ctrl, Cplx a, Cplx b) {
 }
 
 // the rotation about axis (x, y, z) by `angle` as a compact pair
-void setRotation(Gate &g, int target, uint64_t ctrl, double angle, double x, double y, double z) {
+void rotationPair(double angle, double x, double y, double z, Cplx &a, Cplx &b) {
     const double c = std::cos(angle / 2.0), s = std::sin(angle / 2.0);
-    setCompact(g, target, ctrl, Cplx{c, -s * z}, Cplx{s * y, -s * x});
+    a = Cplx{c, -s * z};
+    b = Cplx{s * y, -s * x};
+}
+
+void setRotation(Gate &g, int target, uint64_t ctrl, double angle, double x, double y, double z) {
+    Cplx a, b;
+    rotationPair(angle, x, y, z, a, b);
+    setCompact(g, target, ctrl, a, b);
+}
+
+// QuantumLab's operation `code` on qubits q with angle t in matrix form; false
+// where it has none (noise, collapses, undispatched codes)
+bool basicGate(int code, const int *q, double t, FlatGate &g) {
+    const double r = 1.0 / std::sqrt(2.0);
+    auto matrix = [&](int target, uint64_t ctrl, Cplx u00, Cplx u01, Cplx u10, Cplx u11) {
+        g.kind = FlatGate::MATRIX2;
+        g.target = target;
+        g.ctrl = ctrl;
+        g.u[0] = u00;
+        g.u[1] = u01;
+        g.u[2] = u10;
+        g.u[3] = u11;
+        return true;
+    };
+    auto rotation = [&](int target, uint64_t ctrl, double x, double y, double z) {
+        Cplx a, b;
+        rotationPair(t, x, y, z, a, b);
+        return matrix(target, ctrl, a, Cplx{-b.re, b.im}, b, Cplx{a.re, -a.im});
+    };
+    auto bitNot = [&](int target, uint64_t ctrl) {
+        g.kind = FlatGate::NOT;
+        g.target = target;
+        g.ctrl = ctrl;
+        return true;
+    };
+    const Cplx zero{0, 0}, one{1, 0};
+    switch (code) {
+        case QMX_OP_H: return matrix(q[0], 0, {r, 0}, {r, 0}, {r, 0}, {-r, 0});
+        case QMX_OP_X: return bitNot(q[0], 0);
+        case QMX_OP_Y: return matrix(q[0], 0, zero, {0, -1}, {0, 1}, zero);
+        case QMX_OP_Z: return matrix(q[0], 0, one, zero, zero, {-1, 0});
+        case QMX_OP_P: return matrix(q[0], 0, one, zero, zero, {std::cos(t), std::sin(t)});
+        case QMX_OP_RX: return rotation(q[0], 0, 1, 0, 0);
+        case QMX_OP_RY: return rotation(q[0], 0, 0, 1, 0);
+        case QMX_OP_RZ: return rotation(q[0], 0, 0, 0, 1);
+        case QMX_OP_CX: return bitNot(q[1], 1ull << q[0]);
+        case QMX_OP_CY: return matrix(q[1], 1ull << q[0], zero, {0, -1}, {0, 1}, zero);
+        case QMX_OP_CZ: return matrix(q[1], 1ull << q[0], one, zero, zero, {-1, 0});
+        case QMX_OP_CP: return matrix(q[1], 1ull << q[0], one, zero, zero, {std::cos(t), std::sin(t)});
+        case QMX_OP_CRX: return rotation(q[1], 1ull << q[0], 1, 0, 0);
+        case QMX_OP_CRY: return rotation(q[1], 1ull << q[0], 0, 1, 0);
+        case QMX_OP_CRZ: return rotation(q[1], 1ull << q[0], 0, 0, 1);
+        default: return false;
+    }
 }
 
 bool basicGate(Op &o) {
-    const int *q = o.qubits.data();
-    const double t = o.param;
-    const double r = 1.0 / std::sqrt(2.0);
-    Gate &g = o.gate;
-    switch (o.code) {
-        case QMX_OP_H: setMatrix2(g, q[0], 0, {r, 0}, {r, 0}, {r, 0}, {-r, 0}); return true;
-        case QMX_OP_X:
-            g.kind = G_NOT;
-            g.target = q[0];
-            return true;
-        case QMX_OP_Y: setMatrix2(g, q[0], 0, {0, 0}, {0, -1}, {0, 1}, {0, 0}); return true;
-        case QMX_OP_Z: setMatrix2(g, q[0], 0, {1, 0}, {0, 0}, {0, 0}, {-1, 0}); return true;
-        case QMX_OP_P: setMatrix2(g, q[0], 0, {1, 0}, {0, 0}, {0, 0}, {std::cos(t), std::sin(t)}); return true;
-        case QMX_OP_RX: setRotation(g, q[0], 0, t, 1, 0, 0); return true;
-        case QMX_OP_RY: setRotation(g, q[0], 0, t, 0, 1, 0); return true;
-        case QMX_OP_RZ: setRotation(g, q[0], 0, t, 0, 0, 1); return true;
-        case QMX_OP_CX:
-            g.kind = G_NOT;
-            g.target = q[1];
-            g.ctrlMask = 1ull << q[0];
-            return true;
-        case QMX_OP_CY: setMatrix2(g, q[1], 1ull << q[0], {0, 0}, {0, -1}, {0, 1}, {0, 0}); return true;
-        case QMX_OP_CZ: setMatrix2(g, q[1], 1ull << q[0], {1, 0}, {0, 0}, {0, 0}, {-1, 0}); return true;
-        case QMX_OP_CP:
-            setMatrix2(g, q[1], 1ull << q[0], {1, 0}, {0, 0}, {0, 0}, {std::cos(t), std::sin(t)});
-            return true;
-        case QMX_OP_CRX: setRotation(g, q[1], 1ull << q[0], t, 1, 0, 0); return true;
-        case QMX_OP_CRY: setRotation(g, q[1], 1ull << q[0], t, 0, 1, 0); return true;
-        case QMX_OP_CRZ: setRotation(g, q[1], 1ull << q[0], t, 0, 0, 1); return true;
-        default: return false;
+    FlatGate f;
+    if (!basicGate(o.code, o.qubits.data(), o.param, f)) return false;
+    o.gate.kind = f.kind == FlatGate::NOT ? G_NOT : G_MATRIX2;
+    o.gate.target = f.target;
+    o.gate.ctrlMask = f.ctrl;
+    if (f.kind == FlatGate::MATRIX2) o.gate.u.assign(f.u, f.u + 4);
+    return true;
+}
+
+FlatGate flatGate(const Gate &g) {
+    FlatGate f;
+    f.target = g.target;
+    f.ctrl = g.ctrlMask;
+    if (g.kind == G_MATRIXN) {
+        f.kind = FlatGate::MATRIXN;
+        f.k = (int)g.targs.size();
+        f.targs = g.targs.data();
+        f.uN = g.u.data();
+    } else if (g.kind == G_NOT) {
+        f.kind = FlatGate::NOT;
+    } else {
+        std::copy(g.u.begin(), g.u.end(), f.u);
     }
+    return f;
 }
 
 // qubits an operation code takes (0: not a recordable QuantumLab code)
@@ -228,16 +274,39 @@ bool isNoise(int code) { return code >= QMX_OP_NOISE_DAMPING && code <= QMX_OP_N
 
 }  // namespace
 
+// The gates of a list in matrix form, and where the list stops for an operation
+// that is not one (a collapse): ops[stops[i].second] runs before gate stops[i].first.
+struct GateList {
+    std::vector<FlatGate> gates;
+    std::vector<int> op;                       // each gate's operation
+    std::vector<std::pair<int, int>> stops;
+};
+
+// A fused circuit's sweeps for one storage precision; stops as in GateList, but
+// before sweep stops[i].first.
+struct CircuitSweeps {
+    GateList list;
+    qmx::SweepPlan plan;
+    std::vector<std::pair<int, int>> stops;
+    qmx::SweepProgram *program = nullptr;
+};
+
 struct qmxCircuit {
     int numQubits;
     Qureg shape;                // register of this width, for the recorders' validation
     std::vector<Op> ops;
     std::vector<Block> blocks;
     int fusedQubits = 0;
+    int fusedOps = 0;           // operations the last fuse covered
+    CircuitSweeps *sweeps[2] = {nullptr, nullptr};  // by storage precision, planned when first needed
     qmxNoiseAfterGate noise{};
     void releaseBlocks() {
-        for (Block &b : blocks) qmx::fused5Free(b.prepared5);
         blocks.clear();
+        for (CircuitSweeps *&s : sweeps) {
+            if (s) qmx::sweepProgramFree(s->program);
+            delete s;
+            s = nullptr;
+        }
     }
     ~qmxCircuit() {
         releaseBlocks();
@@ -346,23 +415,20 @@ bool hasNoise(const qmxNoiseAfterGate &nz) {
            nz.twoQubitDephasing > 0 || nz.twoQubitDepolarising > 0;
 }
 
-void recordBasic(qmxCircuit *c, int code, const int *qubits, int numQubits, double param, const char *f) {
+// accepted and not dispatched, as in PerformBasicOperation
+bool undispatched(int code) { return code == QMX_OP_PHASE || code == QMX_OP_COMPOSITE; }
+
+void checkBasic(const Qureg &s, int code, const int *qubits, int numQubits, double param, const char *f) {
     const int need = arity(code);
-    if (code == QMX_OP_PHASE || code == QMX_OP_COMPOSITE) {
+    if (undispatched(code)) {
         if (numQubits < 0 || numQubits > 2) qv::raise("An operation lists at most two qubits.", f);
-        for (int i = 0; i < numQubits; ++i) qv::target(c->shape, qubits[i], f);
-        Op o;  // accepted and not dispatched, as in PerformBasicOperation
-        o.code = code;
-        o.qubits.assign(qubits, qubits + std::max(0, numQubits));
-        o.param = param;
-        c->ops.push_back(std::move(o));
+        for (int i = 0; i < numQubits; ++i) qv::target(s, qubits[i], f);
         return;
     }
     if (need == 0) qv::raise("Invalid operation code. Must be one of QuantumLab's basic operations (0-26).", f);
     if (numQubits != need)
         qv::raise(need == 1 ? "This operation takes exactly one qubit." : "This operation takes exactly two qubits.",
                   f);
-    const Qureg &s = c->shape;
     if (need == 1) {
         qv::target(s, qubits[0], f);
     } else if (isNoise(code)) {
@@ -383,12 +449,16 @@ void recordBasic(qmxCircuit *c, int code, const int *qubits, int numQubits, doub
         case QMX_OP_NOISE_TWO_QUBIT_DEPOLARISING: qv::twoQubitDepolProb(param, f); break;
         default: break;
     }
+}
+
+void recordBasic(qmxCircuit *c, int code, const int *qubits, int numQubits, double param, const char *f) {
+    checkBasic(c->shape, code, qubits, numQubits, param, f);
     Op o;
     o.code = code;
-    o.qubits.assign(qubits, qubits + numQubits);
+    o.qubits.assign(qubits, qubits + std::max(0, numQubits));
     o.param = param;
     o.barrier = code == QMX_OP_CC;
-    basicGate(o);
+    if (!undispatched(code)) basicGate(o);
     c->ops.push_back(std::move(o));
 }
 
@@ -407,17 +477,97 @@ void checkRegister(const qmxCircuit *c, const Qureg &q, const char *f) {
         qv::raise("The circuit and the register have different numbers of qubits.", f);
 }
 
+// the first numOps operations as a gate list; `everyOp`: operations without a
+// matrix form stop the list (they run as the QuEST calls they are), else only
+// collapses do and the others are skipped, as fused application has it
+GateList gateList(const qmxCircuit *c, int numOps, bool everyOp) {
+    GateList l;
+    l.gates.reserve(numOps);
+    l.op.reserve(numOps);
+    for (int i = 0; i < numOps; ++i) {
+        const Op &o = c->ops[i];
+        if (o.gate.kind != G_NONE) {
+            l.gates.push_back(flatGate(o.gate));
+            l.op.push_back(i);
+        } else if (everyOp || o.barrier) {
+            l.stops.push_back({(int)l.gates.size(), i});
+        }
+    }
+    return l;
+}
+
+// a gate list on a register of at most kSmallCircuitQubits qubits; stop(op)
+// runs an operation that is not a gate
+template <class F>
+void runSmall(qmx::QuregDev *d, const GateList &l, F stop) {
+    size_t s = 0;
+    int i = 0;
+    const int n = (int)l.gates.size();
+    while (i < n || s < l.stops.size()) {
+        const int until = s < l.stops.size() ? l.stops[s].first : n;
+        while (i < until) {
+            int j = i;
+            while (j < until && l.gates[j].kind != FlatGate::MATRIXN) ++j;
+            if (j > i) qmx::smallCircuit(d, l.gates.data() + i, j - i);
+            if (j < until) qmx::applyFlatGate(d, l.gates[j++]);
+            i = j;
+        }
+        if (s < l.stops.size()) stop(l.stops[s++].second);
+    }
+}
+
+// sweeps for the list's gates, segment by segment: no sweep crosses a stop
+void planList(int numQubits, int prec, const GateList &l, qmx::SweepPlan &plan,
+              std::vector<std::pair<int, int>> &stops) {
+    int i = 0;
+    for (size_t s = 0; s <= l.stops.size(); ++s) {
+        const int until = s < l.stops.size() ? l.stops[s].first : (int)l.gates.size();
+        if (until > i)
+            qmx::planSweeps(numQubits, qmx::sweepLowBits(prec), l.gates.data() + i, until - i, i, plan);
+        i = until;
+        if (s < l.stops.size()) stops.push_back({(int)plan.sweeps.size(), l.stops[s].second});
+    }
+}
+
+CircuitSweeps *sweepsOf(qmxCircuit *c, int prec) {
+    CircuitSweeps *&s = c->sweeps[prec];
+    if (!s) {
+        s = new CircuitSweeps;
+        s->list = gateList(c, c->fusedOps, false);
+        planList(c->numQubits, prec, s->list, s->plan, s->stops);
+    }
+    return s;
+}
+
 double applyCircuit(const Qureg &q, qmxCircuit *c, int fused) {
     double prob = 1.0;
     const bool noisy = q.isDensityMatrix && hasNoise(c->noise);
-    if (!fused || c->blocks.empty() || q.isDensityMatrix) {
+    qmx::QuregDev *d = qmx::dev(q);
+    const bool asBlocks = fused && !c->blocks.empty() && !q.isDensityMatrix;
+    if (qmx::smallCircuitSupported(d)) {
+        runSmall(d, asBlocks ? gateList(c, c->fusedOps, false) : gateList(c, (int)c->ops.size(), true),
+                 [&](int op) { prob *= runOp(q, c->ops[op]); });
+        return prob;
+    }
+    if (!asBlocks) {
         for (Op &o : c->ops) {
             prob *= runOp(q, o);
             if (noisy) noiseAfterGate(q, o, c->noise);
         }
         return prob;
     }
-    qmx::QuregDev *d = qmx::dev(q);
+    if (c->fusedQubits == qmx::kSweepBlockQubits && qmx::sweepSupported(d->numQubits)) {
+        CircuitSweeps *s = sweepsOf(c, d->prec);
+        if (!s->program) s->program = qmx::sweepProgramCreate(d->prec, s->plan, s->list.gates.data());
+        int at = 0;
+        for (size_t i = 0; i <= s->stops.size(); ++i) {
+            const int until = i < s->stops.size() ? s->stops[i].first : (int)s->plan.sweeps.size();
+            qmx::sweepProgramRun(d, s->program, s->plan, s->list.gates.data(), at, until);
+            at = until;
+            if (i < s->stops.size()) prob *= runOp(q, c->ops[s->stops[i].second]);
+        }
+        return prob;
+    }
     for (Block &b : c->blocks) {
         if (b.barrierOp >= 0) {
             prob *= runOp(q, c->ops[b.barrierOp]);
@@ -425,11 +575,6 @@ double applyCircuit(const Qureg &q, qmxCircuit *c, int fused) {
         }
         if (b.gates.size() == 1) {
             runOp(q, c->ops[b.gates[0]]);  // a lone gate keeps its cheaper kernel
-            continue;
-        }
-        if (d->prec == qmx::FP32 && b.targs.size() == 5 && d->numQubits >= 9) {
-            if (!b.prepared5) b.prepared5 = qmx::fused5Prepare(b.targs.data(), b.u.data());
-            qmx::fused5Apply(d, b.prepared5);
             continue;
         }
         qmx::applyMatrixN(d, 0, b.targs.data(), (int)b.targs.size(), b.u.data());
@@ -523,6 +668,7 @@ void fuseSegment(qmxCircuit *c, const std::vector<int> &seg, int maxQubits) {
 int fuseCircuit(qmxCircuit *c, int maxQubits) {
     c->releaseBlocks();
     c->fusedQubits = maxQubits;
+    c->fusedOps = (int)c->ops.size();
     std::vector<int> seg;  // gates since the latest barrier
     for (int gi = 0; gi < (int)c->ops.size(); ++gi) {
         const Op &o = c->ops[gi];
@@ -711,6 +857,38 @@ int qmxCircuitStep(const qmxCircuit *c, int step, int *targs, qreal *re, qreal *
     return k;
 }
 
+int qmxCircuitSweepBlock(qmxCircuit *c, int precision, int sweep, int block, int *targs, qreal *re, qreal *im) {
+    CIRCUIT_TRY
+    if (c->blocks.empty() || c->fusedQubits != qmx::kSweepBlockQubits || !qmx::sweepSupported(c->numQubits) ||
+        (precision != QMX_PREC_FP64 && precision != QMX_PREC_FP32))
+        return -1;
+    const CircuitSweeps *s = sweepsOf(c, precision == QMX_PREC_FP64 ? qmx::FP64 : qmx::FP32);
+    if (sweep < 0 || sweep >= (int)s->plan.sweeps.size()) return -1;
+    const qmx::Sweep &w = s->plan.sweeps[sweep];
+    if (block < 0 || block >= (w.lone >= 0 ? 1 : w.numBlocks)) return 0;
+    Block b;
+    if (w.lone >= 0) {
+        b.gates.push_back(s->list.op[w.lone]);
+        b.mask = s->list.gates[w.lone].mask();
+    } else {
+        const qmx::SweepBlock &sb = s->plan.blocks[w.firstBlock + block];
+        for (int g = 0; g < sb.numGates; ++g) b.gates.push_back(s->list.op[s->plan.order[sb.firstGate + g]]);
+        for (int j = 0; j < sb.k; ++j) b.mask |= 1ull << sb.targs[j];
+    }
+    buildBlockMatrix(*c, b);
+    const int k = (int)b.targs.size();
+    const size_t dim = 1ull << k;
+    if (targs)
+        for (int j = 0; j < k; ++j) targs[j] = b.targs[j];
+    if (re && im)
+        for (size_t e = 0; e < dim * dim; ++e) {
+            re[e] = (qreal)b.u[e].re;
+            im[e] = (qreal)b.u[e].im;
+        }
+    return k;
+    CIRCUIT_CATCH(-1)
+}
+
 int qmxCircuitNumBlocks(const qmxCircuit *c) {
     int n = 0;
     for (const Block &b : c->blocks) n += b.barrierOp < 0;
@@ -738,6 +916,51 @@ qreal qmxApplyOperations(Qureg qureg, const qmxBasicOperation *ops, int numOps, 
     if (noise) {
         noiseParams(*noise, __func__);
         c.noise = *noise;
+    }
+    // State vectors whose gates need no recording (one LDS circuit, or sweeps):
+    // straight from the caller's list to the kernels' gates.
+    qmx::QuregDev *d = qmx::dev(qureg);
+    const bool small = qmx::smallCircuitSupported(d);
+    const bool sweeps = !qureg.isDensityMatrix && fuseQubits == qmx::kSweepBlockQubits &&
+                        qmx::sweepSupported(d->numQubits);
+    if (small || sweeps) {
+        GateList l;
+        l.gates.reserve(numOps);
+        for (int i = 0; i < numOps; ++i) {
+            const qmxBasicOperation &o = ops[i];
+            checkBasic(c.shape, o.operation, o.qubits, o.numQubits, (double)o.param, __func__);
+            FlatGate g;
+            if (!undispatched(o.operation) && basicGate(o.operation, o.qubits, (double)o.param, g))
+                l.gates.push_back(g);
+            else if (o.operation == QMX_OP_CC || (fuseQubits == 0 && undispatched(o.operation)))
+                l.stops.push_back({(int)l.gates.size(), i});
+        }
+        if (fuseQubits < 0 || fuseQubits > 10)
+            qv::raise("Invalid block size. Fused blocks span at least 1 and at most 10 qubits.", __func__);
+        double prob = 1.0;
+        auto stop = [&](int i) {
+            Op o;
+            o.code = ops[i].operation;
+            o.qubits.assign(ops[i].qubits, ops[i].qubits + std::max(0, ops[i].numQubits));
+            o.param = (double)ops[i].param;
+            prob *= runOp(qureg, o);
+        };
+        if (small) {
+            runSmall(d, l, stop);
+            return (qreal)prob;
+        }
+        int at = 0;
+        for (size_t s = 0; s <= l.stops.size(); ++s) {
+            const int until = s < l.stops.size() ? l.stops[s].first : (int)l.gates.size();
+            if (until > at) {
+                qmx::SweepPlan plan;
+                qmx::planSweeps(c.numQubits, qmx::sweepLowBits(d->prec), l.gates.data() + at, until - at, 0, plan);
+                qmx::sweepRunOnce(d, plan, l.gates.data() + at);
+            }
+            at = until;
+            if (s < l.stops.size()) stop(l.stops[s].second);
+        }
+        return (qreal)prob;
     }
     for (int i = 0; i < numOps; ++i)
         recordBasic(&c, ops[i].operation, ops[i].qubits, ops[i].numQubits, (double)ops[i].param, __func__);

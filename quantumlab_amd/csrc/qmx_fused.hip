@@ -409,12 +409,6 @@ __global__ void __launch_bounds__(kBlock, 2) kFused5Tile64(Amp<double> *__restri
     }
 }
 
-struct Fused5Prepared {
-    Fused5Spec spec;
-    float *M;     // device copy of the block's three real 32x32 matrices (Ur, Ui, Ur + Ui)
-    void *form;   // device copy of its tile form
-};
-
 constexpr int kFused5MatrixFloats = 3 * 32 * 32;
 
 // The kernel's form of a 5-qubit block (targs[0] = least significant bit of
@@ -608,22 +602,6 @@ void launchFused5Direct(QuregDev *q, const Fused5Spec &spec, const float *M) {
 
 }  // namespace
 
-// Build the device-resident forms of a 5-qubit block once, for blocks applied
-// many times (circuits): the row-major matrices (registers of 9-10 qubits) and
-// the tile form (11 qubits and more).
-void *fused5Prepare(const int *targs, const Cplx *u) {
-    auto *p = new Fused5Prepared;
-    std::vector<float> hm(kFused5MatrixFloats);
-    fused5Build(targs, u, p->spec, hm.data());
-    std::vector<char> form(kFused5TileFormBytes);
-    tileFormBuild(hm.data(), tileSpecOf(p->spec.targetsSorted), form.data());
-    p->M = static_cast<float *>(devAlloc(hm.size() * sizeof(float)));
-    hostToDevice(p->M, hm.data(), hm.size() * sizeof(float));
-    p->form = devAlloc(form.size());
-    hostToDevice(p->form, form.data(), form.size());
-    return p;
-}
-
 // One application of a block (multiQubitUnitary on an FP32 register): the
 // form the register size needs goes through the staging ring, with no
 // allocation or synchronisation.
@@ -646,22 +624,6 @@ void fused5ApplyOnce(QuregDev *q, const int *targs, const Cplx *u) {
     fused5Build(targs, u, spec, static_cast<float *>(s.host));
     stageCommit(s, bytes, st);
     launchFused5Direct(q, spec, static_cast<const float *>(s.dev));
-}
-
-void fused5Free(void *prepared) {
-    auto *p = static_cast<Fused5Prepared *>(prepared);
-    if (!p) return;
-    devFree(p->M);
-    devFree(p->form);
-    delete p;
-}
-
-// Apply a prepared block to an FP32 register of >= 9 qubits (one 16-group
-// chunk is 512 amplitudes).
-void fused5Apply(QuregDev *q, const void *prepared) {
-    const auto *p = static_cast<const Fused5Prepared *>(prepared);
-    if (q->numQubits >= kTileLog) launchFused5Tile(q, p->spec, p->form);
-    else launchFused5Direct(q, p->spec, p->M);
 }
 
 // One application of an uncontrolled 5-qubit matrix to an FP64 register of

@@ -1,0 +1,80 @@
+// Runs of unitaries applied many to a sweep: the planner (qmx_plan.cpp, host
+// only) and the kernels that carry a plan out (qmx_sweep.hip).
+#pragma once
+
+#include <vector>
+
+#include "qmx_internal.h"
+
+namespace qmx {
+
+// one unitary in matrix form
+struct FlatGate {
+    enum Kind { MATRIX2 = 0, NOT = 1, MATRIXN = 2 };
+    int kind = MATRIX2;
+    int target = 0;                // MATRIX2, NOT
+    uint64_t ctrl = 0;             // controls (all kinds; acts where they are 1)
+    Cplx u[4] = {};                // MATRIX2, row-major
+    int k = 0;                     // MATRIXN: targets (targs[0] = least significant bit), 2^k x 2^k
+    const int *targs = nullptr;
+    const Cplx *uN = nullptr;
+    uint64_t mask() const {
+        uint64_t m = ctrl;
+        if (kind == MATRIXN)
+            for (int j = 0; j < k; ++j) m |= 1ull << targs[j];
+        else
+            m |= 1ull << target;
+        return m;
+    }
+};
+
+// ---- large registers: tiles of 2^kSweepTileBits amplitudes ---------------------
+// A sweep reads and writes the register once. Its tile is kSweepTileBits qubits:
+// the lowest sweepLowBits (whole 128 B lines) and others; every gate of the sweep
+// acts inside the tile, as blocks of 4 or 5 qubits applied one after another in LDS.
+constexpr int kSweepTileBits = 12;
+constexpr int kSweepBlockQubits = 5;
+constexpr int kSweepMaxBlocks = 64;    // blocks of one sweep
+constexpr int kSweepMaxWeight = 512;   // gates of one block (a MATRIXN counts as 64)
+inline int sweepLowBits(int prec) { return prec == FP64 ? 3 : 4; }
+// registers the sweeps serve (smaller ones are one tile: see smallCircuit)
+inline bool sweepSupported(int numQubits) { return numQubits > kSweepTileBits; }
+
+struct SweepBlock {
+    int k;                             // 4 or 5
+    int targs[kSweepBlockQubits];      // qubits, ascending (targs[0] = least significant matrix bit)
+    int firstGate, numGates;           // range of SweepPlan::order
+};
+struct Sweep {
+    uint64_t tile;                     // the tile's qubits
+    int firstBlock, numBlocks;
+    int lone;                          // >= 0: this gate on its own kernel instead
+};
+struct SweepPlan {
+    std::vector<int> order;            // gate indices, block by block
+    std::vector<SweepBlock> blocks;
+    std::vector<Sweep> sweeps;
+};
+// Appends the sweeps of gates[0 .. count) to `plan` (gate indices offset by `base`).
+void planSweeps(int numQubits, int lowBits, const FlatGate *gates, int count, int base, SweepPlan &plan);
+
+// A plan's blocks on the device (matrices built there from the gates).
+struct SweepProgram;
+SweepProgram *sweepProgramCreate(int prec, const SweepPlan &plan, const FlatGate *gates);
+void sweepProgramFree(SweepProgram *p);
+// sweeps [first, last) of the plan
+void sweepProgramRun(QuregDev *q, const SweepProgram *p, const SweepPlan &plan, const FlatGate *gates, int first,
+                     int last);
+// the whole plan once, through the library's workspace (nothing allocated per call)
+void sweepRunOnce(QuregDev *q, const SweepPlan &plan, const FlatGate *gates);
+
+// one gate on its own kernel
+void applyFlatGate(QuregDev *q, const FlatGate &g);
+
+// ---- small registers: the whole register in one workgroup's LDS -----------------
+constexpr int kSmallCircuitQubits = 12;
+inline bool smallCircuitSupported(const QuregDev *q) { return !q->isDensity && q->numQubits <= kSmallCircuitQubits; }
+// gates[0 .. count) in order, one launch per few hundred of them; no MATRIXN
+void smallCircuit(QuregDev *q, const FlatGate *gates, int count);
+
+}  // namespace qmx

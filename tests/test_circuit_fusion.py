@@ -205,3 +205,83 @@ def _relabel(fields, live):
         else:
             out.append(f)
     return out
+
+
+def sweeps_of(host, c, precision):
+    """[(qubits, matrix)] of every block of every sweep, in order, and the number
+    of blocks of each sweep."""
+    out, counts = [], []
+    targs = (C.c_int * 64)()
+    re, im = np.zeros(1 << 20), np.zeros(1 << 20)
+    for sweep in range(1 << 20):
+        for block in range(1 << 20):
+            k = host.lib.qmxCircuitSweepBlock(c, precision, sweep, block, targs, re.ctypes.data_as(host.real_ptr),
+                                              im.ctypes.data_as(host.real_ptr))
+            if k <= 0:
+                break
+            dim = 1 << k
+            out.append((list(targs[:k]), (re[:dim * dim] + 1j * im[:dim * dim]).reshape(dim, dim)))
+        if k < 0:
+            return out, counts
+        counts.append(block)
+
+
+def spread(gates, live):
+    return [(g[0],) + tuple(_relabel(g[1:], live)) for g in gates]
+
+
+@pytest.mark.parametrize("precision", [Q.QMX_PREC_FP64, Q.QMX_PREC_FP32])
+@pytest.mark.parametrize("n,count,live,seed", [
+    (13, 300, None, 1), (14, 5, None, 2), (16, 400, None, 3),          # whole registers, few and many gates
+    (13, 3000, list(range(13)), 4),                                    # far more blocks than one sweep may hold
+    (30, 150, [0, 1, 2, 3, 9, 10, 11, 17, 23, 28, 29], 5),             # scattered: tiles of low and far qubits
+    (40, 150, [7, 12, 13, 19, 20, 26, 31, 32, 33, 38, 39], 6)])        # none of the lowest; past 32 qubits
+def test_sweeps_reproduce_the_gate_list(host, n, count, live, seed, precision):
+    """The blocks of the sweeps, in order, are the gate list's operator: every
+    gate once, no gate moved past one that shares a qubit with it."""
+    m0 = n if live is None else len(live)
+    gates = random_circuit(m0, count, seed)
+    if seed == 3:  # wider than a block: on its own kernel
+        gates.insert(40, ("mqu", [1, 5, 2, 9, 12, 14], W.haar_unitary(np.random.default_rng(8), 64)))
+        gates.insert(90, ("mcu", [0, 3, 6, 8, 11, 13], 2, W.haar_unitary(np.random.default_rng(9), 2)))
+    if live is not None:
+        gates = spread(gates, live)
+    c = W.build_circuit(host, n, gates)
+    try:
+        host.lib.qmxCircuitFuse(c, 5)
+        blocks, counts = sweeps_of(host, c, precision)
+        assert max(counts) <= 64 and sum(counts) == len(blocks)
+        used = sorted(set(range(n) if live is None else live) | {q for qs, _ in blocks for q in qs})
+        m = len(used)
+        assert m <= 20
+        pos = {q: i for i, q in enumerate(used)}
+        rng = np.random.default_rng(seed)
+        psi = rng.standard_normal(1 << m) + 1j * rng.standard_normal(1 << m)
+        want, got = psi.copy(), psi.copy()
+        for g in gates:
+            qs, u = local_gate(g)
+            want = apply_local(want, m, [pos[q] for q in qs], u)
+        for qs, u in blocks:
+            assert qs == sorted(set(qs)) and 0 <= qs[0] and qs[-1] < n
+            got = apply_local(got, m, [pos[q] for q in qs], u)
+        assert np.max(np.abs(got - want)) < 1e-11 * np.max(np.abs(want))
+    finally:
+        host.lib.qmxCircuitDestroy(c)
+
+
+@pytest.mark.parametrize("precision,low", [(Q.QMX_PREC_FP64, 3), (Q.QMX_PREC_FP32, 4)])
+def test_a_sweep_stays_in_its_tile(host, precision, low):
+    """A sweep's blocks together with the lowest qubits span at most 12; the
+    30-qubit brick period makes at most 8 sweeps of 28 blocks."""
+    c = W.build_circuit(host, 30, W.brick_circuit(30, 5, 5, extra_every=5))
+    try:
+        host.lib.qmxCircuitFuse(c, 5)
+        blocks, counts = sweeps_of(host, c, precision)
+        assert len(counts) <= 8 and len(blocks) <= 28
+        at = 0
+        for k in counts:
+            span = set(range(low)).union(*[set(qs) for qs, _ in blocks[at:at + k]])
+            assert len(span) <= 12
+            at += k
+    finally:
+        host.lib.qmxCircuitDestroy(c)

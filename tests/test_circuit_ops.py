@@ -252,3 +252,97 @@ def test_fused_brick_fp32_mfma_matches_oracle(gpu, cpuref, n):
     assert 1 - f < 1e-6
     gpu.destroy(q)
     gpu.qmxCircuitDestroy(c)
+
+
+def _edge_gates(n, count, seed):
+    """Brick and random gates with 2- to 4-control and 2- to 6-target ones where the
+    register has the qubits: every form a tile, an LDS circuit or a lone kernel takes."""
+    rng = np.random.default_rng(seed)
+    gates = W.brick_circuit(n, 2, seed=seed, extra_every=2 if n >= 5 else 0)
+    for i in range(count):
+        qs = [int(x) for x in rng.permutation(n)]
+        kind = i % 6
+        if kind == 0 and n >= 3:
+            c = min(n - 1, 2 + i % 3)
+            gates.append(("mcu", qs[:c], qs[c], W.haar_unitary(rng, 2)))
+        elif kind == 1 and n >= 2 and i % 24 == 1:
+            k = min(n, 2 + (i // 24) % 5)
+            gates.append(("mqu", qs[:k], W.haar_unitary(rng, 1 << k)))
+        elif kind in (2, 3) and n >= 2:
+            gates.append(("cnot", qs[0], qs[1]))
+        elif kind == 4:
+            gates.append(("rz", qs[0], float(rng.uniform(0, 6))))
+        else:
+            a = W.compact_pair(rng)
+            gates.append(("cu", qs[0], *a))
+    return gates
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,count", [(1, 5), (2, 20), (3, 40), (6, 60), (9, 200), (11, 60), (12, 200),
+                                     (13, 3), (13, 400), (14, 150), (17, 300), (20, 150)])
+@pytest.mark.parametrize("precision", [None, QMX_PREC_FP32])
+def test_circuits_at_the_edges_of_their_kernels(gpu, cpuref, n, count, precision):
+    """A recorded circuit applied fused (twice: the prepared blocks serve every
+    application) and unfused, where the register is one workgroup's (n <= 12), the
+    smallest and larger tile sweeps, lists of one and of many sweeps."""
+    gates = _edge_gates(n, count, 900 + n)
+    qc = cpuref.qureg(n)
+    for j in range(n):
+        cpuref.lib.rotateY(qc, j, 0.3 + 0.1 * j)
+    W.apply_gates(cpuref, qc, gates)
+    once = cpuref.state(qc)
+    W.apply_gates(cpuref, qc, gates)
+    twice = cpuref.state(qc)
+    cpuref.destroy(qc)
+    # every gate is unitary: an amplitude's error is at most the sum of the gates'
+    # roundings, a few ulps of an amplitude each (2^-53 or 2^-24)
+    tol = 1e-12 if precision is None else 2.0 ** -22 * np.sqrt(2 * len(gates))
+    for fused in (1, 0):
+        c = W.build_circuit(gpu, n, gates)
+        if fused:
+            assert gpu.qmxCircuitFuse(c, 5) >= 1
+        q = gpu.qureg(n, precision=precision)
+        for j in range(n):
+            gpu.lib.rotateY(q, j, 0.3 + 0.1 * j)
+        for ref in (once, twice):
+            gpu.qmxCircuitApply(q, c, fused)
+            assert np.max(np.abs(gpu.state(q) - ref)) < tol
+        gpu.destroy(q)
+        gpu.qmxCircuitDestroy(c)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [2, 5, 12, 13, 15])
+@pytest.mark.parametrize("fuse", [0, 5])
+def test_operation_lists_with_collapses_between_sweeps(gpu, cpuref, n, fuse):
+    """qmxApplyOperations on lists whose collapses cut the sweeps (and the LDS
+    circuits), with noise and undispatched operations among them: state and
+    probability as the oracle's loop."""
+    rng = np.random.default_rng(n)
+    ops = []
+    for i in range(240):
+        qs = [int(x) for x in rng.permutation(n)[:2]]
+        code = int(rng.choice([O.H, O.X, O.Y, O.Z, O.P, O.RX, O.RY, O.RZ, O.CX, O.CY, O.CZ, O.CP, O.CRX, O.CRY, O.CRZ]))
+        ops.append((code, qs if code >= O.CX else qs[:1], float(rng.uniform(0, 6))))
+        if i in (60, 61, 150):
+            ops.append((O.H, qs[:1], 0.0))
+            ops.append((O.RY, qs[:1], 0.9))
+            ops.append((O.CC, qs[:1], float(i & 1)))
+        if i == 100:
+            ops.append((O.NOISE_DEPHASING, qs[:1], 0.1))
+            ops.append((O.PHASE, qs[:1], 0.2))  # accepted, not dispatched
+    qc = cpuref.qureg(n)
+    want = O.run_ops(cpuref, qc, [o for o in ops if o[0] != O.PHASE])
+    ref = cpuref.state(qc)
+    cpuref.destroy(qc)
+    arr = (BasicOperation * len(ops))()
+    for a, (code, qs, t) in zip(arr, ops):
+        a.operation, a.numQubits, a.param = code, len(qs), t
+        for j, x in enumerate(qs):
+            a.qubits[j] = x
+    q = gpu.qureg(n)
+    got = gpu.qmxApplyOperations(q, arr, len(ops), None, fuse)
+    assert abs(got - want) < TOL
+    assert np.max(np.abs(gpu.state(q) - ref)) < TOL
+    gpu.destroy(q)
