@@ -140,7 +140,7 @@ void planBlocks(std::vector<Item> rem, int base, SweepPlan &plan, std::vector<ui
 void planSweeps(int n, int lowBits, const FlatGate *gates, int count, int base, SweepPlan &plan) {
     std::vector<Item> rem(count);
     for (int i = 0; i < count; ++i) rem[i] = Item{i, gates[i].mask(), weightOf(gates[i])};
-    const int tileBits = std::min(kSweepTileBits, n);
+    const int tileBits = std::min(sweepTileBits(n), n);
     const uint64_t low = (1ull << std::min(lowBits, n)) - 1ull;
     std::vector<int> taken;
     std::vector<Item> mine;

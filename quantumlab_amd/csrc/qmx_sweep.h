@@ -28,17 +28,22 @@ struct FlatGate {
     }
 };
 
-// ---- large registers: tiles of 2^kSweepTileBits amplitudes ---------------------
-// A sweep reads and writes the register once. Its tile is kSweepTileBits qubits:
+// ---- large registers: tiles of 2^sweepTileBits amplitudes -----------------------
+// A sweep reads and writes the register once. Its tile is sweepTileBits qubits:
 // the lowest sweepLowBits (whole 128 B lines) and others; every gate of the sweep
 // acts inside the tile, as blocks of 4 or 5 qubits applied one after another in LDS.
+// 12 qubits, and 11 where tiles of 12 would leave CUs without a workgroup: up to 19
+// qubits a tile of half the size takes half the time a block, for one sweep more in
+// six (300 random operations on 17 qubits).
 constexpr int kSweepTileBits = 12;
+constexpr int sweepTileBits(int numQubits) { return numQubits < 20 ? kSweepTileBits - 1 : kSweepTileBits; }
 constexpr int kSweepBlockQubits = 5;
 constexpr int kSweepMaxBlocks = 64;    // blocks of one sweep
 constexpr int kSweepMaxWeight = 512;   // gates of one block (a MATRIXN counts as 64)
 inline int sweepLowBits(int prec) { return prec == FP64 ? 3 : 4; }
 // registers the sweeps serve (smaller ones are one tile: see smallCircuit)
-inline bool sweepSupported(int numQubits) { return numQubits > kSweepTileBits; }
+constexpr int kSmallCircuitQubits = 12;
+inline bool sweepSupported(int numQubits) { return numQubits > kSmallCircuitQubits; }
 
 struct SweepBlock {
     int k;                             // 4 or 5
@@ -72,7 +77,6 @@ void sweepRunOnce(QuregDev *q, const SweepPlan &plan, const FlatGate *gates);
 void applyFlatGate(QuregDev *q, const FlatGate &g);
 
 // ---- small registers: the whole register in one workgroup's LDS -----------------
-constexpr int kSmallCircuitQubits = 12;
 inline bool smallCircuitSupported(const QuregDev *q) { return !q->isDensity && q->numQubits <= kSmallCircuitQubits; }
 // gates[0 .. count) in order, one launch per few hundred of them; no MATRIXN
 void smallCircuit(QuregDev *q, const FlatGate *gates, int count);

@@ -19,7 +19,10 @@
 // flops an amplitude, which HBM takes 1.7 times as long for as the matrix cores
 // do; two or three blocks a sweep bring the two to the same time. 4-qubit blocks
 // take half a 5-qubit block's arithmetic and absorb two thirds of its gates, so
-// the planner prefers them. Measured per five-layer brick period: MEASURED_TABLE
+// the planner prefers them. Five-layer brick period, one block a sweep before and
+// now: 30 qubits FP32 50.9 -> 30.2 ms (16 sweeps -> 7, of 25 4-qubit blocks), 27 qubits
+// FP64 12.4 -> 7.2 ms. Seven blocks a sweep keep the matrix cores busy 70 % of the
+// time, two leave it to HBM (3.1 ms for 16 GiB).
 //
 // Operand placement (16x16x4, wave64; lane = 16 kq + col):
 //   A: lane holds U[r][4 st + kq] of its row r, one fragment per step st;
@@ -50,19 +53,56 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef double d2 __attribute__((ext_vector_type(2)));
 typedef double d4 __attribute__((ext_vector_type(4)));
 
-constexpr int kTB = kSweepTileBits;
+constexpr int kMaxTB = kSweepTileBits;
 
 // ---- block matrices, built on the device ---------------------------------------
+typedef double d8 __attribute__((ext_vector_type(8)));
+
 struct GateDev {
     int kind;            // FlatGate::Kind
-    int t;               // target, a bit of the block's index
+    unsigned t;          // target, a bit of the block's index; MATRIXN: its targets, 4 bits each
     unsigned ctrl;       // controls, bits of the block's index
     int k;               // MATRIXN
-    int lt[kSweepBlockQubits];
     int mat;             // MATRIXN: its matrix (entry offset)
-    Amp<double> u[4];
+    int pad[3];
+    alignas(16) double u[8];  // the matrix, (re, im) by rows
 };
-static_assert(sizeof(GateDev) == 112, "no uninitialised tail");
+
+// gates staged in LDS at a time (whole coalesced loads; one entry more is read)
+constexpr int kStage = 64;
+template <typename G>
+__device__ __forceinline__ void stageGates(G *stage, const G *__restrict__ src, int num, int tid, int threads) {
+    static_assert(sizeof(G) % 16 == 0, "gates move in 16 B pieces");
+    const uint4 *from = reinterpret_cast<const uint4 *>(src);
+    for (int i = tid; i < num * (int)(sizeof(G) / 16); i += threads) reinterpret_cast<uint4 *>(stage)[i] = from[i];
+}
+
+// a staged gate's matrix as one vector value (indexed as an array, entries that
+// differ between branches end up in scratch memory)
+__device__ __forceinline__ d8 matrixOf(const double *u) {
+    const d2 *v = reinterpret_cast<const d2 *>(u);
+    const d2 a = v[0], b = v[1], c = v[2], d = v[3];
+    return d8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
+}
+
+__device__ __forceinline__ unsigned uniform(unsigned x) { return (unsigned)__builtin_amdgcn_readfirstlane((int)x); }
+
+// the gate with its integers in scalar registers (every lane holds the same gate)
+__device__ __forceinline__ GateDev uniformGate(const GateDev &g) {
+    GateDev r = g;
+    r.kind = (int)uniform((unsigned)g.kind);
+    r.t = uniform(g.t);
+    r.ctrl = uniform(g.ctrl);
+    r.k = (int)uniform((unsigned)g.k);
+    r.mat = (int)uniform((unsigned)g.mat);
+    return r;
+}
+
+// u0 p + u1 q of a gate's row (u0, u1) = (u[0] + i u[1], u[2] + i u[3])
+__device__ __forceinline__ Amp<double> rowTimes(double a, double b, double c, double d, const Amp<double> &p,
+                                                const Amp<double> &q) {
+    return Amp<double>{a * p.x - b * p.y + c * q.x - d * q.y, a * p.y + b * p.x + c * q.y + d * q.x};
+}
 struct BuildDev {
     int firstGate, numGates, k, pad;
     // byte offsets of the LDS slots: column bits, combination bits 0 and 1,
@@ -81,74 +121,72 @@ template <typename T> struct Frag;
 template <> struct Frag<float> { typedef f4 V; };
 template <> struct Frag<double> { typedef d2 V; };
 
-// One workgroup per block: the product of its gates in FP64, column by column of
-// the identity, in LDS; then the matrix-core fragments. The gates arrive as the
-// host recorded them, so a list of any length costs one small copy instead of a
-// matrix per block (on the host a block of ten gates took ~25 us).
+// One workgroup per block: the product of its gates in FP64, in LDS, then the
+// block's vectors. The gates arrive as the host recorded them, so a list of any
+// length costs one small copy instead of a matrix per block (on the host a block
+// of ten gates took ~25 us). A wave owns a quarter of the matrix's columns, which no
+// other wave touches, so gates follow one another without barriers; each gate is
+// read from LDS while the one before it is applied (scalar loads straight from
+// memory arrive a line at a time, 0.65 us a gate).
 template <typename T>
 __global__ void __launch_bounds__(kBlock) kBuildBlocks(const BuildDev *__restrict__ todo,
                                                        const GateDev *__restrict__ gates,
                                                        const Amp<double> *__restrict__ mats, char *__restrict__ out) {
-    // gates staged in LDS at a time (a scalar load of each on the critical path
-    // made a block of 15 gates 23 us)
-    constexpr int kStage = 32;
-    static_assert(sizeof(GateDev) % 16 == 0, "gates move in 16 B pieces");
     __shared__ Amp<double> buf[2][32 * 32];
-    __shared__ GateDev stage[kStage];
-    const BuildDev b = todo[blockIdx.x];
-    const int k = b.k, dim = 1 << k, tid = threadIdx.x;
+    __shared__ GateDev stage[kStage + 1];
+    const BuildDev &b = todo[blockIdx.x];
+    const int k = b.k, dim = 1 << k, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     Amp<double> *M = buf[0], *N = buf[1];
     for (int i = tid; i < dim * dim; i += kBlock) M[i] = Amp<double>{(i >> k) == (i & (dim - 1)) ? 1.0 : 0.0, 0.0};
-    __syncthreads();
+    // pairs of a wave: dim/4 columns x dim/2 row pairs, 32 (k = 4) or 128 (k = 5)
+    const int cb = k - 2, col = wave * (dim / 4) + (lane & ((1 << cb) - 1)), pairs = dim / 2;
+    GateDev next{};
     for (int g = 0; g < b.numGates; ++g) {
         if (g % kStage == 0) {
-            const int words = min(kStage, b.numGates - g) * (int)(sizeof(GateDev) / 16);
-            const uint4 *src = reinterpret_cast<const uint4 *>(gates + b.firstGate + g);
-            for (int i = tid; i < words; i += kBlock) reinterpret_cast<uint4 *>(stage)[i] = src[i];
             __syncthreads();
+            stageGates(stage, gates + b.firstGate + g, min(kStage, b.numGates - g), tid, kBlock);
+            __syncthreads();
+            next = stage[0];
         }
-        const GateDev &G = stage[g % kStage];
-        const unsigned ctrl = (unsigned)__builtin_amdgcn_readfirstlane((int)G.ctrl);
-        const int kind = __builtin_amdgcn_readfirstlane(G.kind);
-        if (kind != FlatGate::MATRIXN) {
-            const int t = __builtin_amdgcn_readfirstlane(G.t);
-            const bool isNot = kind == FlatGate::NOT;
-            const Amp<double> u0 = G.u[0], u1 = G.u[1], u2 = G.u[2], u3 = G.u[3];
-            for (int i = tid; i < dim * dim / 2; i += kBlock) {
-                const int col = i & (dim - 1);
-                const unsigned r0 = (unsigned)insertZero((uint64_t)(i >> k), t), r1 = r0 | (1u << t);
-                if ((r0 & ctrl) != ctrl) continue;
-                const Amp<double> x = M[r0 * dim + col], y = M[r1 * dim + col];
-                if (isNot) {
-                    M[r0 * dim + col] = y;
-                    M[r1 * dim + col] = x;
+        const GateDev G = uniformGate(next);
+        next = stage[g % kStage + 1];  // past a stage's last one: unused
+        if (G.kind != FlatGate::MATRIXN) {
+            // row r0 of pair p: p with a zero inserted at the target
+            const unsigned bit = 1u << G.t, high = ~(bit - 1u);
+            for (unsigned p = lane >> cb; p < (unsigned)pairs; p += 64 >> cb) {
+                const unsigned r0 = p + (p & high);
+                if ((r0 & G.ctrl) != G.ctrl) continue;
+                Amp<double> *px = M + (r0 << k) + col, *py = px + (bit << k);
+                const Amp<double> x = *px, y = *py;
+                if (G.kind == FlatGate::NOT) {
+                    *px = y;
+                    *py = x;
                 } else {
-                    M[r0 * dim + col] = Amp<double>{u0.x * x.x - u0.y * x.y + u1.x * y.x - u1.y * y.y,
-                                                    u0.x * x.y + u0.y * x.x + u1.x * y.y + u1.y * y.x};
-                    M[r1 * dim + col] = Amp<double>{u2.x * x.x - u2.y * x.y + u3.x * y.x - u3.y * y.y,
-                                                    u2.x * x.y + u2.y * x.x + u3.x * y.y + u3.y * y.x};
+                    *px = rowTimes(G.u[0], G.u[1], G.u[2], G.u[3], x, y);
+                    *py = rowTimes(G.u[4], G.u[5], G.u[6], G.u[7], x, y);
                 }
             }
-            __syncthreads();
+            // LDS accesses of one wave complete in order; keep the compiler's too
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
             continue;
         }
         const int gk = G.k, gd = 1 << gk;
         const Amp<double> *U = mats + G.mat;
-        for (int i = tid; i < dim * dim; i += kBlock) {
-            const int col = i & (dim - 1);
-            const unsigned r = (unsigned)(i >> k);
+        for (int r = lane >> cb; r < dim; r += 64 >> cb) {
             Amp<double> s = M[r * dim + col];
-            if ((r & ctrl) == ctrl) {
-                unsigned base = r;
+            if (((unsigned)r & G.ctrl) == G.ctrl) {
+                unsigned base = (unsigned)r;
                 int row = 0;
                 for (int j = 0; j < gk; ++j) {
-                    row |= (int)((r >> G.lt[j]) & 1u) << j;
-                    base &= ~(1u << G.lt[j]);
+                    const unsigned q = (G.t >> (4 * j)) & 15u;
+                    row |= ((r >> q) & 1) << j;
+                    base &= ~(1u << q);
                 }
                 s = Amp<double>{0.0, 0.0};
                 for (int c = 0; c < gd; ++c) {
                     unsigned rc = base;
-                    for (int j = 0; j < gk; ++j) rc |= ((unsigned)(c >> j) & 1u) << G.lt[j];
+                    for (int j = 0; j < gk; ++j) rc |= ((unsigned)(c >> j) & 1u) << ((G.t >> (4 * j)) & 15u);
                     const Amp<double> u = U[row * gd + c], x = M[rc * dim + col];
                     s.x += u.x * x.x - u.y * x.y;
                     s.y += u.x * x.y + u.y * x.x;
@@ -156,11 +194,13 @@ __global__ void __launch_bounds__(kBlock) kBuildBlocks(const BuildDev *__restric
             }
             N[r * dim + col] = s;
         }
-        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         Amp<double> *sw = M;
         M = N;
         N = sw;
     }
+    __syncthreads();
     // fragment (h steps + st) of each of the three matrices: Ur, Ui, Ur + Ui in FP32,
     // Ur, -(Ur + Ui), Ui - Ur in FP64
     char *dst = out + (size_t)blockIdx.x * kBlockBytes;
@@ -208,7 +248,7 @@ struct BlockDev {
 };
 
 struct TileGeom {
-    int pos[kTB];        // the tile's qubits, ascending
+    int pos[kMaxTB];     // the tile's qubits, ascending
     uint64_t jAddr[16];  // register offset of a thread's j-th transfer
     unsigned jSlot[16];  // its slot's part from j (bytes)
 };
@@ -237,11 +277,12 @@ template <> struct Acc4<double> { typedef d4 type; };
 
 // A block of K qubits on the chunks of one wave, IL chunks at a time: v holds the
 // block's vectors, s0 the slot of each chunk of the wave.
-template <typename T, int K, int WAVES>
+template <typename T, int K, int WAVES, int TB>
 __device__ __forceinline__ void blockChunks(char *tile, const typename Frag<T>::V *v, const BlockDev &B, int wave) {
     typedef typename Acc4<T>::type A;
     constexpr int S = 1 << (K - 2), H = K == 5 ? 2 : 1, PV = 16 / sizeof(T), NV = H * S / PV, SV = S / 4;
-    constexpr int CH = (1 << (kTB - 4 - K)) / WAVES, IL = K == 5 ? 1 : 2;
+    constexpr int CH = (1 << (TB - 4 - K)) / WAVES, IL = K == 5 ? 1 : 2;
+    static_assert(CH % IL == 0, "every wave has whole runs of chunks");
     unsigned slot[S];
 #pragma unroll
     for (int i = 0; i < SV; ++i) {
@@ -261,7 +302,7 @@ __device__ __forceinline__ void blockChunks(char *tile, const typename Frag<T>::
             const int ch = wave + WAVES * (c0 + l);
             s0[l] = 0;
 #pragma unroll
-            for (int b = 0; b < kTB - 4 - K; ++b) s0[l] ^= ((ch >> b) & 1) ? B.rest[b] : 0u;
+            for (int b = 0; b < TB - 4 - K; ++b) s0[l] ^= ((ch >> b) & 1) ? B.rest[b] : 0u;
         }
         Amp<T> x[IL][S];
 #pragma unroll
@@ -335,18 +376,18 @@ __device__ __forceinline__ void blockChunks(char *tile, const typename Frag<T>::
     }
 }
 
-template <typename T, bool NT, int WAVES>
+template <typename T, bool NT, int WAVES, int TB>
 __global__ void __launch_bounds__(64 * WAVES, sizeof(T) == 4 ? 4 : 2)
     kTileSweep(Amp<T> *__restrict__ a, TileGeom geo, const BlockDev *__restrict__ blocks, int numBlocks,
                const char *__restrict__ frags) {
     // a thread moves 16 B at a time: two FP32 amplitudes or one FP64
-    constexpr int PAIR = sizeof(T) == 4 ? 1 : 0, THREADS = 6 + (WAVES == 8 ? 3 : 2), J = 1 << (kTB - THREADS - PAIR);
+    constexpr int PAIR = sizeof(T) == 4 ? 1 : 0, THREADS = 6 + (WAVES == 8 ? 3 : 2), J = 1 << (TB - THREADS - PAIR);
     typedef typename Frag<T>::V V;
-    __shared__ __attribute__((aligned(16))) char tile[sizeof(Amp<T>) << kTB];
+    __shared__ __attribute__((aligned(16))) char tile[sizeof(Amp<T>) << TB];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     uint64_t addr = (uint64_t)flatBlock();
 #pragma unroll
-    for (int i = 0; i < kTB; ++i) addr = insertZero(addr, geo.pos[i]);
+    for (int i = 0; i < TB; ++i) addr = insertZero(addr, geo.pos[i]);
 #pragma unroll
     for (int i = 0; i < THREADS; ++i)
         if ((tid >> i) & 1) addr |= 1ull << geo.pos[i + PAIR];
@@ -387,9 +428,9 @@ __global__ void __launch_bounds__(64 * WAVES, sizeof(T) == 4 ? 4 : 2)
         if (B.k == 5) {
 #pragma unroll
             for (int i = V4; i < V5; ++i) v[i] = mineB[i * 64];
-            blockChunks<T, 5, WAVES>(tile, v, B, wave);
+            blockChunks<T, 5, WAVES, TB>(tile, v, B, wave);
         } else {
-            blockChunks<T, 4, WAVES>(tile, v, B, wave);
+            blockChunks<T, 4, WAVES, TB>(tile, v, B, wave);
         }
         B = nB;
         __syncthreads();
@@ -414,102 +455,72 @@ __global__ void __launch_bounds__(64 * WAVES, sizeof(T) == 4 ? 4 : 2)
 // ---- small registers -----------------------------------------------------------------
 // The register (2^n amplitudes, n <= 12) stays in one workgroup's LDS, in FP64 for
 // both storage precisions, while every gate of the list is applied: a circuit is
-// one launch, rounded to FP32 once at its end. Gates run in groups whose targets
-// are at most two qubits: a thread holds the four amplitudes of those two (a
-// "quad"), applies the group's gates in registers and writes them back, so a
-// group costs one LDS round trip and one barrier. Controls may be any qubits.
-// Nothing but that chain bounds it (one workgroup): SMALL_MEASURED
+// one launch, rounded to FP32 once at its end. One pair of amplitudes a thread (two
+// at 12 qubits), one barrier a gate. Nothing but a gate's own chain bounds it (one
+// workgroup): its constants, read from LDS while the gate before it runs, the
+// pair's LDS reads, the products, the writes, the barrier; so the code of a gate is
+// kept short: 0.3 us a gate up to 9 qubits, 0.4 at 10, 0.8 at 12. 80 operations on
+// 10 qubits take 34 us here; as 10 fused blocks of a launch each they took 45 us on
+// the device and 340 us with the host's part of each block.
 struct SmallGate {
-    int group;                   // > 0: opens a group with this many gates on qubits (t0, t1)
-    int t0, t1;                  // the group's qubits, ascending
-    int target;                  // 0: t0, 1: t1
-    int kind;                    // SG_*
-    unsigned ctrl;               // controls, bits of the register index
-    Amp<double> u[4];
+    unsigned what;               // SG_*
+    unsigned bit;                // the target's bit, as a byte offset of the LDS register (16 B an amplitude)
+    unsigned ctrl;               // the controls' bits, likewise
+    unsigned pad;
+    alignas(16) double u[8];     // the matrix, (re, im) by rows
 };
-enum { SG_GENERAL = 0, SG_NOT = 1, SG_DIAGONAL = 2, SG_REAL = 3 };
-
-// gates staged in LDS at a time (coalesced loads once, instead of a scalar load
-// of each gate on the critical path)
-constexpr int kSmallStage = 64;
-constexpr int kSmallThreads = 512;
-
-__device__ __forceinline__ void smallPair(const SmallGate &G, int kind, Amp<double> &x, Amp<double> &y) {
-    const Amp<double> p = x, q = y;
-    switch (kind) {
-    case SG_NOT:
-        x = q;
-        y = p;
-        break;
-    case SG_DIAGONAL: {
-        const Amp<double> a = G.u[0], d = G.u[3];
-        if (a.x != 1.0 || a.y != 0.0) x = Amp<double>{a.x * p.x - a.y * p.y, a.x * p.y + a.y * p.x};
-        y = Amp<double>{d.x * q.x - d.y * q.y, d.x * q.y + d.y * q.x};
-        break;
-    }
-    case SG_REAL:
-        x = Amp<double>{G.u[0].x * p.x + G.u[1].x * q.x, G.u[0].x * p.y + G.u[1].x * q.y};
-        y = Amp<double>{G.u[2].x * p.x + G.u[3].x * q.x, G.u[2].x * p.y + G.u[3].x * q.y};
-        break;
-    default: {
-        const Amp<double> a = G.u[0], b = G.u[1], c = G.u[2], d = G.u[3];
-        x = Amp<double>{a.x * p.x - a.y * p.y + b.x * q.x - b.y * q.y, a.x * p.y + a.y * p.x + b.x * q.y + b.y * q.x};
-        y = Amp<double>{c.x * p.x - c.y * p.y + d.x * q.x - d.y * q.y, c.x * p.y + c.y * p.x + d.x * q.y + d.y * q.x};
-    }
-    }
-}
+enum { SG_GENERAL = 0, SG_NOT = 1, SG_PHASE = 2, SG_REAL = 3 };  // SG_PHASE: diag(1, u)
+constexpr int kSmallStage = 256;
+constexpr int kSmallThreads = 1024;
 
 template <typename T>
 __global__ void __launch_bounds__(kSmallThreads) kSmallCircuit(Amp<T> *__restrict__ a, int n,
                                                                const SmallGate *__restrict__ gates, int numGates) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    // n = 1 runs as two qubits whose upper half stays zero
-    const int nn = n < 2 ? 2 : n;
-    const unsigned dim = 1u << n, step = blockDim.x, quads = 1u << (nn - 2);
-    Amp<double> *s = reinterpret_cast<Amp<double> *>(smem);
-    SmallGate *stage = reinterpret_cast<SmallGate *>(smem + (sizeof(Amp<double>) << nn));
-    for (unsigned i = threadIdx.x; i < 1u << nn; i += step)
-        s[i] = i < dim ? Amp<double>{(double)a[i].x, (double)a[i].y} : Amp<double>{0, 0};
-    for (int g0 = 0; g0 < numGates;) {
-        // whole groups only: the host cuts groups at multiples of the stage
-        const int num = min(kSmallStage, numGates - g0);
-        const unsigned words = num * sizeof(SmallGate) / 16;
-        const uint4 *src = reinterpret_cast<const uint4 *>(gates + g0);
-        uint4 *dst = reinterpret_cast<uint4 *>(stage);
-        for (unsigned i = threadIdx.x; i < words; i += step) dst[i] = src[i];
-        __syncthreads();
-        for (int g = 0; g < num;) {
-            // the same in every lane: read into scalar registers
-            const int count = __builtin_amdgcn_readfirstlane(stage[g].group);
-            const int t0 = __builtin_amdgcn_readfirstlane(stage[g].t0), t1 = __builtin_amdgcn_readfirstlane(stage[g].t1);
-            const unsigned b0 = 1u << t0, b1 = 1u << t1;
-            for (unsigned w = threadIdx.x; w < quads; w += step) {
-                unsigned i = ((w >> t0) << (t0 + 1)) | (w & (b0 - 1u));
-                i = ((i >> t1) << (t1 + 1)) | (i & (b1 - 1u));
-                Amp<double> x00 = s[i], x01 = s[i | b0], x10 = s[i | b1], x11 = s[i | b0 | b1];
-                for (int e = 0; e < count; ++e) {
-                    const SmallGate &G = stage[g + e];
-                    const unsigned c = (unsigned)__builtin_amdgcn_readfirstlane((int)G.ctrl);
-                    const int kind = __builtin_amdgcn_readfirstlane(G.kind);
-                    if (__builtin_amdgcn_readfirstlane(G.target) == 0) {
-                        if ((i & c) == c) smallPair(G, kind, x00, x01);
-                        if (((i | b1) & c) == c) smallPair(G, kind, x10, x11);
-                    } else {
-                        if ((i & c) == c) smallPair(G, kind, x00, x10);
-                        if (((i | b0) & c) == c) smallPair(G, kind, x01, x11);
-                    }
-                }
-                s[i] = x00;
-                s[i | b0] = x01;
-                s[i | b1] = x10;
-                s[i | b0 | b1] = x11;
-            }
-            g += count;
+    const unsigned dim = 1u << n, step = blockDim.x, tid = threadIdx.x;
+    SmallGate *stage = reinterpret_cast<SmallGate *>(smem + (sizeof(Amp<double>) << n));
+    auto at = [&](unsigned off) -> Amp<double> & { return *reinterpret_cast<Amp<double> *>(smem + off); };
+    for (unsigned i = tid; i < dim; i += step) at(16u * i) = Amp<double>{(double)a[i].x, (double)a[i].y};
+    uint4 nextHead{};
+    d8 nextU = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int g = 0; g < numGates; ++g) {
+        if (g % kSmallStage == 0) {
             __syncthreads();
+            stageGates(stage, gates + g, min(kSmallStage, numGates - g), (int)tid, (int)step);
+            __syncthreads();
+            nextHead = *reinterpret_cast<const uint4 *>(stage);
+            nextU = matrixOf(stage[0].u);
         }
-        g0 += num;
+        const unsigned what = uniform(nextHead.x), bit = uniform(nextHead.y), ctrl = uniform(nextHead.z);
+        const unsigned high = ~(bit - 1u);
+        const d8 u = nextU;
+        // past a stage's last one: unused
+        nextHead = *reinterpret_cast<const uint4 *>(stage + g % kSmallStage + 1);
+        nextU = matrixOf(stage[g % kSmallStage + 1].u);
+        for (unsigned w = 16u * tid; w < 8u * dim; w += 16u * step) {
+            const unsigned i = w + (w & high);  // the pair's index with a zero inserted at the target
+            if ((i & ctrl) != ctrl) continue;
+            Amp<double> &X = at(i), &Y = at(i + bit);
+            if (what == SG_NOT) {
+                const Amp<double> x = X, y = Y;
+                X = y;
+                Y = x;
+            } else if (what == SG_PHASE) {
+                const Amp<double> y = Y;
+                Y = Amp<double>{u[6] * y.x - u[7] * y.y, u[6] * y.y + u[7] * y.x};
+            } else if (what == SG_REAL) {
+                const Amp<double> x = X, y = Y;
+                X = Amp<double>{u[0] * x.x + u[2] * y.x, u[0] * x.y + u[2] * y.y};
+                Y = Amp<double>{u[4] * x.x + u[6] * y.x, u[4] * x.y + u[6] * y.y};
+            } else {
+                const Amp<double> x = X, y = Y;
+                X = rowTimes(u[0], u[1], u[2], u[3], x, y);
+                Y = rowTimes(u[4], u[5], u[6], u[7], x, y);
+            }
+        }
+        __syncthreads();
     }
-    for (unsigned i = threadIdx.x; i < dim; i += step) a[i] = Amp<T>{(T)s[i].x, (T)s[i].y};
+    for (unsigned i = tid; i < dim; i += step) a[i] = Amp<T>{(T)at(16u * i).x, (T)at(16u * i).y};
 }
 
 // ---- host side -----------------------------------------------------------------------
@@ -575,38 +586,44 @@ void fillBuild(const SweepPlan &plan, const FlatGate *gates, int firstBlock, int
             for (uint64_t m = f.ctrl; m; m &= m - 1) d.ctrl |= 1u << local(__builtin_ctzll(m));
             if (f.kind == FlatGate::MATRIXN) {
                 d.k = f.k;
-                for (int j = 0; j < f.k; ++j) d.lt[j] = local(f.targs[j]);
+                for (int j = 0; j < f.k; ++j) d.t |= (unsigned)local(f.targs[j]) << (4 * j);
                 d.mat = mat;
                 const int entries = 1 << (2 * f.k);
                 for (int e = 0; e < entries; ++e) mats[mat + e] = Amp<double>{f.uN[e].re, f.uN[e].im};
                 mat += entries;
             } else {
-                d.t = local(f.target);
-                for (int e = 0; e < 4; ++e) d.u[e] = Amp<double>{f.u[e].re, f.u[e].im};
+                d.t = (unsigned)local(f.target);
+                for (int e = 0; e < 4; ++e) {
+                    d.u[2 * e] = f.u[e].re;
+                    d.u[2 * e + 1] = f.u[e].im;
+                }
             }
         }
     }
 }
 
-void tilePositions(uint64_t tile, int pos[kTB]) {
-    int n = 0;
-    for (uint64_t m = tile; m && n < kTB; m &= m - 1) pos[n++] = __builtin_ctzll(m);
-    if (n != kTB || __builtin_popcountll(tile) != kTB) {
-        std::fprintf(stderr, "libquest_mi355x: a planned tile has %d qubits\n", __builtin_popcountll(tile));
+// the tile's qubits, ascending; returns how many
+int tilePositions(uint64_t tile, int pos[kMaxTB]) {
+    const int bits = __builtin_popcountll(tile);
+    if (bits != kMaxTB && bits != kMaxTB - 1) {
+        std::fprintf(stderr, "libquest_mi355x: a planned tile has %d qubits\n", bits);
         std::abort();
     }
+    int n = 0;
+    for (uint64_t m = tile; m; m &= m - 1) pos[n++] = __builtin_ctzll(m);
+    return n;
 }
 
 template <typename T>
-void blockSlots(const SweepBlock &b, const int pos[kTB], BuildDev &todo, BlockDev &d) {
+void blockSlots(const SweepBlock &b, const int *pos, int tb, BuildDev &todo, BlockDev &d) {
     constexpr int R = sizeof(T) == 4 ? 4 : 3;   // columns per bank cycle: 2^R lanes
     d = BlockDev{};
     d.k = b.k;
     int t[kSweepBlockQubits];
-    bool used[kTB] = {};
+    bool used[kMaxTB] = {};
     for (int j = 0; j < b.k; ++j) {
         t[j] = -1;
-        for (int i = 0; i < kTB; ++i)
+        for (int i = 0; i < tb; ++i)
             if (pos[i] == b.targs[j]) t[j] = i;
         if (t[j] < 0) {
             std::fprintf(stderr, "libquest_mi355x: a planned block leaves its tile\n");
@@ -617,12 +634,12 @@ void blockSlots(const SweepBlock &b, const int pos[kTB], BuildDev &todo, BlockDe
     // columns: the first R take tile bits of different residues modulo R
     int cols[4], nc = 0;
     bool residue[4] = {};
-    for (int i = 0; i < kTB && nc < R; ++i)
+    for (int i = 0; i < tb && nc < R; ++i)
         if (!used[i] && !residue[i % R]) {
             residue[i % R] = used[i] = true;
             cols[nc++] = i;
         }
-    for (int i = 0; i < kTB && nc < 4; ++i)
+    for (int i = 0; i < tb && nc < 4; ++i)
         if (!used[i]) {
             used[i] = true;
             cols[nc++] = i;
@@ -633,7 +650,7 @@ void blockSlots(const SweepBlock &b, const int pos[kTB], BuildDev &todo, BlockDe
     for (int st = 0; st < 1 << (b.k - 2); ++st)
         for (int j = 2; j < b.k; ++j)
             if ((st >> (j - 2)) & 1) todo.st[st] ^= slot(t[j]);
-    for (int i = 0, r = 0; i < kTB; ++i)
+    for (int i = 0, r = 0; i < tb; ++i)
         if (!used[i]) d.rest[r++] = slot(i);
 }
 
@@ -644,10 +661,10 @@ void fillBlocks(int prec, const SweepPlan &plan, int first, int last, int firstB
     for (int s = first; s < last; ++s) {
         const Sweep &w = plan.sweeps[s];
         if (w.lone >= 0) continue;
-        int pos[kTB];
-        tilePositions(w.tile, pos);
+        int pos[kMaxTB];
+        const int tb = tilePositions(w.tile, pos);
         for (int b = w.firstBlock; b < w.firstBlock + w.numBlocks; ++b)
-            QMX_DISPATCH(prec, T, { blockSlots<T>(plan.blocks[b], pos, todo[b - firstBlock], out[b - firstBlock]); });
+            QMX_DISPATCH(prec, T, { blockSlots<T>(plan.blocks[b], pos, tb, todo[b - firstBlock], out[b - firstBlock]); });
     }
 }
 
@@ -661,36 +678,41 @@ void launchBuild(int prec, int numBlocks, const Upload &u, char *dev, char *frag
     checkLaunch("sweep block matrices");
 }
 
-template <typename T, int WAVES>
-void launchSweepWaves(QuregDev *q, const Sweep &w, const BlockDev *blocks, const char *frags) {
-    constexpr int PAIR = sizeof(T) == 4 ? 1 : 0, THREADS = 6 + (WAVES == 8 ? 3 : 2), J = 1 << (kTB - THREADS - PAIR);
+template <typename T, bool NT, int WAVES, int TB>
+void launchTiles(QuregDev *q, const Sweep &w, const BlockDev *blocks, const char *frags) {
+    constexpr int PAIR = sizeof(T) == 4 ? 1 : 0, THREADS = 6 + (WAVES == 8 ? 3 : 2), J = 1 << (TB - THREADS - PAIR);
     TileGeom geo{};
-    tilePositions(w.tile, geo.pos);
+    if (tilePositions(w.tile, geo.pos) != TB) {
+        std::fprintf(stderr, "libquest_mi355x: a sweep's tile does not have %d qubits\n", TB);
+        std::abort();
+    }
     for (int j = 0; j < J; ++j)
-        for (int i = 0; THREADS + PAIR + i < kTB; ++i)
+        for (int i = 0; THREADS + PAIR + i < TB; ++i)
             if ((j >> i) & 1) {
                 geo.jAddr[j] |= 1ull << geo.pos[THREADS + PAIR + i];
                 geo.jSlot[j] ^= slotBit<T>(THREADS + PAIR + i) * (unsigned)sizeof(Amp<T>);
             }
-    // streaming accesses where the register outgrows the last-level cache
-    const bool nt = q->numAmps * (long long)sizeof(Amp<T>) > (256ll << 20);
-    const dim3 grid = gridOf(q->numAmps >> kTB);
-    if (nt)
-        hipLaunchKernelGGL((kTileSweep<T, true, WAVES>), grid, dim3(64 * WAVES), 0, hstream(), (Amp<T> *)q->amps, geo,
-                           blocks, w.numBlocks, frags);
-    else
-        hipLaunchKernelGGL((kTileSweep<T, false, WAVES>), grid, dim3(64 * WAVES), 0, hstream(), (Amp<T> *)q->amps,
-                           geo, blocks, w.numBlocks, frags);
+    hipLaunchKernelGGL((kTileSweep<T, NT, WAVES, TB>), gridOf(q->numAmps >> TB), dim3(64 * WAVES), 0, hstream(),
+                       (Amp<T> *)q->amps, geo, blocks, w.numBlocks, frags);
     checkLaunch("tile sweep");
 }
 
-// Eight waves a tile where the register has too few tiles to fill the CUs with
-// four (4 workgroups of 32 KiB, or 2 of 64, fit a CU): WAVES_MEASURED
+// Four waves a tile; eight where tiles of 12 qubits are too few to fill the CUs with
+// workgroups of four (4 of 32 KiB or 2 of 64 KiB fit a CU; eight waves on large
+// registers: 33.6 instead of 30.8 ms for the 30-qubit FP32 period, 9.8 instead of
+// 7.7 for the 27-qubit FP64 one). Nontemporal accesses where the register outgrows
+// the last-level cache.
 template <typename T>
 void launchSweep(QuregDev *q, const Sweep &w, const BlockDev *blocks, const char *frags) {
     constexpr int perCU = sizeof(T) == 4 ? 4 : 2;
-    if ((q->numAmps >> kTB) < (long long)perCU * numCUs()) launchSweepWaves<T, 8>(q, w, blocks, frags);
-    else launchSweepWaves<T, 4>(q, w, blocks, frags);
+    if (sweepTileBits(q->numQubits) < kSweepTileBits)
+        launchTiles<T, false, 4, kSweepTileBits - 1>(q, w, blocks, frags);
+    else if ((q->numAmps >> kSweepTileBits) < (long long)perCU * numCUs())
+        launchTiles<T, false, 8, kSweepTileBits>(q, w, blocks, frags);
+    else if (q->numAmps * (long long)sizeof(Amp<T>) > (256ll << 20))
+        launchTiles<T, true, 4, kSweepTileBits>(q, w, blocks, frags);
+    else
+        launchTiles<T, false, 4, kSweepTileBits>(q, w, blocks, frags);
 }
 
 void runSweeps(QuregDev *q, const SweepPlan &plan, const FlatGate *gates, int first, int last, int firstBlock,
@@ -838,60 +860,43 @@ void applyFlatGate(QuregDev *q, const FlatGate &g) {
 // a gate's arithmetic, by the entries of its matrix
 static int smallKind(const FlatGate &f) {
     if (f.kind == FlatGate::NOT) return SG_NOT;
-    auto zero = [](const Cplx &z) { return z.re == 0 && z.im == 0; };
-    if (zero(f.u[1]) && zero(f.u[2])) return SG_DIAGONAL;
+    auto is = [](const Cplx &z, double re) { return z.re == re && z.im == 0; };
+    if (is(f.u[0], 1) && is(f.u[1], 0) && is(f.u[2], 0)) return SG_PHASE;
     for (const Cplx &z : f.u)
         if (z.im != 0) return SG_GENERAL;
     return SG_REAL;
 }
 
-// the SmallGates of gates[0 .. count): greedy runs of consecutive gates on at most
-// two targets, no run across a multiple of kSmallStage
-static void smallGroups(int n, const FlatGate *gates, int count, SmallGate *out) {
-    for (int i = 0; i < count;) {
-        int t0 = gates[i].target, t1 = -1, j = i;
-        for (; j < count && (j == i || j % kSmallStage); ++j) {
-            const int t = gates[j].target;
-            if (t == t0 || t == t1) continue;
-            if (t1 >= 0) break;
-            t1 = t;
-        }
-        if (t1 < 0) t1 = t0 == 0 ? 1 : 0;  // any other qubit (n = 1: the one that stays zero)
-        if (t0 > t1) std::swap(t0, t1);
-        for (int k = i; k < j; ++k) {
-            const FlatGate &f = gates[k];
-            SmallGate &d = out[k];
-            d.group = k == i ? j - i : 0;
-            d.t0 = t0;
-            d.t1 = t1;
-            d.target = f.target == t0 ? 0 : 1;
-            d.kind = smallKind(f);
-            d.ctrl = (unsigned)f.ctrl;
-            for (int e = 0; e < 4; ++e) d.u[e] = Amp<double>{f.u[e].re, f.u[e].im};
-        }
-        i = j;
-    }
-}
-
 void smallCircuit(QuregDev *q, const FlatGate *gates, int count) {
     runtimeInit();
-    static_assert(sizeof(SmallGate) % 16 == 0, "gates move in 16 B pieces");
     // gates per launch: bounds the upload
-    constexpr int kPerLaunch = 64 * kSmallStage;
-    const int n = q->numQubits, nn = std::max(n, 2);
-    const unsigned threads = std::min((unsigned)kSmallThreads, std::max(64u, 1u << (nn - 2)));
-    const size_t lds = (sizeof(Amp<double>) << nn) + kSmallStage * sizeof(SmallGate);
+    constexpr int kPerLaunch = 4096;
+    const int n = q->numQubits;
+    const unsigned threads = std::min((unsigned)kSmallThreads, std::max(64u, 1u << (n - 1)));
+    constexpr size_t stageBytes = (kSmallStage + 1) * sizeof(SmallGate);
+    const size_t lds = (sizeof(Amp<double>) << n) + stageBytes;
     for (int first = 0; first < count; first += kPerLaunch) {
         const int num = std::min(kPerLaunch, count - first);
         SmallGate *h = reinterpret_cast<SmallGate *>(g_ws.hostRoom((size_t)num * sizeof(SmallGate)));
-        smallGroups(n, gates + first, num, h);
+        for (int i = 0; i < num; ++i) {
+            const FlatGate &f = gates[first + i];
+            SmallGate &d = h[i];
+            d.what = (unsigned)smallKind(f);
+            d.bit = 16u << f.target;
+            d.ctrl = 16u * (unsigned)f.ctrl;
+            d.pad = 0;
+            for (int e = 0; e < 4; ++e) {
+                d.u[2 * e] = f.u[e].re;
+                d.u[2 * e + 1] = f.u[e].im;
+            }
+        }
         g_ws.commit((size_t)num * sizeof(SmallGate));
         const SmallGate *dg = reinterpret_cast<const SmallGate *>(g_ws.dev);
         QMX_DISPATCH(q->prec, T, {
             static bool ldsAllowed = false;
             if (!ldsAllowed) {
                 if (!allowDynamicLds(reinterpret_cast<const void *>(&kSmallCircuit<T>),
-                                     (sizeof(Amp<double>) << kSmallCircuitQubits) + kSmallStage * sizeof(SmallGate),
+                                     (sizeof(Amp<double>) << kSmallCircuitQubits) + stageBytes,
                                      "a small register's circuit"))
                     std::abort();
                 ldsAllowed = true;
