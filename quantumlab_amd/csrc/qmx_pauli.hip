@@ -20,6 +20,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
+#include <cstring>
 #include <vector>
 
 #include "qmx_device.h"
@@ -238,22 +240,36 @@ __global__ void __launch_bounds__(kBlock) kPauliBlock(Amp<T> *__restrict__ a, un
 // then a pair (v, v ^ m) of one thread's registers, m = lx's coordinates, so
 // the group costs one LDS round trip where the pass form costs one per
 // distinct mask. Signs: parity(index & lz) = parity(r & lz) xor parity(v & zv)
-// with zv_j = parity(b_j & lz).
+// with zv_j = parity(b_j & lz); parity(r & lz) = parity(t & tz), tz_j the parity
+// of thread bit j's tile bit.
+//
+// LDS slots are linear in the tile index: bits 4 and up of the index are each
+// folded onto one of its lowest 4 (FP32; 3 in FP64), chosen per block so that the
+// groups' thread bits 0-3 (0-2) fall on different banks; a slot is the XOR of its
+// bits' slots, all precomputed as byte offsets.
+template <typename T>
 struct CosetExpDev {
     uint64_t z;          // global z mask (parity of the tile base)
-    unsigned lz;         // tile-local z mask
+    unsigned tz;         // thread-bit z mask
     unsigned m;          // the X/Y mask's coordinates in the group's basis (0: diagonal)
     unsigned zv;         // bit j: parity(b_j & lz)
     int kind;            // as PauliExpDev
-    double c, kap;
+    T c, kap;
 };
 
 constexpr int kMaxCosetBits = 4;
 
 struct CosetGroupDev {
-    int first, count;             // the group's rotations (block-relative)
-    int piv[kMaxCosetBits];       // pivot tile bits, ascending
-    unsigned C[1 << kMaxCosetBits];  // tile offset of coset element v
+    int first, count;                // the group's rotations (block-relative)
+    unsigned thr[8];                 // slot of thread bit j
+    unsigned C[1 << kMaxCosetBits];  // slot of coset element v
+};
+
+struct CosetTile {
+    int pos[kMaxTileBits];    // global bit of tile bit j, ascending
+    uint64_t hi[kMaxPer];     // global offset of tile index 256 k
+    unsigned slot[8];         // slot of tile bit j < 8 (a thread's transfer elements)
+    unsigned hiSlot[kMaxPer]; // slot of tile index 256 k
 };
 
 template <typename T> constexpr int cosetBits() { return sizeof(T) == 8 ? 3 : 4; }
@@ -266,10 +282,17 @@ template <typename T, int E> struct CosetRegs {
     V re, im;
 };
 
+// How the signs s(u) = (-1)^parity(u & zv) of a mask's pairs are known: none
+// (zv = 0: all +), or the partner's sign equal or opposite to one's own, so that
+// one flip a pair serves both its amplitudes. Flips are a third of an exchange's
+// instructions, and half of a chain's rotations have zv = 0 (X fields, XX bonds).
+// SIGNS_ANY flips each (the rarer plain forms: a variant less to hold in the
+// instruction cache).
+enum CosetSigns { SIGNS_NONE = 0, SIGNS_EQUAL = 1, SIGNS_OPPOSITE = 2, SIGNS_ANY = 3 };
+
 // out_u = c x_u + kap s(u ^ M) F x_{u ^ M} for every u, F = 1 (KIND 1, 4) or i
-// (KIND 2, 5), s(v) = (-1)^parity(v & zv) (the thread's own parity is in kap);
-// KIND 4, 5: the tangent form (c = 1)
-template <typename T, int E, int M, int KIND>
+// (KIND 2, 5) (the thread's own parity is in kap); KIND 4, 5: the tangent form (c = 1)
+template <typename T, int E, int M, int KIND, int SIGNS>
 __device__ __forceinline__ void cosetPairs(CosetRegs<T, E> &x, T c, T kap, unsigned zv) {
     if constexpr (M < E) {
         constexpr int lowM = M & -M;
@@ -277,8 +300,11 @@ __device__ __forceinline__ void cosetPairs(CosetRegs<T, E> &x, T c, T kap, unsig
         for (int u = 0; u < E; ++u) {
             if (u & lowM) continue;
             const int p = u ^ M;
-            const T Bu = signFlip(kap, (unsigned)__popc((unsigned)p & zv));  // for out_u: the partner's sign
-            const T Ap = signFlip(kap, (unsigned)__popc((unsigned)u & zv));  // for out_p
+            // for out_u the partner's sign, for out_p u's
+            const T Bu = SIGNS == SIGNS_NONE ? kap : signFlip(kap, (unsigned)__popc((unsigned)p & zv));
+            const T Ap = SIGNS == SIGNS_OPPOSITE ? -Bu
+                         : SIGNS == SIGNS_ANY    ? signFlip(kap, (unsigned)__popc((unsigned)u & zv))
+                                                 : Bu;
             const T ur = x.re[u], ui = x.im[u], pr = x.re[p], pi = x.im[p];
             if constexpr (KIND == 1) {
                 x.re[u] = c * ur + Bu * pr;
@@ -305,108 +331,148 @@ __device__ __forceinline__ void cosetPairs(CosetRegs<T, E> &x, T c, T kap, unsig
     }
 }
 
-template <typename T, int E, int KIND>
+template <typename T, int E, int KIND, int SIGNS>
 __device__ __forceinline__ void cosetExchange(CosetRegs<T, E> &x, unsigned m, T c, T kap, unsigned zv) {
     switch (m) {
-    case 1: cosetPairs<T, E, 1, KIND>(x, c, kap, zv); break;
-    case 2: cosetPairs<T, E, 2, KIND>(x, c, kap, zv); break;
-    case 3: cosetPairs<T, E, 3, KIND>(x, c, kap, zv); break;
-    case 4: cosetPairs<T, E, 4, KIND>(x, c, kap, zv); break;
-    case 5: cosetPairs<T, E, 5, KIND>(x, c, kap, zv); break;
-    case 6: cosetPairs<T, E, 6, KIND>(x, c, kap, zv); break;
-    case 7: cosetPairs<T, E, 7, KIND>(x, c, kap, zv); break;
-    case 8: cosetPairs<T, E, 8, KIND>(x, c, kap, zv); break;
-    case 9: cosetPairs<T, E, 9, KIND>(x, c, kap, zv); break;
-    case 10: cosetPairs<T, E, 10, KIND>(x, c, kap, zv); break;
-    case 11: cosetPairs<T, E, 11, KIND>(x, c, kap, zv); break;
-    case 12: cosetPairs<T, E, 12, KIND>(x, c, kap, zv); break;
-    case 13: cosetPairs<T, E, 13, KIND>(x, c, kap, zv); break;
-    case 14: cosetPairs<T, E, 14, KIND>(x, c, kap, zv); break;
-    default: cosetPairs<T, E, 15, KIND>(x, c, kap, zv); break;
+    case 1: cosetPairs<T, E, 1, KIND, SIGNS>(x, c, kap, zv); break;
+    case 2: cosetPairs<T, E, 2, KIND, SIGNS>(x, c, kap, zv); break;
+    case 3: cosetPairs<T, E, 3, KIND, SIGNS>(x, c, kap, zv); break;
+    case 4: cosetPairs<T, E, 4, KIND, SIGNS>(x, c, kap, zv); break;
+    case 5: cosetPairs<T, E, 5, KIND, SIGNS>(x, c, kap, zv); break;
+    case 6: cosetPairs<T, E, 6, KIND, SIGNS>(x, c, kap, zv); break;
+    case 7: cosetPairs<T, E, 7, KIND, SIGNS>(x, c, kap, zv); break;
+    case 8: cosetPairs<T, E, 8, KIND, SIGNS>(x, c, kap, zv); break;
+    case 9: cosetPairs<T, E, 9, KIND, SIGNS>(x, c, kap, zv); break;
+    case 10: cosetPairs<T, E, 10, KIND, SIGNS>(x, c, kap, zv); break;
+    case 11: cosetPairs<T, E, 11, KIND, SIGNS>(x, c, kap, zv); break;
+    case 12: cosetPairs<T, E, 12, KIND, SIGNS>(x, c, kap, zv); break;
+    case 13: cosetPairs<T, E, 13, KIND, SIGNS>(x, c, kap, zv); break;
+    case 14: cosetPairs<T, E, 14, KIND, SIGNS>(x, c, kap, zv); break;
+    default: cosetPairs<T, E, 15, KIND, SIGNS>(x, c, kap, zv); break;
     }
+}
+
+template <typename T, int E, int KIND>
+__device__ __forceinline__ void cosetRotation(CosetRegs<T, E> &x, unsigned m, T c, T kap, unsigned zv) {
+    if constexpr (KIND == 1 || KIND == 2) cosetExchange<T, E, KIND, SIGNS_ANY>(x, m, c, kap, zv);
+    else if (zv == 0) cosetExchange<T, E, KIND, SIGNS_NONE>(x, m, c, kap, zv);
+    else if (__popc(m & zv) & 1) cosetExchange<T, E, KIND, SIGNS_OPPOSITE>(x, m, c, kap, zv);
+    else cosetExchange<T, E, KIND, SIGNS_EQUAL>(x, m, c, kap, zv);
 }
 
 // x_u *= c - i kap s(u) (TAN: c = 1)
 template <typename T, int E, bool TAN>
 __device__ __forceinline__ void cosetDiagonal(CosetRegs<T, E> &x, T c, T kap, unsigned zv) {
+    // the elements u < E/2 and u + E/2 have equal or opposite signs: one flip for both
+    const T top = signFlip((T)1, zv >> (E == 16 ? 3 : 2));
 #pragma unroll
-    for (int u = 0; u < E; ++u) {
-        const T A = signFlip(kap, (unsigned)__popc((unsigned)u & zv));
-        const T vr = x.re[u], vi = x.im[u];
+    for (int u = 0; u < E / 2; ++u) {
+        const T A = signFlip(kap, (unsigned)__popc((unsigned)u & zv)), B = A * top;
+        const int w = u + E / 2;
+        const T vr = x.re[u], vi = x.im[u], wr = x.re[w], wi = x.im[w];
         x.re[u] = TAN ? vr + A * vi : c * vr + A * vi;
         x.im[u] = TAN ? vi - A * vr : c * vi - A * vr;
+        x.re[w] = TAN ? wr + B * wi : c * wr + B * wi;
+        x.im[w] = TAN ? wi - B * wr : c * wi - B * wr;
     }
 }
 
-// Tile staging and the final scaled store as in kPauliBlock, one tile per
-// workgroup; the groups replace its passes. A persistent FP32 grid that
-// prefetched the next tile into registers measured slower once the groups had
-// cut the LDS round trips (24 qubits: 290 vs 284 ms; 27 qubits: 1470 vs 1298
-// ms; 29 qubits: 6318 vs 5580 ms for the same solves, identical states).
+// One tile per workgroup; a persistent FP32 grid that prefetched the next tile
+// into registers measured slower once the groups had cut the LDS round trips (24
+// qubits: 290 vs 284 ms; 27 qubits: 1470 vs 1298 ms; 29 qubits: 6318 vs 5580 ms for
+// the same solves, identical states). A rotation's record is read while the one
+// before it is applied. COSET_MEASURED
 template <typename T>
-__global__ void __launch_bounds__(kBlock) kPauliCoset(Amp<T> *__restrict__ a, PauliTile tile,
+__global__ void __launch_bounds__(kBlock) kPauliCoset(Amp<T> *__restrict__ a, CosetTile tile,
                                                       const CosetGroupDev *__restrict__ groups, int numGroups,
-                                                      const CosetExpDev *__restrict__ ops, double scale) {
+                                                      const CosetExpDev<T> *__restrict__ ops, T scale) {
     constexpr int R = cosetBits<T>();
     constexpr int E = 1 << R;   // amplitudes per thread; the tile is kBlock * E
-    extern __shared__ unsigned char smem[];
-    Amp<T> *st = reinterpret_cast<Amp<T> *>(smem);
+    __shared__ __attribute__((aligned(16))) char st[sizeof(Amp<T>) * kBlock * E];
     const unsigned tx = threadIdx.x;
+    unsigned on[8];             // all ones where thread bit j is set
+#pragma unroll
+    for (int j = 0; j < 8; ++j) on[j] = 0u - ((tx >> j) & 1u);
     uint64_t dt = 0;
+    unsigned ts = 0;
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-        if ((tx >> j) & 1) dt |= 1ull << tile.pos[j];
-    const uint64_t base = insertZeros((uint64_t)flatBlockLinear(), tile.fixed);
+    for (int j = 0; j < 8; ++j) {
+        if (on[j]) dt |= 1ull << tile.pos[j];
+        ts ^= on[j] & tile.slot[j];
+    }
+    auto at = [&](unsigned slot) -> Amp<T> & { return *reinterpret_cast<Amp<T> *>(st + slot); };
+    uint64_t base = (uint64_t)flatBlockLinear();
+#pragma unroll
+    for (int j = 0; j < 8 + R; ++j) base = insertZero(base, tile.pos[j]);
     Amp<T> *src = a + (base | dt);
+    {
+        Amp<T> in[E];
 #pragma unroll
-    for (int k = 0; k < E; ++k) st[tx + (k << 8)] = src[tile.hi[k]];
+        for (int k = 0; k < E; ++k) in[k] = src[tile.hi[k]];
+#pragma unroll
+        for (int k = 0; k < E; ++k) at(ts ^ tile.hiSlot[k]) = in[k];
+    }
+    CosetExpDev<T> next = ops[0];   // a block has at least one rotation; the list one more than its last
     __syncthreads();
     for (int g = 0; g < numGroups; ++g) {
         const CosetGroupDev &grp = groups[g];
-        unsigned r = tx;
+        unsigned r = 0;
 #pragma unroll
-        for (int j = 0; j < R; ++j) {
-            const int p = grp.piv[j];
-            r = ((r >> p) << (p + 1)) | (r & ((1u << p) - 1u));
-        }
+        for (int j = 0; j < 8; ++j) r ^= on[j] & grp.thr[j];
         CosetRegs<T, E> x;
 #pragma unroll
         for (int v = 0; v < E; ++v) {
-            const Amp<T> t = st[r ^ grp.C[v]];
+            const Amp<T> t = at(r ^ grp.C[v]);
             x.re[v] = t.x;
             x.im[v] = t.y;
         }
         const int first = grp.first, count = grp.count;
         for (int o = 0; o < count; ++o) {
-            const CosetExpDev e = ops[first + o];
-            const unsigned p0 = (unsigned)__popcll(base & e.z) + (unsigned)__popc(r & e.lz);
-            const T kap = signFlip((T)e.kap, p0);
-            const T c = (T)e.c;
+            const CosetExpDev<T> e = next;
+            next = ops[first + o + 1];
+            const unsigned p0 = (unsigned)__popcll(base & e.z) + (unsigned)__popc(tx & e.tz);
+            const T kap = signFlip(e.kap, p0);
+            const T c = e.c;
             switch (e.kind) {
             case 0: cosetDiagonal<T, E, false>(x, c, kap, e.zv); break;
-            case 1: cosetExchange<T, E, 1>(x, e.m, c, kap, e.zv); break;
-            case 2: cosetExchange<T, E, 2>(x, e.m, c, kap, e.zv); break;
+            case 1: cosetRotation<T, E, 1>(x, e.m, c, kap, e.zv); break;
+            case 2: cosetRotation<T, E, 2>(x, e.m, c, kap, e.zv); break;
             case 3: cosetDiagonal<T, E, true>(x, c, kap, e.zv); break;
-            case 4: cosetExchange<T, E, 4>(x, e.m, c, kap, e.zv); break;
-            default: cosetExchange<T, E, 5>(x, e.m, c, kap, e.zv); break;
+            case 4: cosetRotation<T, E, 4>(x, e.m, c, kap, e.zv); break;
+            default: cosetRotation<T, E, 5>(x, e.m, c, kap, e.zv); break;
             }
         }
 #pragma unroll
-        for (int v = 0; v < E; ++v) st[r ^ grp.C[v]] = Amp<T>{x.re[v], x.im[v]};
+        for (int v = 0; v < E; ++v) at(r ^ grp.C[v]) = Amp<T>{x.re[v], x.im[v]};
         __syncthreads();
     }
-    const T sc = (T)scale;
 #pragma unroll
     for (int k = 0; k < E; ++k) {
-        const Amp<T> v = st[tx + (k << 8)];
-        src[tile.hi[k]] = Amp<T>{sc * v.x, sc * v.y};
+        const Amp<T> v = at(ts ^ tile.hiSlot[k]);
+        src[tile.hi[k]] = Amp<T>{scale * v.x, scale * v.y};
     }
 }
 
 constexpr int kMaxBlockOps = 1 << 16;  // rotations per block (bounds the host's records only)
 
+// host records of the coset form, before slots and thread bits are known
+struct CosetRot {
+    uint64_t z;
+    unsigned lx, lz;   // tile-local masks
+    int kind;
+    double c, kap;
+    unsigned tz, m, zv;
+};
+struct CosetSpan {
+    int first, count;
+    int piv[kMaxCosetBits];          // pivot tile bits, ascending
+    int thr[8];                      // tile bit of thread bit j: the others, ascending
+    unsigned C[1 << kMaxCosetBits];  // tile index of coset element v
+};
+
 struct Block {
     PauliTile tile;
+    CosetTile coTile;           // coset form
     int firstPass, numPasses;   // coset form: its groups
     int firstOp, numOps;
     int single;        // >= 0: one rotation too wide for a tile, applied alone (index into seq)
@@ -414,53 +480,55 @@ struct Block {
     double scale;      // product of cos(theta/2) over the block's tangent-form rotations
 };
 
-// Split a block's rotations (tile-local X/Y masks lx, z masks lz) into coset
-// groups of at most R exchange dimensions; fills the ops' m and zv.
-void buildCosetGroups(const std::vector<unsigned> &lx, std::vector<CosetExpDev> &ops, int firstOp, int tb, int R,
-                      std::vector<CosetGroupDev> &groups) {
-    const int count = (int)lx.size();
+// Split a block's rotations into coset groups of at most R exchange dimensions;
+// fills the rotations' m, zv and tz.
+void buildCosetGroups(std::vector<CosetRot> &ops, int firstOp, int tb, int R, std::vector<CosetSpan> &groups) {
+    const int count = (int)ops.size() - firstOp;
     int start = 0;
     while (start < count) {
         // grow the group while the masks' span stays within R dimensions
-        std::vector<unsigned> ech;  // echelon form by highest bit, for the membership test
-        int end = start;
+        unsigned ech[kMaxCosetBits];  // echelon form, highest first, for the membership test
+        int ne = 0, end = start;
         for (; end < count; ++end) {
-            unsigned v = lx[end];
-            for (unsigned e : ech)
-                if ((v ^ e) < v) v ^= e;
+            unsigned v = ops[firstOp + end].lx;
+            for (int e = 0; e < ne; ++e)
+                if ((v ^ ech[e]) < v) v ^= ech[e];
             if (v == 0) continue;
-            if ((int)ech.size() == R) break;
-            ech.push_back(v);
-            std::sort(ech.begin(), ech.end(), [](unsigned p, unsigned q) { return p > q; });
+            if (ne == R) break;
+            ech[ne++] = v;
+            std::sort(ech, ech + ne, [](unsigned p, unsigned q) { return p > q; });
         }
         // reduced echelon basis (pivot = highest bit), extended by unit
         // vectors at the highest free tile bits to exactly R vectors
-        std::vector<unsigned> b;
-        std::vector<int> piv;
+        unsigned b[kMaxCosetBits];
+        int piv[kMaxCosetBits], nb = 0;
         auto add = [&](unsigned v) {
-            for (size_t j = 0; j < b.size(); ++j)
+            for (int j = 0; j < nb; ++j)
                 if ((v >> piv[j]) & 1) v ^= b[j];
             const int p = 31 - __builtin_clz(v);
-            for (size_t j = 0; j < b.size(); ++j)
+            for (int j = 0; j < nb; ++j)
                 if ((b[j] >> p) & 1) b[j] ^= v;
-            b.push_back(v);
-            piv.push_back(p);
+            b[nb] = v;
+            piv[nb++] = p;
         };
-        for (unsigned e : ech) add(e);
-        for (int p = tb - 1; p >= 0 && (int)b.size() < R; --p)
-            if (std::find(piv.begin(), piv.end(), p) == piv.end()) add(1u << p);
+        for (int e = 0; e < ne; ++e) add(ech[e]);
+        for (int p = tb - 1; p >= 0 && nb < R; --p)
+            if (std::find(piv, piv + nb, p) == piv + nb) add(1u << p);
         // order the basis by pivot, ascending
-        std::vector<int> ord(R);
-        for (int j = 0; j < R; ++j) ord[j] = j;
-        std::sort(ord.begin(), ord.end(), [&](int p, int q) { return piv[p] < piv[q]; });
-        CosetGroupDev g{};
+        int ord[kMaxCosetBits] = {0, 1, 2, 3};
+        std::sort(ord, ord + R, [&](int p, int q) { return piv[p] < piv[q]; });
+        CosetSpan g{};
         g.first = start;
         g.count = end - start;
         unsigned bs[kMaxCosetBits];
+        unsigned pivots = 0;
         for (int j = 0; j < R; ++j) {
             g.piv[j] = piv[ord[j]];
             bs[j] = b[ord[j]];
+            pivots |= 1u << g.piv[j];
         }
+        for (int i = 0, j = 0; i < tb && j < 8; ++i)
+            if (!((pivots >> i) & 1)) g.thr[j++] = i;
         for (int v = 0; v < (1 << R); ++v) {
             unsigned cv = 0;
             for (int j = 0; j < R; ++j)
@@ -468,23 +536,59 @@ void buildCosetGroups(const std::vector<unsigned> &lx, std::vector<CosetExpDev> 
             g.C[v] = cv;
         }
         for (int k = start; k < end; ++k) {
-            CosetExpDev &d = ops[firstOp + k];
+            CosetRot &d = ops[firstOp + k];
             unsigned m = 0, back = 0;
             for (int j = 0; j < R; ++j)
-                if ((lx[k] >> g.piv[j]) & 1) {
+                if ((d.lx >> g.piv[j]) & 1) {
                     m |= 1u << j;
                     back ^= bs[j];
                 }
-            if (back != lx[k]) {
+            if (back != d.lx) {
                 std::fprintf(stderr, "libquest_mi355x: Pauli coset basis does not span a rotation's mask\n");
                 std::abort();
             }
             d.m = m;
             d.zv = 0;
             for (int j = 0; j < R; ++j) d.zv |= ((unsigned)__builtin_popcount(bs[j] & d.lz) & 1u) << j;
+            d.tz = 0;
+            for (int j = 0; j < 8; ++j) d.tz |= ((d.lz >> g.thr[j]) & 1u) << j;
         }
         groups.push_back(g);
         start = end;
+    }
+}
+
+// The slots (in amplitudes) of a tile's bits: bit i >= R folded onto bit f(i) < R,
+// R = 4 (16 FP32 amplitudes are one cycle of the LDS banks) or 3. Each fold goes
+// where it leaves the most of the groups' first R thread bits (and the transfers',
+// bits 0 .. R-1) on different banks: the sum of the ranks of their low slot bits.
+void cosetSlots(const std::vector<CosetSpan> &groups, int firstGroup, int tb, int R, unsigned slot[kMaxTileBits]) {
+    for (int i = 0; i < tb; ++i) slot[i] = 1u << i;
+    auto rank = [&](const CosetSpan &g, int upTo) {
+        unsigned e[4];
+        int n = 0;
+        for (int j = 0; j < R; ++j) {
+            if (g.thr[j] > upTo) continue;
+            unsigned v = slot[g.thr[j]] & ((1u << R) - 1u);
+            for (int k = 0; k < n; ++k)
+                if ((v ^ e[k]) < v) v ^= e[k];
+            if (v) e[n++] = v;
+        }
+        return n;
+    };
+    for (int i = R; i < tb; ++i) {
+        int best = -1;
+        unsigned bestSlot = slot[i];
+        for (int f = 0; f < R; ++f) {
+            slot[i] = (1u << i) | (1u << ((f + i) % R));  // ties: bits 4, 5, ... onto 0, 1, ...
+            int sum = 0;
+            for (size_t g = firstGroup; g < groups.size(); ++g) sum += rank(groups[g], i);
+            if (sum > best) {
+                best = sum;
+                bestSlot = slot[i];
+            }
+        }
+        slot[i] = bestSlot;
     }
 }
 
@@ -561,8 +665,9 @@ void applyPauliSequence(QuregDev *q, const PauliExp *seqIn, int countIn, int rep
     const double scaleFloor = q->prec == FP64 ? std::ldexp(1.0, -500) : std::ldexp(1.0, -40);
     std::vector<PauliExpDev> ops;
     std::vector<PassDev> passes;
-    std::vector<CosetExpDev> cops;
-    std::vector<CosetGroupDev> groups;
+    std::vector<CosetRot> cops;
+    std::vector<CosetSpan> groups;
+    std::vector<CosetGroupDev> dgroups;
     std::vector<Block> blocks;
     int i = 0;
     while (i < count) {
@@ -571,7 +676,9 @@ void applyPauliSequence(QuregDev *q, const PauliExp *seqIn, int countIn, int rep
             continue;
         }
         if (__builtin_popcountll(seq[i].x) > maxX) {
-            blocks.push_back(Block{PauliTile{}, 0, 0, 0, 0, i, false, 1.0});
+            Block alone{};
+            alone.single = i;
+            blocks.push_back(alone);
             ++i;
             continue;
         }
@@ -603,7 +710,6 @@ void applyPauliSequence(QuregDev *q, const PauliExp *seqIn, int countIn, int rep
         blk.coset = coset;
         blk.firstPass = coset ? (int)groups.size() : (int)passes.size();
         blk.firstOp = coset ? (int)cops.size() : (int)ops.size();
-        std::vector<unsigned> lxs;  // coset form: the rotations' tile-local X/Y masks
         int open = -1;  // pass accepting rotations
         for (int k = i; k < j; ++k) {
             const PauliExp &e = seq[k];
@@ -639,8 +745,7 @@ void applyPauliSequence(QuregDev *q, const PauliExp *seqIn, int countIn, int rep
                 blk.scale *= d.c;
             }
             if (coset) {
-                cops.push_back(CosetExpDev{d.z, d.lz, 0, 0, d.kind, d.c, d.kap});
-                lxs.push_back(lx);
+                cops.push_back(CosetRot{d.z, lx, d.lz, d.kind, d.c, d.kap, 0, 0, 0});
                 continue;
             }
             const int rel = (int)ops.size() - blk.firstOp;  // passes index the block's own ops
@@ -657,8 +762,31 @@ void applyPauliSequence(QuregDev *q, const PauliExp *seqIn, int countIn, int rep
             ++passes[open].count;
         }
         if (coset) {
-            buildCosetGroups(lxs, cops, blk.firstOp, blk.tile.tb, R, groups);
+            buildCosetGroups(cops, blk.firstOp, tb, R, groups);
             blk.numPasses = (int)groups.size() - blk.firstPass;
+            unsigned slot[kMaxTileBits];
+            cosetSlots(groups, blk.firstPass, tb, R, slot);
+            const unsigned ab = (unsigned)ampBytes(q->prec);
+            auto slotOf = [&](unsigned e) {
+                unsigned o = 0;
+                for (int b = 0; b < tb; ++b)
+                    if ((e >> b) & 1) o ^= slot[b];
+                return o * ab;
+            };
+            for (int t = 0; t < tb; ++t) blk.coTile.pos[t] = blk.tile.pos[t];
+            for (int t = 0; t < 8; ++t) blk.coTile.slot[t] = slot[t] * ab;
+            for (int k = 0; k < (1 << R); ++k) {
+                blk.coTile.hi[k] = blk.tile.hi[k];
+                blk.coTile.hiSlot[k] = slotOf(256u * (unsigned)k);
+            }
+            for (size_t g = (size_t)blk.firstPass; g < groups.size(); ++g) {
+                CosetGroupDev d{};
+                d.first = groups[g].first;
+                d.count = groups[g].count;
+                for (int j = 0; j < 8; ++j) d.thr[j] = slot[groups[g].thr[j]] * ab;
+                for (int v = 0; v < (1 << R); ++v) d.C[v] = slotOf(groups[g].C[v]);
+                dgroups.push_back(d);
+            }
             blk.numOps = (int)cops.size() - blk.firstOp;
             if (blk.numPasses > 0) blocks.push_back(blk);
             i = j;
@@ -689,20 +817,31 @@ void applyPauliSequence(QuregDev *q, const PauliExp *seqIn, int countIn, int rep
         i = j;
     }
     if (blocks.empty()) return;
-    std::vector<void *> owned;
-    auto upload = [&](const void *h, size_t bytes) -> void * {
-        if (bytes == 0) return nullptr;
-        void *d = devAlloc(bytes);
-        hostToDevice(d, h, bytes);
-        owned.push_back(d);
-        return d;
-    };
-    const PauliExpDev *dOps = static_cast<const PauliExpDev *>(upload(ops.data(), ops.size() * sizeof(PauliExpDev)));
-    const PassDev *dPasses = static_cast<const PassDev *>(upload(passes.data(), passes.size() * sizeof(PassDev)));
-    const CosetExpDev *dCops =
-        static_cast<const CosetExpDev *>(upload(cops.data(), cops.size() * sizeof(CosetExpDev)));
-    const CosetGroupDev *dGroups =
-        static_cast<const CosetGroupDev *>(upload(groups.data(), groups.size() * sizeof(CosetGroupDev)));
+    // one upload, through the library's growable staging pair: nothing is
+    // allocated or waited for per call
+    auto align = [](size_t x) { return (x + 63) & ~(size_t)63; };
+    const size_t opBytes = coset ? (cops.size() + 1) * (q->prec == FP64 ? sizeof(CosetExpDev<double>)
+                                                                        : sizeof(CosetExpDev<float>))
+                                 : ops.size() * sizeof(PauliExpDev);
+    const size_t groupAt = align(opBytes);
+    const size_t bytes = groupAt + (coset ? dgroups.size() * sizeof(CosetGroupDev) : passes.size() * sizeof(PassDev));
+    std::vector<char> image(bytes);
+    if (coset) {
+        QMX_DISPATCH(q->prec, T, {
+            CosetExpDev<T> *d = reinterpret_cast<CosetExpDev<T> *>(image.data());
+            for (size_t k = 0; k < cops.size(); ++k)
+                d[k] = CosetExpDev<T>{cops[k].z, cops[k].tz, cops[k].m, cops[k].zv, cops[k].kind, (T)cops[k].c,
+                                      (T)cops[k].kap};
+        });
+        if (!dgroups.empty()) std::memcpy(image.data() + groupAt, dgroups.data(), dgroups.size() * sizeof(CosetGroupDev));
+    } else {
+        if (!ops.empty()) std::memcpy(image.data(), ops.data(), opBytes);
+        if (!passes.empty()) std::memcpy(image.data() + groupAt, passes.data(), passes.size() * sizeof(PassDev));
+    }
+    const char *dev = static_cast<const char *>(stageLarge(image.data(), bytes, hstream()));
+    const PauliExpDev *dOps = reinterpret_cast<const PauliExpDev *>(dev);
+    const PassDev *dPasses = reinterpret_cast<const PassDev *>(dev + groupAt);
+    const CosetGroupDev *dGroups = reinterpret_cast<const CosetGroupDev *>(dev + groupAt);
     const unsigned prefetchGrid = 4u * (unsigned)numCUs();
     for (int r = 0; r < reps; ++r) {
         for (const Block &b : blocks) {
@@ -714,14 +853,11 @@ void applyPauliSequence(QuregDev *q, const PauliExp *seqIn, int countIn, int rep
             const unsigned tiles = (unsigned)(q->numAmps >> b.tile.tb);
             const size_t lds = (q->prec == FP64 ? sizeof(Amp<double>) : sizeof(Amp<float>)) << b.tile.tb;
             if (b.coset) {
-                if (q->prec == FP64)
-                    hipLaunchKernelGGL(kPauliCoset<double>, dim3(tiles), dim3(kBlock), lds, hstream(),
-                                       (Amp<double> *)q->amps, b.tile, dGroups + b.firstPass, b.numPasses,
-                                       dCops + b.firstOp, b.scale);
-                else
-                    hipLaunchKernelGGL(kPauliCoset<float>, dim3(tiles), dim3(kBlock), lds, hstream(),
-                                       (Amp<float> *)q->amps, b.tile, dGroups + b.firstPass, b.numPasses,
-                                       dCops + b.firstOp, b.scale);
+                QMX_DISPATCH(q->prec, T, {
+                    hipLaunchKernelGGL(kPauliCoset<T>, gridOf(tiles), dim3(kBlock), 0, hstream(), (Amp<T> *)q->amps,
+                                       b.coTile, dGroups + b.firstPass, b.numPasses,
+                                       reinterpret_cast<const CosetExpDev<T> *>(dev) + b.firstOp, (T)b.scale);
+                });
                 continue;
             }
             // pairs per thread: 2^tb / 2 / kBlock at the full tile size (8 FP32, 4 FP64)
@@ -735,10 +871,6 @@ void applyPauliSequence(QuregDev *q, const PauliExp *seqIn, int countIn, int rep
                                    dPasses + b.firstPass, b.numPasses, dOps + b.firstOp, b.scale);
         }
         checkLaunch("applyPauliSequence");
-    }
-    if (!owned.empty()) {
-        deviceSync();
-        for (void *d : owned) devFree(d);
     }
 }
 
