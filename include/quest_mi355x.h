@@ -52,8 +52,9 @@ double qmxTimerSlotMs(int slot);
 /* Density registers: operations on at most two qubits (gates, controlled
  * gates, channels, Kraus maps) compose into one superoperator that is swept
  * over the register once, when the next operation needs other qubits, another
- * register or the stream. Cumulative counts since load: sweeps made and
- * operations absorbed into them. */
+ * register or the stream. Operation lists (qmxApplyOperations) of one- and two-qubit
+ * gates, one-qubit channels and collapses are planned as a whole into fewer sweeps.
+ * Cumulative counts since load: sweeps made and operations absorbed into them. */
 void qmxDensityFusionStats(long long *sweeps, long long *operations);
 /* QuantumLab's amplitude-encoding circuit for the real vector vec (2^numQubits
  * entries, encoded on qubits 0..numQubits-1, bit l <-> qubit l) applied to

@@ -22,8 +22,9 @@
 // the register); other block sizes take one sweep a block (qmx::applyMatrixN).
 // State vectors of at most 12 qubits take every list, fused or not, gate by gate
 // in one workgroup's LDS, one launch for the list. On density registers, fused
-// application is the unfused sequence: the library already composes every
-// operation on at most two qubits into superoperator sweeps there.
+// application is the unfused sequence: a recorded circuit's operations are the QuEST
+// calls, which compose into superoperator sweeps two qubits at a time, and
+// qmxApplyOperations plans its list as gates on the row and column bits.
 //
 // The block planner below (qmxCircuitFuse's steps) is greedy and dependency-aware:
 // see fuseSegment. Block matrices are products of the expanded gate matrices,
@@ -255,6 +256,48 @@ FlatGate flatGate(const Gate &g) {
     return f;
 }
 
+// the one-qubit channel `code` of strength p on qubit q of an n-qubit density
+// register, with the numbers of its QuEST call; false for two-qubit channels
+bool channelGate(int code, int q, int n, double p, FlatGate &g) {
+    auto channel = [&](double f, double swap, double d00, double d01, double d10, double d11) {
+        g.kind = FlatGate::CHANNEL;
+        g.target = q;
+        g.ctrl = 0;
+        g.k = q + n;
+        g.u[0] = Cplx{f, swap};
+        g.u[1] = Cplx{d00, d01};
+        g.u[2] = Cplx{d10, d11};
+        g.u[3] = Cplx{0, 0};
+        return true;
+    };
+    auto pauli = [&](double x, double y, double z) {
+        const double none = 1 - (x + y + z);
+        return channel(none - z, x - y, none + z, x + y, x + y, none + z);
+    };
+    switch (code) {
+        case QMX_OP_NOISE_DAMPING: return channel(std::sqrt(1 - p), 0, 1, p, 0, 1 - p);
+        case QMX_OP_NOISE_DEPHASING: return channel(1 - 2 * p, 0, 1, 0, 0, 1);
+        case QMX_OP_NOISE_DEPOLARISING: {
+            const double level = (4 * p) / 3.0, h = level / 2;
+            return channel(1 - level, 0, 1 - h, h, h, 1 - h);
+        }
+        case QMX_OP_NOISE_MIX_PAULI_X: return pauli(p, 0, 0);
+        case QMX_OP_NOISE_MIX_PAULI_Y: return pauli(0, p, 0);
+        case QMX_OP_NOISE_MIX_PAULI_Z: return pauli(0, 0, p);
+        case QMX_OP_NOISE_MIX_PAULI_ALL: return pauli(p, p, p);
+        default: return false;
+    }
+}
+
+// channel b after channel a on the same qubit, as one
+void joinChannel(FlatGate &a, const FlatGate &b) {
+    const double f = a.u[0].re, s = a.u[0].im;
+    a.u[0] = Cplx{b.u[0].re * f + b.u[0].im * s, b.u[0].re * s + b.u[0].im * f};
+    const Cplx r0 = a.u[1], r1 = a.u[2];
+    a.u[1] = Cplx{b.u[1].re * r0.re + b.u[1].im * r1.re, b.u[1].re * r0.im + b.u[1].im * r1.im};
+    a.u[2] = Cplx{b.u[2].re * r0.re + b.u[2].im * r1.re, b.u[2].re * r0.im + b.u[2].im * r1.im};
+}
+
 // qubits an operation code takes (0: not a recordable QuantumLab code)
 int arity(int code) {
     switch (code) {
@@ -332,6 +375,21 @@ void buildBlockMatrix(const qmxCircuit &c, Block &b) {
     }
 }
 
+void mixNoise(const Qureg &q, int code, int a, int b, qreal p) {
+    switch (code) {
+        case QMX_OP_NOISE_DAMPING: mixDamping(q, a, p); break;
+        case QMX_OP_NOISE_DEPHASING: mixDephasing(q, a, p); break;
+        case QMX_OP_NOISE_DEPOLARISING: mixDepolarising(q, a, p); break;
+        case QMX_OP_NOISE_MIX_PAULI_X: mixPauli(q, a, p, 0, 0); break;
+        case QMX_OP_NOISE_MIX_PAULI_Y: mixPauli(q, a, 0, p, 0); break;
+        case QMX_OP_NOISE_MIX_PAULI_Z: mixPauli(q, a, 0, 0, p); break;
+        case QMX_OP_NOISE_MIX_PAULI_ALL: mixPauli(q, a, p, p, p); break;
+        case QMX_OP_NOISE_TWO_QUBIT_DEPHASING: mixTwoQubitDephasing(q, a, b, p); break;
+        case QMX_OP_NOISE_TWO_QUBIT_DEPOLARISING: mixTwoQubitDepolarising(q, a, b, p); break;
+        default: break;
+    }
+}
+
 // the QuEST call QLGate::PerformBasicOperation makes (QLGate.cpp:652-803);
 // returns the collapse probability, else 1
 double runOp(const Qureg &q, Op &o) {
@@ -356,15 +414,12 @@ double runOp(const Qureg &q, Op &o) {
         case QMX_OP_CRZ: controlledRotateZ(q, qs[0], qs[1], t); break;
         case QMX_OP_CC: return collapseToOutcome(q, qs[0], (int)o.param);
         // noise: density registers only; a state vector ignores it, as the reference does
-        case QMX_OP_NOISE_DAMPING: if (dm) mixDamping(q, qs[0], t); break;
-        case QMX_OP_NOISE_DEPHASING: if (dm) mixDephasing(q, qs[0], t); break;
-        case QMX_OP_NOISE_DEPOLARISING: if (dm) mixDepolarising(q, qs[0], t); break;
-        case QMX_OP_NOISE_MIX_PAULI_X: if (dm) mixPauli(q, qs[0], t, 0, 0); break;
-        case QMX_OP_NOISE_MIX_PAULI_Y: if (dm) mixPauli(q, qs[0], 0, t, 0); break;
-        case QMX_OP_NOISE_MIX_PAULI_Z: if (dm) mixPauli(q, qs[0], 0, 0, t); break;
-        case QMX_OP_NOISE_MIX_PAULI_ALL: if (dm) mixPauli(q, qs[0], t, t, t); break;
-        case QMX_OP_NOISE_TWO_QUBIT_DEPHASING: if (dm) mixTwoQubitDephasing(q, qs[0], qs[1], t); break;
-        case QMX_OP_NOISE_TWO_QUBIT_DEPOLARISING: if (dm) mixTwoQubitDepolarising(q, qs[0], qs[1], t); break;
+        case QMX_OP_NOISE_DAMPING: case QMX_OP_NOISE_DEPHASING: case QMX_OP_NOISE_DEPOLARISING:
+        case QMX_OP_NOISE_MIX_PAULI_X: case QMX_OP_NOISE_MIX_PAULI_Y: case QMX_OP_NOISE_MIX_PAULI_Z:
+        case QMX_OP_NOISE_MIX_PAULI_ALL: case QMX_OP_NOISE_TWO_QUBIT_DEPHASING:
+        case QMX_OP_NOISE_TWO_QUBIT_DEPOLARISING:
+            if (dm) mixNoise(q, o.code, qs[0], o.qubits.size() > 1 ? qs[1] : -1, t);
+            break;
         case OP_COMPACT_UNITARY: compactUnitary(q, o.target, o.alpha, o.beta); break;
         case OP_UNITARY: unitary(q, o.target, o.m2); break;
         case OP_ROTATE_Z: rotateZ(q, o.target, t); break;
@@ -381,33 +436,31 @@ double runOp(const Qureg &q, Op &o) {
 }
 
 // the density simulator's noise after every operation that is neither noise
-// nor a collapse, on the qubits that operation lists (QLSimulatorDensityMatrix.cpp:88-153)
-void noiseAfterGate(const Qureg &q, const Op &o, const qmxNoiseAfterGate &nz) {
-    if (isNoise(o.code) || o.code == QMX_OP_CC) return;
+// nor a collapse, on the qubits that operation lists (QLSimulatorDensityMatrix.cpp:88-153):
+// emit(code, q0, q1, p) for each channel
+template <class F>
+void noiseAfterGate(int code, const int *qs, int n, const qmxNoiseAfterGate &nz, F emit) {
+    if (isNoise(code) || code == QMX_OP_CC) return;
     const qreal tiny = std::numeric_limits<qreal>::min();
+    auto each = [&](int channel, qreal p) {
+        for (int i = 0; i < n; ++i) emit(channel, qs[i], -1, p);
+    };
+    if (nz.damping > tiny) each(QMX_OP_NOISE_DAMPING, nz.damping);
+    if (nz.dephasing > tiny && (nz.twoQubitDephasing < tiny || n == 1)) each(QMX_OP_NOISE_DEPHASING, nz.dephasing);
+    if (nz.depolarising > tiny && (nz.twoQubitDepolarising < tiny || n == 1))
+        each(QMX_OP_NOISE_DEPOLARISING, nz.depolarising);
+    if (nz.mixPauli > tiny) each(QMX_OP_NOISE_MIX_PAULI_ALL, nz.mixPauli);
+    if (nz.twoQubitDepolarising > tiny && n == 2)
+        emit(QMX_OP_NOISE_TWO_QUBIT_DEPOLARISING, qs[0], qs[1], nz.twoQubitDepolarising);
+    if (nz.twoQubitDephasing > tiny && n == 2)
+        emit(QMX_OP_NOISE_TWO_QUBIT_DEPHASING, qs[0], qs[1], nz.twoQubitDephasing);
+}
+
+void noiseAfterGate(const Qureg &q, const Op &o, const qmxNoiseAfterGate &nz) {
     std::vector<int> qs = o.qubits;
     if (o.target >= 0) qs.push_back(o.target);
-    const int n = (int)qs.size();
-    if (nz.damping > tiny)
-        for (int t : qs) mixDamping(q, t, nz.damping);
-    if (nz.dephasing > tiny) {
-        if (nz.twoQubitDephasing < tiny) {
-            for (int t : qs) mixDephasing(q, t, nz.dephasing);
-        } else if (n == 1) {
-            mixDephasing(q, qs[0], nz.dephasing);
-        }
-    }
-    if (nz.depolarising > tiny) {
-        if (nz.twoQubitDepolarising < tiny) {
-            for (int t : qs) mixDepolarising(q, t, nz.depolarising);
-        } else if (n == 1) {
-            mixDepolarising(q, qs[0], nz.depolarising);
-        }
-    }
-    if (nz.mixPauli > tiny)
-        for (int t : qs) mixPauli(q, t, nz.mixPauli, nz.mixPauli, nz.mixPauli);
-    if (nz.twoQubitDepolarising > tiny && n == 2) mixTwoQubitDepolarising(q, qs[0], qs[1], nz.twoQubitDepolarising);
-    if (nz.twoQubitDephasing > tiny && n == 2) mixTwoQubitDephasing(q, qs[0], qs[1], nz.twoQubitDephasing);
+    noiseAfterGate(o.code, qs.data(), (int)qs.size(), nz,
+                   [&](int channel, int a, int b, qreal p) { mixNoise(q, channel, a, b, p); });
 }
 
 bool hasNoise(const qmxNoiseAfterGate &nz) {
@@ -496,6 +549,63 @@ GateList gateList(const qmxCircuit *c, int numOps, bool everyOp) {
     return l;
 }
 
+// An operation list on a density register of n qubits as gates on its 2n row and
+// column bits (qmx_sweep.h), noise included. Lists that hold anything but one- and
+// two-qubit gates in matrix form, one-qubit channels and collapses are not taken.
+struct DensityList {
+    int n;
+    GateList l;
+    int last[64];               // per qubit: the last gate of the list that touches it
+    int operations = 0;
+    explicit DensityList(int numQubits) : n(numQubits) { std::fill(last, last + 64, -1); }
+    bool noise(int code, int q, double p) {
+        FlatGate g;
+        if (!channelGate(code, q, n, p, g)) return false;
+        ++operations;
+        // a run of channels on one qubit is one channel
+        if (last[q] >= 0 && l.gates[last[q]].kind == FlatGate::CHANNEL) {
+            joinChannel(l.gates[last[q]], g);
+            return true;
+        }
+        last[q] = (int)l.gates.size();
+        l.gates.push_back(g);
+        return true;
+    }
+    void gate(const FlatGate &g) {
+        ++operations;
+        FlatGate c = g;
+        c.target += n;
+        c.ctrl <<= n;
+        for (Cplx &z : c.u) z.im = -z.im;
+        l.gates.push_back(g);
+        l.gates.push_back(c);
+        for (uint64_t m = g.mask(); m; m &= m - 1) last[__builtin_ctzll(m)] = (int)l.gates.size() - 1;
+    }
+    void stop(int op) {
+        l.stops.push_back({(int)l.gates.size(), op});
+        std::fill(last, last + 64, -1);
+    }
+    // false: the list holds something that has no place here
+    bool add(int i, int code, const int *qs, int numQubits, double param, const qmxNoiseAfterGate *nz) {
+        FlatGate g;
+        if (code == QMX_OP_CC) {
+            stop(i);
+        } else if (isNoise(code)) {
+            if (!noise(code, qs[0], param)) return false;
+        } else if (!undispatched(code) && basicGate(code, qs, param, g)) {
+            gate(g);
+        } else {
+            return false;
+        }
+        bool ok = true;
+        if (nz)
+            noiseAfterGate(code, qs, numQubits, *nz, [&](int channel, int a, int, qreal p) {
+                ok = ok && noise(channel, a, p);
+            });
+        return ok;
+    }
+};
+
 // a gate list on a register of at most kSmallCircuitQubits qubits; stop(op)
 // runs an operation that is not a gate
 template <class F>
@@ -522,10 +632,27 @@ void planList(int numQubits, int prec, const GateList &l, qmx::SweepPlan &plan,
     int i = 0;
     for (size_t s = 0; s <= l.stops.size(); ++s) {
         const int until = s < l.stops.size() ? l.stops[s].first : (int)l.gates.size();
-        if (until > i)
-            qmx::planSweeps(numQubits, qmx::sweepLowBits(prec), l.gates.data() + i, until - i, i, plan);
+        if (until > i) qmx::planSweeps(qmx::sweepShape(numQubits, prec, false), l.gates.data() + i, until - i, i, plan);
         i = until;
         if (s < l.stops.size()) stops.push_back({(int)plan.sweeps.size(), l.stops[s].second});
+    }
+}
+
+// the list in sweeps of the register, planned and run at once
+template <class F>
+void runSweepsOnce(qmx::QuregDev *d, const GateList &l, F stop) {
+    int at = 0;
+    for (size_t s = 0; s <= l.stops.size(); ++s) {
+        const int until = s < l.stops.size() ? l.stops[s].first : (int)l.gates.size();
+        if (until > at) {
+            qmx::SweepPlan plan;
+            qmx::planSweeps(qmx::sweepShape(d->numQubits, d->prec, d->isDensity), l.gates.data() + at, until - at, 0,
+                            plan);
+            qmx::sweepRunOnce(d, plan, l.gates.data() + at);
+            if (d->isDensity) qmx::densCountSweeps((long long)plan.sweeps.size(), 0);
+        }
+        at = until;
+        if (s < l.stops.size()) stop(l.stops[s].second);
     }
 }
 
@@ -544,7 +671,7 @@ double applyCircuit(const Qureg &q, qmxCircuit *c, int fused) {
     const bool noisy = q.isDensityMatrix && hasNoise(c->noise);
     qmx::QuregDev *d = qmx::dev(q);
     const bool asBlocks = fused && !c->blocks.empty() && !q.isDensityMatrix;
-    if (qmx::smallCircuitSupported(d)) {
+    if (!q.isDensityMatrix && qmx::smallCircuitSupported(d)) {
         runSmall(d, asBlocks ? gateList(c, c->fusedOps, false) : gateList(c, (int)c->ops.size(), true),
                  [&](int op) { prob *= runOp(q, c->ops[op]); });
         return prob;
@@ -917,13 +1044,42 @@ qreal qmxApplyOperations(Qureg qureg, const qmxBasicOperation *ops, int numOps, 
         noiseParams(*noise, __func__);
         c.noise = *noise;
     }
-    // State vectors whose gates need no recording (one LDS circuit, or sweeps):
-    // straight from the caller's list to the kernels' gates.
+    // Lists that need no recording (one LDS circuit, or sweeps): straight from the
+    // caller's list to the kernels' gates. On density registers the list, noise
+    // included, is planned as a whole over the 2n row and column bits; one pass for
+    // each two composed pairs of qubits, what API calls make of it, costs 4 us of host
+    // time an operation and fills a pass with two blocks: 7 qubits FP64, 60 operations
+    // with noise and 8 reads, 1380 us that way and 240 in sweeps; 13 qubits FP32, 120
+    // operations and 14 reads, 27 passes in 6.9 ms and 12 sweeps in 3.6.
     qmx::QuregDev *d = qmx::dev(qureg);
     const bool small = qmx::smallCircuitSupported(d);
-    const bool sweeps = !qureg.isDensityMatrix && fuseQubits == qmx::kSweepBlockQubits &&
-                        qmx::sweepSupported(d->numQubits);
-    if (small || sweeps) {
+    const bool sweeps = fuseQubits == qmx::kSweepBlockQubits && qmx::sweepSupported(d->numQubits);
+    double prob = 1.0;
+    auto stop = [&](int i) {
+        Op o;
+        o.code = ops[i].operation;
+        o.qubits.assign(ops[i].qubits, ops[i].qubits + std::max(0, ops[i].numQubits));
+        o.param = (double)ops[i].param;
+        prob *= runOp(qureg, o);
+    };
+    const char *badFuse = "Invalid block size. Fused blocks span at least 1 and at most 10 qubits.";
+    if (qureg.isDensityMatrix && fuseQubits >= 0 && fuseQubits <= 10) {
+        for (int i = 0; i < numOps; ++i)
+            checkBasic(c.shape, ops[i].operation, ops[i].qubits, ops[i].numQubits, (double)ops[i].param, __func__);
+        DensityList dl(c.numQubits);
+        bool taken = true;
+        for (int i = 0; i < numOps && taken; ++i)
+            taken = dl.add(i, ops[i].operation, ops[i].qubits, ops[i].numQubits, (double)ops[i].param,
+                           hasNoise(c.noise) ? &c.noise : nullptr);
+        if (taken) {
+            if (small)
+                runSmall(d, dl.l, stop);
+            else
+                runSweepsOnce(d, dl.l, stop);
+            qmx::densCountSweeps(0, dl.operations);
+            return (qreal)prob;
+        }
+    } else if (!qureg.isDensityMatrix && (small || sweeps)) {
         GateList l;
         l.gates.reserve(numOps);
         for (int i = 0; i < numOps; ++i) {
@@ -935,38 +1091,17 @@ qreal qmxApplyOperations(Qureg qureg, const qmxBasicOperation *ops, int numOps, 
             else if (o.operation == QMX_OP_CC || (fuseQubits == 0 && undispatched(o.operation)))
                 l.stops.push_back({(int)l.gates.size(), i});
         }
-        if (fuseQubits < 0 || fuseQubits > 10)
-            qv::raise("Invalid block size. Fused blocks span at least 1 and at most 10 qubits.", __func__);
-        double prob = 1.0;
-        auto stop = [&](int i) {
-            Op o;
-            o.code = ops[i].operation;
-            o.qubits.assign(ops[i].qubits, ops[i].qubits + std::max(0, ops[i].numQubits));
-            o.param = (double)ops[i].param;
-            prob *= runOp(qureg, o);
-        };
-        if (small) {
+        if (fuseQubits < 0 || fuseQubits > 10) qv::raise(badFuse, __func__);
+        if (small)
             runSmall(d, l, stop);
-            return (qreal)prob;
-        }
-        int at = 0;
-        for (size_t s = 0; s <= l.stops.size(); ++s) {
-            const int until = s < l.stops.size() ? l.stops[s].first : (int)l.gates.size();
-            if (until > at) {
-                qmx::SweepPlan plan;
-                qmx::planSweeps(c.numQubits, qmx::sweepLowBits(d->prec), l.gates.data() + at, until - at, 0, plan);
-                qmx::sweepRunOnce(d, plan, l.gates.data() + at);
-            }
-            at = until;
-            if (s < l.stops.size()) stop(l.stops[s].second);
-        }
+        else
+            runSweepsOnce(d, l, stop);
         return (qreal)prob;
     }
     for (int i = 0; i < numOps; ++i)
         recordBasic(&c, ops[i].operation, ops[i].qubits, ops[i].numQubits, (double)ops[i].param, __func__);
     if (fuseQubits != 0) {
-        if (fuseQubits < 1 || fuseQubits > 10)
-            qv::raise("Invalid block size. Fused blocks span at least 1 and at most 10 qubits.", __func__);
+        if (fuseQubits < 1 || fuseQubits > 10) qv::raise(badFuse, __func__);
         if (!qureg.isDensityMatrix) fuseCircuit(&c, fuseQubits);
     }
     return (qreal)applyCircuit(qureg, &c, fuseQubits != 0);

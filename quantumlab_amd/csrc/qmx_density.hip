@@ -9,7 +9,8 @@
 // and damping (QuEST_gpu.cu:3027-3078). Here every operation on at most two
 // qubits composes on the host into one 4^k x 4^k superoperator (k <= 2), and
 // the register is swept once per composed run: a brick-circuit gate with its
-// three channels per touched qubit is one sweep instead of five to eight.
+// three channels per touched qubit is one sweep instead of five to eight. (Operation
+// lists know what comes next and are planned as a whole instead: qmx_circuit.cpp.)
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -336,6 +337,11 @@ void densDropPending(const QuregDev *q) {
         g_pend.blocks.clear();
         setPendingWork(nullptr);
     }
+}
+
+void densCountSweeps(long long passes, long long absorbed) {
+    g_passes += passes;
+    g_absorbed += absorbed;
 }
 
 void densSuperOpStats(long long *passes, long long *absorbed) {

@@ -215,5 +215,7 @@ void densSuperOp(QuregDev *q, const int *targets, int k, const Cplx *S);
 void densUnitary(QuregDev *q, const int *targets, int k, const Cplx *u, const Cplx *uc);
 void densDropPending(const QuregDev *q);        // register being destroyed
 void densSuperOpStats(long long *passes, long long *absorbed);
+// counts of operations applied in sweeps planned elsewhere
+void densCountSweeps(long long passes, long long absorbed);
 
 }  // namespace qmx

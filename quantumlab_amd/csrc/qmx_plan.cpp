@@ -18,7 +18,30 @@ namespace {
 
 int popcount(uint64_t x) { return __builtin_popcountll(x); }
 
-int weightOf(const FlatGate &g) { return g.kind == FlatGate::MATRIXN ? 64 : 1; }
+int weightOf(const FlatGate &g) { return g.kind == FlatGate::MATRIXN && g.k > 2 ? (1 << (2 * g.k)) / 16 : 1; }
+
+// Planning order of a register's bits: itself, or for density registers row and
+// column bit of a qubit side by side (bit q to 2q, bit q + bits/2 to 2q + 1), so that
+// a window of consecutive bits is a run of whole qubits.
+uint64_t toOrder(const SweepShape &s, uint64_t mask) {
+    if (!s.density) return mask;
+    const int half = s.bits / 2;
+    uint64_t m = 0;
+    for (; mask; mask &= mask - 1) {
+        const int b = __builtin_ctzll(mask);
+        m |= 1ull << (b < half ? 2 * b : 2 * (b - half) + 1);
+    }
+    return m;
+}
+uint64_t fromOrder(const SweepShape &s, uint64_t mask) {
+    if (!s.density) return mask;
+    uint64_t m = 0;
+    for (; mask; mask &= mask - 1) {
+        const int b = __builtin_ctzll(mask);
+        m |= 1ull << (b / 2 + (b & 1 ? s.bits / 2 : 0));
+    }
+    return m;
+}
 
 struct Item {
     int id;          // index into the gate list
@@ -137,11 +160,13 @@ void planBlocks(std::vector<Item> rem, int base, SweepPlan &plan, std::vector<ui
 
 }  // namespace
 
-void planSweeps(int n, int lowBits, const FlatGate *gates, int count, int base, SweepPlan &plan) {
+void planSweeps(const SweepShape &shape, const FlatGate *gates, int count, int base, SweepPlan &plan) {
+    const int n = shape.bits;
     std::vector<Item> rem(count);
-    for (int i = 0; i < count; ++i) rem[i] = Item{i, gates[i].mask(), weightOf(gates[i])};
-    const int tileBits = std::min(sweepTileBits(n), n);
-    const uint64_t low = (1ull << std::min(lowBits, n)) - 1ull;
+    for (int i = 0; i < count; ++i) rem[i] = Item{i, toOrder(shape, gates[i].mask()), weightOf(gates[i])};
+    const int tileBits = std::min(shape.tileBits, n), lowBits = std::min(shape.lowBits, n);
+    const uint64_t low = toOrder(shape, (1ull << lowBits) - 1ull);
+    const int firstStart = shape.density ? 0 : lowBits, step = shape.density ? 2 : 1;
     std::vector<int> taken;
     std::vector<Item> mine;
     std::vector<uint64_t> blockMasks;
@@ -153,7 +178,7 @@ void planSweeps(int n, int lowBits, const FlatGate *gates, int count, int base, 
         // the lowest qubits and a window of consecutive others
         uint64_t window = 0;
         int best = 0;
-        for (int s = std::min(lowBits, n); s == std::min(lowBits, n) || s + tileBits - lowBits <= n; ++s) {
+        for (int s = firstStart; s == firstStart || s + tileBits - lowBits <= n; s += step) {
             uint64_t w = low;
             for (int b = s; b < n && popcount(w) < tileBits; ++b) w |= 1ull << b;
             w = padLow(w, n, tileBits);
@@ -197,12 +222,13 @@ void planSweeps(int n, int lowBits, const FlatGate *gates, int count, int base, 
             uint64_t m = blockMasks[i];
             for (int q = 63; q >= 0 && popcount(m) < b.k; --q)
                 if ((tile >> q) & 1) m |= 1ull << q;
+            m = fromOrder(shape, m);
             int j = 0;
             for (uint64_t x = m; x; x &= x - 1) b.targs[j++] = __builtin_ctzll(x);
         }
         for (int b = firstBlock; b < (int)plan.blocks.size(); b += kSweepMaxBlocks)
             plan.sweeps.push_back(
-                Sweep{tile, b, std::min(kSweepMaxBlocks, (int)plan.blocks.size() - b), -1});
+                Sweep{fromOrder(shape, tile), b, std::min(kSweepMaxBlocks, (int)plan.blocks.size() - b), -1});
     }
 }
 

@@ -8,9 +8,14 @@
 
 namespace qmx {
 
-// one unitary in matrix form
+// One operation on a state vector in matrix form. A density register is the
+// vector of its 2n row and column bits: a unitary is a gate on its row bits and the
+// conjugate one on its column bits. CHANNEL is a one-qubit channel with real maps of
+// its qubit's diagonal entries, (x00, x11) -> (d00 x00 + d01 x11, d10 x00 + d11 x11),
+// and off-diagonal ones, (x01, x10) -> (f x01 + g x10, g x01 + f x10): target = the
+// row bit, k = the column bit, u = {(f, g), (d00, d01), (d10, d11), unused}.
 struct FlatGate {
-    enum Kind { MATRIX2 = 0, NOT = 1, MATRIXN = 2 };
+    enum Kind { MATRIX2 = 0, NOT = 1, MATRIXN = 2, CHANNEL = 3 };
     int kind = MATRIX2;
     int target = 0;                // MATRIX2, NOT
     uint64_t ctrl = 0;             // controls (all kinds; acts where they are 1)
@@ -24,6 +29,7 @@ struct FlatGate {
             for (int j = 0; j < k; ++j) m |= 1ull << targs[j];
         else
             m |= 1ull << target;
+        if (kind == CHANNEL) m |= 1ull << k;
         return m;
     }
 };
@@ -39,7 +45,7 @@ constexpr int kSweepTileBits = 12;
 constexpr int sweepTileBits(int numQubits) { return numQubits < 20 ? kSweepTileBits - 1 : kSweepTileBits; }
 constexpr int kSweepBlockQubits = 5;
 constexpr int kSweepMaxBlocks = 64;    // blocks of one sweep
-constexpr int kSweepMaxWeight = 512;   // gates of one block (a MATRIXN counts as 64)
+constexpr int kSweepMaxWeight = 512;   // gates of one block (a MATRIXN of more than two qubits counts as 4^k / 16)
 inline int sweepLowBits(int prec) { return prec == FP64 ? 3 : 4; }
 // registers the sweeps serve (smaller ones are one tile: see smallCircuit)
 constexpr int kSmallCircuitQubits = 12;
@@ -60,8 +66,19 @@ struct SweepPlan {
     std::vector<SweepBlock> blocks;
     std::vector<Sweep> sweeps;
 };
+// What is planned for: registers of `bits` bits, tiles of `tileBits` that always hold
+// the lowest `lowBits`. density: bits b and b + bits/2 belong together (a qubit's
+// row and column bit), so windows take them in pairs.
+struct SweepShape {
+    int bits, lowBits, tileBits;
+    bool density;
+};
+inline SweepShape sweepShape(int numBits, int prec, bool density) {
+    // density tiles: a qubit is two bits, so 12 hold twice the pairs of 8
+    return SweepShape{numBits, sweepLowBits(prec), density ? kSweepTileBits : sweepTileBits(numBits), density};
+}
 // Appends the sweeps of gates[0 .. count) to `plan` (gate indices offset by `base`).
-void planSweeps(int numQubits, int lowBits, const FlatGate *gates, int count, int base, SweepPlan &plan);
+void planSweeps(const SweepShape &shape, const FlatGate *gates, int count, int base, SweepPlan &plan);
 
 // A plan's blocks on the device (matrices built there from the gates).
 struct SweepProgram;
@@ -77,7 +94,15 @@ void sweepRunOnce(QuregDev *q, const SweepPlan &plan, const FlatGate *gates);
 void applyFlatGate(QuregDev *q, const FlatGate &g);
 
 // ---- small registers: the whole register in one workgroup's LDS -----------------
-inline bool smallCircuitSupported(const QuregDev *q) { return !q->isDensity && q->numQubits <= kSmallCircuitQubits; }
+// A density operation is three or four steps of the LDS kernel (rows, columns,
+// channels; 0.8 us each), where a tile of 12 bits takes whole blocks of them: 6
+// qubits, 82 operations with their noise and reads, FP64 379 us there and 216 in
+// sweeps. In FP32 it would be 378 and 198, but the LDS kernel's FP64 arithmetic keeps
+// 2.2e-7 from the 64-bit state where sweeps leave 3.5e-7 (and one pass for each pair
+// of qubits 2.4e-7).
+inline bool smallCircuitSupported(const QuregDev *q) {
+    return q->numQubits <= (q->isDensity && q->prec == FP64 ? 10 : kSmallCircuitQubits);
+}
 // gates[0 .. count) in order, one launch per few hundred of them; no MATRIXN
 void smallCircuit(QuregDev *q, const FlatGate *gates, int count);
 

@@ -60,12 +60,13 @@ typedef double d8 __attribute__((ext_vector_type(8)));
 
 struct GateDev {
     int kind;            // FlatGate::Kind
-    unsigned t;          // target, a bit of the block's index; MATRIXN: its targets, 4 bits each
+    unsigned t;          // target, a bit of the block's index; MATRIXN: its targets, 4 bits each;
+                         // CHANNEL: row bit | column bit << 4
     unsigned ctrl;       // controls, bits of the block's index
     int k;               // MATRIXN
     int mat;             // MATRIXN: its matrix (entry offset)
     int pad[3];
-    alignas(16) double u[8];  // the matrix, (re, im) by rows
+    alignas(16) double u[8];  // the matrix, (re, im) by rows; CHANNEL: f, g, d00, d01, d10, d11
 };
 
 // gates staged in LDS at a time (whole coalesced loads; one entry more is read)
@@ -150,6 +151,24 @@ __global__ void __launch_bounds__(kBlock) kBuildBlocks(const BuildDev *__restric
         }
         const GateDev G = uniformGate(next);
         next = stage[g % kStage + 1];  // past a stage's last one: unused
+        if (G.kind == FlatGate::CHANNEL) {
+            const unsigned b0 = 1u << (G.t & 15u), b1 = 1u << (G.t >> 4);
+            const unsigned lo = ~(min(b0, b1) - 1u), hi = ~(max(b0, b1) - 1u);
+            for (unsigned p = lane >> cb; p < (unsigned)pairs / 2; p += 64 >> cb) {
+                unsigned r = p + (p & lo);
+                r += r & hi;
+                Amp<double> *p00 = M + (r << k) + col, *p11 = p00 + ((b0 | b1) << k);
+                Amp<double> *p01 = p00 + (b0 << k), *p10 = p00 + (b1 << k);
+                const Amp<double> x = *p00, y = *p11, v = *p01, w = *p10;
+                *p00 = Amp<double>{G.u[2] * x.x + G.u[3] * y.x, G.u[2] * x.y + G.u[3] * y.y};
+                *p11 = Amp<double>{G.u[4] * x.x + G.u[5] * y.x, G.u[4] * x.y + G.u[5] * y.y};
+                *p01 = Amp<double>{G.u[0] * v.x + G.u[1] * w.x, G.u[0] * v.y + G.u[1] * w.y};
+                *p10 = Amp<double>{G.u[1] * v.x + G.u[0] * w.x, G.u[1] * v.y + G.u[0] * w.y};
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            continue;
+        }
         if (G.kind != FlatGate::MATRIXN) {
             // row r0 of pair p: p with a zero inserted at the target
             const unsigned bit = 1u << G.t, high = ~(bit - 1u);
@@ -465,11 +484,11 @@ __global__ void __launch_bounds__(64 * WAVES, sizeof(T) == 4 ? 4 : 2)
 struct SmallGate {
     unsigned what;               // SG_*
     unsigned bit;                // the target's bit, as a byte offset of the LDS register (16 B an amplitude)
-    unsigned ctrl;               // the controls' bits, likewise
+    unsigned ctrl;               // the controls' bits, likewise; SG_CHANNEL: the column bit
     unsigned pad;
     alignas(16) double u[8];     // the matrix, (re, im) by rows
 };
-enum { SG_GENERAL = 0, SG_NOT = 1, SG_PHASE = 2, SG_REAL = 3 };  // SG_PHASE: diag(1, u)
+enum { SG_GENERAL = 0, SG_NOT = 1, SG_PHASE = 2, SG_REAL = 3, SG_CHANNEL = 4 };  // SG_PHASE: diag(1, u)
 constexpr int kSmallStage = 256;
 constexpr int kSmallThreads = 1024;
 
@@ -497,6 +516,21 @@ __global__ void __launch_bounds__(kSmallThreads) kSmallCircuit(Amp<T> *__restric
         // past a stage's last one: unused
         nextHead = *reinterpret_cast<const uint4 *>(stage + g % kSmallStage + 1);
         nextU = matrixOf(stage[g % kSmallStage + 1].u);
+        if (what == SG_CHANNEL) {
+            const unsigned lo = ~(min(bit, ctrl) - 1u), hi = ~(max(bit, ctrl) - 1u);
+            for (unsigned w = 16u * tid; w < 4u * dim; w += 16u * step) {
+                unsigned i = w + (w & lo);
+                i += i & hi;
+                Amp<double> &A = at(i), &B = at(i + bit), &C = at(i + ctrl), &D = at(i + bit + ctrl);
+                const Amp<double> x = A, y = D, v = B, z = C;
+                A = Amp<double>{u[2] * x.x + u[3] * y.x, u[2] * x.y + u[3] * y.y};
+                D = Amp<double>{u[4] * x.x + u[5] * y.x, u[4] * x.y + u[5] * y.y};
+                B = Amp<double>{u[0] * v.x + u[1] * z.x, u[0] * v.y + u[1] * z.y};
+                C = Amp<double>{u[1] * v.x + u[0] * z.x, u[1] * v.y + u[0] * z.y};
+            }
+            __syncthreads();
+            continue;
+        }
         for (unsigned w = 16u * tid; w < 8u * dim; w += 16u * step) {
             const unsigned i = w + (w & high);  // the pair's index with a zero inserted at the target
             if ((i & ctrl) != ctrl) continue;
@@ -591,6 +625,12 @@ void fillBuild(const SweepPlan &plan, const FlatGate *gates, int firstBlock, int
                 const int entries = 1 << (2 * f.k);
                 for (int e = 0; e < entries; ++e) mats[mat + e] = Amp<double>{f.uN[e].re, f.uN[e].im};
                 mat += entries;
+            } else if (f.kind == FlatGate::CHANNEL) {
+                d.t = (unsigned)local(f.target) | (unsigned)local(f.k) << 4;
+                for (int e = 0; e < 4; ++e) {
+                    d.u[2 * e] = f.u[e].re;
+                    d.u[2 * e + 1] = f.u[e].im;
+                }
             } else {
                 d.t = (unsigned)local(f.target);
                 for (int e = 0; e < 4; ++e) {
@@ -705,7 +745,7 @@ void launchTiles(QuregDev *q, const Sweep &w, const BlockDev *blocks, const char
 template <typename T>
 void launchSweep(QuregDev *q, const Sweep &w, const BlockDev *blocks, const char *frags) {
     constexpr int perCU = sizeof(T) == 4 ? 4 : 2;
-    if (sweepTileBits(q->numQubits) < kSweepTileBits)
+    if (__builtin_popcountll(w.tile) < kSweepTileBits)
         launchTiles<T, false, 4, kSweepTileBits - 1>(q, w, blocks, frags);
     else if ((q->numAmps >> kSweepTileBits) < (long long)perCU * numCUs())
         launchTiles<T, false, 8, kSweepTileBits>(q, w, blocks, frags);
@@ -849,6 +889,19 @@ void applyFlatGate(QuregDev *q, const FlatGate &g) {
         applyNot(q, g.ctrl, 1ull << g.target);
         return;
     }
+    if (g.kind == FlatGate::CHANNEL) {
+        // entry e = row bit + 2 * column bit
+        const int bits[2] = {g.target, g.k};
+        Cplx S[16] = {};
+        S[0] = {g.u[1].re, 0};
+        S[3] = {g.u[1].im, 0};
+        S[12] = {g.u[2].re, 0};
+        S[15] = {g.u[2].im, 0};
+        S[5] = S[10] = {g.u[0].re, 0};
+        S[6] = S[9] = {g.u[0].im, 0};
+        applyDense(q, bits, 2, S);
+        return;
+    }
     auto is = [](const Cplx &z, double re) { return z.re == re && z.im == 0; };
     if (is(g.u[0], 1) && is(g.u[1], 0) && is(g.u[2], 0)) {
         applyPhaseOnAllOnes(q, g.ctrl | (1ull << g.target), g.u[3]);
@@ -860,6 +913,7 @@ void applyFlatGate(QuregDev *q, const FlatGate &g) {
 // a gate's arithmetic, by the entries of its matrix
 static int smallKind(const FlatGate &f) {
     if (f.kind == FlatGate::NOT) return SG_NOT;
+    if (f.kind == FlatGate::CHANNEL) return SG_CHANNEL;
     auto is = [](const Cplx &z, double re) { return z.re == re && z.im == 0; };
     if (is(f.u[0], 1) && is(f.u[1], 0) && is(f.u[2], 0)) return SG_PHASE;
     for (const Cplx &z : f.u)
@@ -883,7 +937,7 @@ void smallCircuit(QuregDev *q, const FlatGate *gates, int count) {
             SmallGate &d = h[i];
             d.what = (unsigned)smallKind(f);
             d.bit = 16u << f.target;
-            d.ctrl = 16u * (unsigned)f.ctrl;
+            d.ctrl = f.kind == FlatGate::CHANNEL ? 16u << f.k : 16u * (unsigned)f.ctrl;
             d.pad = 0;
             for (int e = 0; e < 4; ++e) {
                 d.u[2 * e] = f.u[e].re;

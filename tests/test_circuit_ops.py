@@ -346,3 +346,55 @@ def test_operation_lists_with_collapses_between_sweeps(gpu, cpuref, n, fuse):
     assert abs(got - want) < TOL
     assert np.max(np.abs(gpu.state(q) - ref)) < TOL
     gpu.destroy(q)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 6, 7, 8, 10])
+@pytest.mark.parametrize("precision", [None, QMX_PREC_FP32])
+@pytest.mark.parametrize("after", [None, dict(damping=0.03, dephasing=0.02, depolarising=0.01),
+                                   dict(mixPauli=0.02)])
+def test_density_lists_match_oracle(gpu, cpuref, n, precision, after):
+    """qmxApplyOperations on density registers at the edges of its two forms (the
+    register in one workgroup's LDS up to 5 or 6 qubits, tile sweeps of the rows and
+    columns above): every gate, every one-qubit channel and a collapse, from a state
+    that is not symmetric between rows and columns."""
+    rng = np.random.default_rng(40 + n)
+    one = [O.H, O.X, O.Y, O.Z, O.P, O.RX, O.RY, O.RZ]
+    two = [O.CX, O.CY, O.CZ, O.CP, O.CRX, O.CRY, O.CRZ]
+    channels = [O.NOISE_DAMPING, O.NOISE_DEPHASING, O.NOISE_DEPOLARISING, O.NOISE_MIX_X, O.NOISE_MIX_Y,
+                O.NOISE_MIX_Z, O.NOISE_MIX_ALL]
+    ops = []
+    for i in range(60):
+        qs = [int(x) for x in rng.permutation(n)[:2]]
+        code = int(rng.choice(one + two if n > 1 else one))
+        ops.append((code, qs if code in two else qs[:1], float(rng.uniform(0, 6))))
+        if i % 3 == 0:
+            ops.append((int(rng.choice(channels)), qs[:1], float(rng.uniform(0, 0.2))))
+        if i == 40:
+            ops += [(O.RY, qs[:1], 0.9), (O.CC, qs[:1], 0.0)]
+
+    def start(lib, q):
+        lib.initPlusState(q)
+        for j in range(n):
+            lib.rotateZ(q, j, 0.4 + 0.2 * j)
+
+    qc = cpuref.qureg(n, density=True)
+    start(cpuref, qc)
+    ops = resolve_collapses(cpuref, qc, [(c, q, -1.0 if c == O.CC else t) for c, q, t in ops], after)
+    ref = cpuref.state(qc)
+    cpuref.destroy(qc)
+    arr = (BasicOperation * len(ops))()
+    for a, (code, qs, t) in zip(arr, ops):
+        a.operation, a.numQubits, a.param = code, len(qs), t
+        for j, x in enumerate(qs):
+            a.qubits[j] = x
+    noise = C.byref(NoiseAfterGate(**after)) if after else None
+    # entries are at most 1 and no operation enlarges an error by more than the
+    # collapse's 1/p <= 2: a few ulps an operation
+    tol = TOL if precision is None else 2.0 ** -21 * np.sqrt(len(ops))
+    for fuse in (0, 5):
+        q = gpu.qureg(n, density=True, precision=precision)
+        start(gpu, q)
+        gpu.qmxApplyOperations(q, arr, len(ops), noise, fuse)
+        assert np.max(np.abs(gpu.state(q) - ref)) < tol
+        gpu.destroy(q)
