@@ -104,11 +104,17 @@ __device__ __forceinline__ Amp<double> rowTimes(double a, double b, double c, do
                                                 const Amp<double> &q) {
     return Amp<double>{a * p.x - b * p.y + c * q.x - d * q.y, a * p.y + b * p.x + c * q.y + d * q.x};
 }
+// what a tile sweep needs of a block besides its vectors
+struct BlockDev {
+    int k;
+    unsigned rest[4];    // slots of the tile's bits beyond columns and targets: 16-group chunks
+};
 struct BuildDev {
     int firstGate, numGates, k, pad;
     // byte offsets of the LDS slots: column bits, combination bits 0 and 1,
     // combinations 4 st
     unsigned col[4], kq[2], st[8];
+    BlockDev tile;
 };
 
 // What a lane needs of a block, in 16 B vectors (vector i of all lanes, then i + 1):
@@ -128,24 +134,32 @@ template <> struct Frag<double> { typedef d2 V; };
 // of ten gates took ~25 us). A wave owns a quarter of the matrix's columns, which no
 // other wave touches, so gates follow one another without barriers; each gate is
 // read from LDS while the one before it is applied (scalar loads straight from
-// memory arrive a line at a time, 0.65 us a gate).
+// memory arrive a line at a time, 0.65 us a gate). todo and gates may lie in pinned host
+// memory: each is read once, whole, into LDS.
 template <typename T>
 __global__ void __launch_bounds__(kBlock) kBuildBlocks(const BuildDev *__restrict__ todo,
                                                        const GateDev *__restrict__ gates,
-                                                       const Amp<double> *__restrict__ mats, char *__restrict__ out) {
+                                                       const Amp<double> *__restrict__ mats, char *__restrict__ out,
+                                                       BlockDev *__restrict__ blocks) {
     __shared__ Amp<double> buf[2][32 * 32];
     __shared__ GateDev stage[kStage + 1];
-    const BuildDev &b = todo[blockIdx.x];
-    const int k = b.k, dim = 1 << k, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ BuildDev b;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    static_assert(sizeof(BuildDev) / 4 <= 64, "one load a lane");
+    if (tid < (int)(sizeof(BuildDev) / 4))
+        reinterpret_cast<unsigned *>(&b)[tid] = reinterpret_cast<const unsigned *>(todo + blockIdx.x)[tid];
+    __syncthreads();
+    if (tid == 0) blocks[blockIdx.x] = b.tile;
+    const int k = (int)uniform((unsigned)b.k), dim = 1 << k, numGates = (int)uniform((unsigned)b.numGates);
     Amp<double> *M = buf[0], *N = buf[1];
     for (int i = tid; i < dim * dim; i += kBlock) M[i] = Amp<double>{(i >> k) == (i & (dim - 1)) ? 1.0 : 0.0, 0.0};
     // pairs of a wave: dim/4 columns x dim/2 row pairs, 32 (k = 4) or 128 (k = 5)
     const int cb = k - 2, col = wave * (dim / 4) + (lane & ((1 << cb) - 1)), pairs = dim / 2;
     GateDev next{};
-    for (int g = 0; g < b.numGates; ++g) {
+    for (int g = 0; g < numGates; ++g) {
         if (g % kStage == 0) {
             __syncthreads();
-            stageGates(stage, gates + b.firstGate + g, min(kStage, b.numGates - g), tid, kBlock);
+            stageGates(stage, gates + b.firstGate + g, min(kStage, numGates - g), tid, kBlock);
             __syncthreads();
             next = stage[0];
         }
@@ -261,11 +275,6 @@ __global__ void __launch_bounds__(kBlock) kBuildBlocks(const BuildDev *__restric
 // ---- the tile kernel ---------------------------------------------------------------
 // LDS slots are linear in the tile element (see the top of the file), so a slot is
 // the XOR of its bits' slots; here as byte offsets
-struct BlockDev {
-    int k;
-    unsigned rest[4];    // slots of the tile's bits beyond columns and targets: 16-group chunks
-};
-
 struct TileGeom {
     int pos[kMaxTB];     // the tile's qubits, ascending
     uint64_t jAddr[16];  // register offset of a thread's j-th transfer
@@ -560,10 +569,9 @@ __global__ void __launch_bounds__(kSmallThreads) kSmallCircuit(Amp<T> *__restric
 // ---- host side -----------------------------------------------------------------------
 size_t align16(size_t x) { return (x + 15) & ~(size_t)15; }
 
-// One upload holds the build list, the gates and their matrices, then the blocks'
-// kernel descriptions.
+// One upload holds the build list, the gates and their matrices.
 struct Upload {
-    size_t todo, gates, mats, blocks, bytes;
+    size_t todo, gates, mats, bytes;
 };
 
 int numMats(const FlatGate *gates, const SweepPlan &plan, int firstBlock, int numBlocks, size_t *entries) {
@@ -592,8 +600,7 @@ Upload layoutOf(const SweepPlan &plan, const FlatGate *gates, int firstBlock, in
     u.todo = 0;
     u.gates = align16(numBlocks * sizeof(BuildDev));
     u.mats = u.gates + align16((size_t)gateCount(plan, firstBlock, numBlocks) * sizeof(GateDev));
-    u.blocks = u.mats + entries * sizeof(Amp<double>);
-    u.bytes = align16(u.blocks + numBlocks * sizeof(BlockDev));
+    u.bytes = u.mats + entries * sizeof(Amp<double>);
     return u;
 }
 
@@ -605,7 +612,10 @@ void fillBuild(const SweepPlan &plan, const FlatGate *gates, int firstBlock, int
     int at = 0, mat = 0;
     for (int i = 0; i < numBlocks; ++i) {
         const SweepBlock &b = plan.blocks[firstBlock + i];
-        todo[i] = BuildDev{at, b.numGates, b.k, 0, {}, {}, {}};
+        todo[i] = BuildDev{};
+        todo[i].firstGate = at;
+        todo[i].numGates = b.numGates;
+        todo[i].k = b.k;
         auto local = [&](int qubit) {
             for (int j = 0; j < b.k; ++j)
                 if (b.targs[j] == qubit) return j;
@@ -655,10 +665,9 @@ int tilePositions(uint64_t tile, int pos[kMaxTB]) {
 }
 
 template <typename T>
-void blockSlots(const SweepBlock &b, const int *pos, int tb, BuildDev &todo, BlockDev &d) {
+void blockSlots(const SweepBlock &b, const int *pos, int tb, BuildDev &todo) {
     constexpr int R = sizeof(T) == 4 ? 4 : 3;   // columns per bank cycle: 2^R lanes
-    d = BlockDev{};
-    d.k = b.k;
+    todo.tile.k = b.k;
     int t[kSweepBlockQubits];
     bool used[kMaxTB] = {};
     for (int j = 0; j < b.k; ++j) {
@@ -691,29 +700,30 @@ void blockSlots(const SweepBlock &b, const int *pos, int tb, BuildDev &todo, Blo
         for (int j = 2; j < b.k; ++j)
             if ((st >> (j - 2)) & 1) todo.st[st] ^= slot(t[j]);
     for (int i = 0, r = 0; i < tb; ++i)
-        if (!used[i]) d.rest[r++] = slot(i);
+        if (!used[i]) todo.tile.rest[r++] = slot(i);
 }
 
-// LDS slots and descriptions of the blocks that sweeps [first, last) hold
+// LDS slots of the blocks that sweeps [first, last) hold
 void fillBlocks(int prec, const SweepPlan &plan, int first, int last, int firstBlock, const Upload &u, char *host) {
     BuildDev *todo = reinterpret_cast<BuildDev *>(host + u.todo);
-    BlockDev *out = reinterpret_cast<BlockDev *>(host + u.blocks);
     for (int s = first; s < last; ++s) {
         const Sweep &w = plan.sweeps[s];
         if (w.lone >= 0) continue;
         int pos[kMaxTB];
         const int tb = tilePositions(w.tile, pos);
         for (int b = w.firstBlock; b < w.firstBlock + w.numBlocks; ++b)
-            QMX_DISPATCH(prec, T, { blockSlots<T>(plan.blocks[b], pos, tb, todo[b - firstBlock], out[b - firstBlock]); });
+            QMX_DISPATCH(prec, T, { blockSlots<T>(plan.blocks[b], pos, tb, todo[b - firstBlock]); });
     }
 }
 
-void launchBuild(int prec, int numBlocks, const Upload &u, char *dev, char *frags) {
-    const BuildDev *todo = reinterpret_cast<const BuildDev *>(dev + u.todo);
-    const GateDev *gd = reinterpret_cast<const GateDev *>(dev + u.gates);
-    const Amp<double> *mats = reinterpret_cast<const Amp<double> *>(dev + u.mats);
+// from `src`, an upload that the device can read
+void launchBuild(int prec, int numBlocks, const Upload &u, const char *src, char *frags, BlockDev *blocks) {
+    const BuildDev *todo = reinterpret_cast<const BuildDev *>(src + u.todo);
+    const GateDev *gd = reinterpret_cast<const GateDev *>(src + u.gates);
+    const Amp<double> *mats = reinterpret_cast<const Amp<double> *>(src + u.mats);
     QMX_DISPATCH(prec, T, {
-        hipLaunchKernelGGL(kBuildBlocks<T>, dim3(numBlocks), dim3(kBlock), 0, hstream(), todo, gd, mats, frags);
+        hipLaunchKernelGGL(kBuildBlocks<T>, dim3(numBlocks), dim3(kBlock), 0, hstream(), todo, gd, mats, frags,
+                           blocks);
     });
     checkLaunch("sweep block matrices");
 }
@@ -769,45 +779,51 @@ void runSweeps(QuregDev *q, const SweepPlan &plan, const FlatGate *gates, int fi
     }
 }
 
-// The library's workspace for lists applied once: the upload (pinned and on the
-// device) and the fragments of a batch of blocks. It grows to what a batch
-// needs and no further; the host copy is rewritten after its last copy's event,
-// the device side by work queued behind everything that read it.
+// The library's workspace for lists applied once. The gates lie in pinned host memory,
+// where the one kernel that wants them reads them (17 qubits FP64, 300 gates: 148 us,
+// 178 with a copy to the device before it and one of the results): two buffers in
+// turn, each rewritten after the event behind its last reader. The fragments and
+// descriptions of a batch of blocks are on the device, rewritten by work queued
+// behind everything that read them. All grow to what a batch needs and no further.
 constexpr int kBatchBlocks = 256;
 struct Workspace {
-    char *host = nullptr, *dev = nullptr, *frags = nullptr;
-    size_t bytes = 0;
+    struct Host {
+        char *p = nullptr;
+        size_t bytes = 0;
+        hipEvent_t ev = nullptr;
+        bool used = false;
+    } host[2];
+    int at = 0;
+    char *frags = nullptr;
     int fragBlocks = 0;
-    hipEvent_t ev = nullptr;
-    bool used = false;
 
     char *hostRoom(size_t need) {
-        if (!ev) QMX_HIP_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-        if (need > bytes) {
-            deviceSync();  // the old buffers may still be in use
-            if (dev) QMX_HIP_CHECK(hipFree(dev));
-            if (host) QMX_HIP_CHECK(hipHostFree(host));
-            bytes = std::max(need, (size_t)1 << 18);
-            QMX_HIP_CHECK(hipMalloc(reinterpret_cast<void **>(&dev), bytes));
-            QMX_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&host), bytes, hipHostMallocDefault));
-            used = false;
+        at ^= 1;
+        Host &h = host[at];
+        if (!h.ev) QMX_HIP_CHECK(hipEventCreateWithFlags(&h.ev, hipEventDisableTiming));
+        if (h.used) QMX_HIP_CHECK(hipEventSynchronize(h.ev));
+        if (need > h.bytes) {
+            if (h.p) QMX_HIP_CHECK(hipHostFree(h.p));
+            h.bytes = std::max(need, (size_t)1 << 17);
+            QMX_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&h.p), h.bytes, hipHostMallocDefault));
+            h.used = false;
         }
-        if (used) QMX_HIP_CHECK(hipEventSynchronize(ev));
-        return host;
+        return h.p;
     }
-    void commit(size_t n) {
-        QMX_HIP_CHECK(hipMemcpyAsync(dev, host, n, hipMemcpyHostToDevice, hstream()));
-        QMX_HIP_CHECK(hipEventRecord(ev, hstream()));
-        used = true;
+    // after the launch that reads the host buffer
+    void launched() {
+        QMX_HIP_CHECK(hipEventRecord(host[at].ev, hstream()));
+        host[at].used = true;
     }
     char *fragRoom(int blocks) {
         if (blocks > fragBlocks) {
             if (frags) devFree(frags);
             fragBlocks = std::max(blocks, 32);
-            frags = static_cast<char *>(devAlloc((size_t)fragBlocks * kBlockBytes));
+            frags = static_cast<char *>(devAlloc((size_t)fragBlocks * (kBlockBytes + sizeof(BlockDev))));
         }
         return frags;
     }
+    BlockDev *blocks() const { return reinterpret_cast<BlockDev *>(frags + (size_t)fragBlocks * kBlockBytes); }
 } g_ws;
 
 }  // namespace
@@ -815,7 +831,7 @@ struct Workspace {
 struct SweepProgram {
     int prec;
     char *upload = nullptr, *frags = nullptr;
-    const BlockDev *blocks = nullptr;
+    BlockDev *blocks = nullptr;
 };
 
 SweepProgram *sweepProgramCreate(int prec, const SweepPlan &plan, const FlatGate *gates) {
@@ -829,9 +845,9 @@ SweepProgram *sweepProgramCreate(int prec, const SweepPlan &plan, const FlatGate
     fillBlocks(prec, plan, 0, (int)plan.sweeps.size(), 0, u, host.data());
     p->upload = static_cast<char *>(devAlloc(u.bytes));
     hostToDevice(p->upload, host.data(), u.bytes);
-    p->frags = static_cast<char *>(devAlloc((size_t)n * kBlockBytes));
-    p->blocks = reinterpret_cast<const BlockDev *>(p->upload + u.blocks);
-    launchBuild(prec, n, u, p->upload, p->frags);
+    p->frags = static_cast<char *>(devAlloc((size_t)n * (kBlockBytes + sizeof(BlockDev))));
+    p->blocks = reinterpret_cast<BlockDev *>(p->frags + (size_t)n * kBlockBytes);
+    launchBuild(prec, n, u, p->upload, p->frags, p->blocks);
     return p;
 }
 
@@ -872,10 +888,9 @@ void sweepRunOnce(QuregDev *q, const SweepPlan &plan, const FlatGate *gates) {
         fillBuild(plan, gates, firstBlock, n, u, host);
         fillBlocks(q->prec, plan, first, last, firstBlock, u, host);
         char *frags = g_ws.fragRoom(n);
-        g_ws.commit(u.bytes);
-        launchBuild(q->prec, n, u, g_ws.dev, frags);
-        runSweeps(q, plan, gates, first, last, firstBlock, reinterpret_cast<const BlockDev *>(g_ws.dev + u.blocks),
-                  frags);
+        launchBuild(q->prec, n, u, host, frags, g_ws.blocks());
+        g_ws.launched();
+        runSweeps(q, plan, gates, first, last, firstBlock, g_ws.blocks(), frags);
         first = last;
     }
 }
@@ -944,8 +959,6 @@ void smallCircuit(QuregDev *q, const FlatGate *gates, int count) {
                 d.u[2 * e + 1] = f.u[e].im;
             }
         }
-        g_ws.commit((size_t)num * sizeof(SmallGate));
-        const SmallGate *dg = reinterpret_cast<const SmallGate *>(g_ws.dev);
         QMX_DISPATCH(q->prec, T, {
             static bool ldsAllowed = false;
             if (!ldsAllowed) {
@@ -955,10 +968,11 @@ void smallCircuit(QuregDev *q, const FlatGate *gates, int count) {
                     std::abort();
                 ldsAllowed = true;
             }
-            hipLaunchKernelGGL(kSmallCircuit<T>, dim3(1), dim3(threads), lds, hstream(), (Amp<T> *)q->amps, n, dg,
+            hipLaunchKernelGGL(kSmallCircuit<T>, dim3(1), dim3(threads), lds, hstream(), (Amp<T> *)q->amps, n, h,
                                num);
         });
         checkLaunch("smallCircuit");
+        g_ws.launched();
     }
 }
 
