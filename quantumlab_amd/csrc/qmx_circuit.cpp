@@ -289,6 +289,32 @@ bool channelGate(int code, int q, int n, double p, FlatGate &g) {
     }
 }
 
+bool lone1(const FlatGate &g) { return (g.kind == FlatGate::MATRIX2 || g.kind == FlatGate::NOT) && !g.ctrl; }
+
+// gate b after gate a, both on the same one qubit, as one
+void joinGate(FlatGate &a, const FlatGate &b) {
+    static const Cplx swap[4] = {{0, 0}, {1, 0}, {1, 0}, {0, 0}};
+    Cplx x[4], y[4];
+    std::copy(b.kind == FlatGate::NOT ? swap : b.u, (b.kind == FlatGate::NOT ? swap : b.u) + 4, x);
+    std::copy(a.kind == FlatGate::NOT ? swap : a.u, (a.kind == FlatGate::NOT ? swap : a.u) + 4, y);
+    a.kind = FlatGate::MATRIX2;
+    for (int r = 0; r < 2; ++r)
+        for (int c = 0; c < 2; ++c) a.u[2 * r + c] = cadd(cmul(x[2 * r], y[c]), cmul(x[2 * r + 1], y[2 + c]));
+}
+
+// Gate g at the end of `gates`, or inside the last one where that is the last to touch
+// its one qubit (last[qubit]: index of the last gate on it, -1 for none): in lists of
+// two one-qubit gates to each two-qubit one, a third of the gates go that way (10
+// qubits FP32, 80 gates: 53 steps of the LDS kernel, 62 -> 49 us with the reads).
+void appendGate(std::vector<FlatGate> &gates, int *last, const FlatGate &g) {
+    if (lone1(g) && last[g.target] >= 0 && lone1(gates[last[g.target]])) {
+        joinGate(gates[last[g.target]], g);
+        return;
+    }
+    for (uint64_t m = g.mask(); m; m &= m - 1) last[__builtin_ctzll(m)] = (int)gates.size();
+    gates.push_back(g);
+}
+
 // channel b after channel a on the same qubit, as one
 void joinChannel(FlatGate &a, const FlatGate &b) {
     const double f = a.u[0].re, s = a.u[0].im;
@@ -555,7 +581,7 @@ GateList gateList(const qmxCircuit *c, int numOps, bool everyOp) {
 struct DensityList {
     int n;
     GateList l;
-    int last[64];               // per qubit: the last gate of the list that touches it
+    int last[64];               // per qubit: the last gate of the list on its row bit
     int operations = 0;
     explicit DensityList(int numQubits) : n(numQubits) { std::fill(last, last + 64, -1); }
     bool noise(int code, int q, double p) {
@@ -567,8 +593,7 @@ struct DensityList {
             joinChannel(l.gates[last[q]], g);
             return true;
         }
-        last[q] = (int)l.gates.size();
-        l.gates.push_back(g);
+        appendGate(l.gates, last, g);
         return true;
     }
     void gate(const FlatGate &g) {
@@ -577,9 +602,8 @@ struct DensityList {
         c.target += n;
         c.ctrl <<= n;
         for (Cplx &z : c.u) z.im = -z.im;
-        l.gates.push_back(g);
-        l.gates.push_back(c);
-        for (uint64_t m = g.mask(); m; m &= m - 1) last[__builtin_ctzll(m)] = (int)l.gates.size() - 1;
+        appendGate(l.gates, last, g);
+        appendGate(l.gates, last, c);
     }
     void stop(int op) {
         l.stops.push_back({(int)l.gates.size(), op});
@@ -1082,14 +1106,18 @@ qreal qmxApplyOperations(Qureg qureg, const qmxBasicOperation *ops, int numOps, 
     } else if (!qureg.isDensityMatrix && (small || sweeps)) {
         GateList l;
         l.gates.reserve(numOps);
+        int last[64];
+        std::fill(last, last + 64, -1);
         for (int i = 0; i < numOps; ++i) {
             const qmxBasicOperation &o = ops[i];
             checkBasic(c.shape, o.operation, o.qubits, o.numQubits, (double)o.param, __func__);
             FlatGate g;
-            if (!undispatched(o.operation) && basicGate(o.operation, o.qubits, (double)o.param, g))
-                l.gates.push_back(g);
-            else if (o.operation == QMX_OP_CC || (fuseQubits == 0 && undispatched(o.operation)))
+            if (!undispatched(o.operation) && basicGate(o.operation, o.qubits, (double)o.param, g)) {
+                appendGate(l.gates, last, g);
+            } else if (o.operation == QMX_OP_CC || (fuseQubits == 0 && undispatched(o.operation))) {
                 l.stops.push_back({(int)l.gates.size(), i});
+                std::fill(last, last + 64, -1);
+            }
         }
         if (fuseQubits < 0 || fuseQubits > 10) qv::raise(badFuse, __func__);
         if (small)
