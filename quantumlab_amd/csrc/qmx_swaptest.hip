@@ -352,18 +352,28 @@ __global__ void __launch_bounds__(kBlock) kCentroidUpdate(const double *__restri
     const size_t dim = (size_t)1 << maxQ;
     double *mag = reinterpret_cast<double *>(smem);
     double *cc = cent + (size_t)c * dim;
-    int mem = 0;
-    for (int k = 0; k < chunks; ++k) mem += members[k * C + c];
+    // whether the cluster has members: one load a lane, not a chain of them
+    const int lane = threadIdx.x & 63;
+    const bool mem = __ballot(lane < chunks && members[lane * C + c] > 0) != 0;
     Acc acc[1];
     for (int i = threadIdx.x; i < D; i += kBlock) {
         double sum = 0.0;
         int cnt = 0;
-        if (mem > 0) {
-#pragma unroll 4
-            for (int k = 0; k < chunks; ++k) {
+        if (mem) {
+            // all chunks' loads in flight, then the sum in order (4096 points, 16
+            // centroids up to 10 qubits: the kernel takes 16 us, 22 with four at a time)
+            double part[kMeanChunks];
+            int num[kMeanChunks];
+#pragma unroll
+            for (int k = 0; k < kMeanChunks; ++k) {
                 const size_t o = ((size_t)k * C + c) * dim + i;
-                sum += sums[o];
-                cnt += counts[o];
+                part[k] = sums[o];
+                num[k] = counts[o];
+            }
+#pragma unroll
+            for (int k = 0; k < kMeanChunks; ++k) {
+                sum += part[k];
+                cnt += num[k];
             }
         }
         double v;
