@@ -120,34 +120,50 @@ def run_fp64_per_gate(qe, n, steps, warmup, seed):
 
 
 def fused_bytes(qe, c, n, amp_bytes=8):
-    """Algorithmic HBM bytes of one application of a fused brick-circuit
-    period, and the number of full sweeps in it. A step of several gates
-    (padded to 5 qubits on registers of >= 9 qubits) or a lone 5-qubit gate
-    reads and writes the register once; a lone gate on fewer qubits runs its
-    per-gate kernel and moves what that moves: a one-qubit gate 2NB, a
-    controlledNot NB, the 3-control unitary 2NB/8."""
+    """Algorithmic HBM bytes of one application of a fused brick-circuit period, the
+    full sweeps in it and the matrix-core flops an amplitude: a sweep of blocks reads
+    and writes the register once, 96 flops an amplitude for a block of 4 qubits and 192
+    for one of 5 (three real products for a complex one). A lone gate runs its per-gate
+    kernel and moves what that moves: a one-qubit or 5-qubit gate 2NB, a controlledNot
+    NB, the 3-control unitary 2NB/8."""
     import ctypes as C
+    from quantumlab_amd.quest import QMX_PREC_FP32, QMX_PREC_FP64, qreal
     N = float(1 << n)
-    targs = (C.c_int * 64)()
-    total, sweeps = 0.0, 0
+    prec = QMX_PREC_FP32 if amp_bytes == 8 else QMX_PREC_FP64
+    targs, re, im = (C.c_int * 64)(), (qreal * 1024)(), (qreal * 1024)()
+    total, sweeps, flops, s = 0.0, 0, 0, 0
+    lone = {1: 2.0, 2: 1.0, 4: 0.25}
+    while True:
+        sizes = []
+        while (k := qe.qmxCircuitSweepBlock(c, prec, s, len(sizes), targs, re, im)) > 0:
+            sizes.append(k)
+            one = sum(re[i * ((1 << k) + 1)] == 1.0 for i in range(1 << k))
+        if not sizes:
+            break
+        s += 1
+        k = sizes[0]
+        # blocks have 4 or 5 qubits; a controlled 2x2 on 4 leaves 14 of the 16 as they are
+        if len(sizes) == 1 and (k < 4 or (k == 4 and one >= 14)):
+            total += lone.get(k, 2.0) * N * amp_bytes
+            continue
+        total += 2 * N * amp_bytes
+        sweeps += 1
+        flops += sum(96 if k == 4 else 192 for k in sizes)
+    if s:
+        return total, sweeps, flops
+    # other block sizes and small registers: a sweep a step
     for s in range(qe.qmxCircuitNumBlocks(c)):
         k = qe.qmxCircuitStep(c, s, targs, None, None)
-        if k >= 5 or k == 1:
-            total += 2 * N * amp_bytes
-            sweeps += k >= 5
-        elif k == 2:
-            total += N * amp_bytes
-        elif k == 4:
-            total += 2 * N * amp_bytes / 8
-        else:
-            total += 2 * N * amp_bytes
-    return total, sweeps
+        total += lone.get(k, 2.0) * N * amp_bytes
+        sweeps += k >= 5
+        flops += 192 * (k >= 5)
+    return total, sweeps, flops
 
 
 def run_fp32_fused(qe, n, plans, warmup, steps, k):
     """Fused periods on an n-qubit FP32 register: (register, wall time of the
     timed periods, their steps, the FP64 norm^2 before renormalising, their
-    algorithmic bytes, their full 5-qubit sweeps)."""
+    algorithmic bytes, their full sweeps, their matrix-core flops an amplitude)."""
     from quantumlab_amd import workloads as W
     from quantumlab_amd.quest import QMX_PREC_FP32
     q = qe.qureg(n, precision=QMX_PREC_FP32)
@@ -158,7 +174,7 @@ def run_fp32_fused(qe, n, plans, warmup, steps, k):
         circuits.append(c)
     blocks = sum(qe.qmxCircuitNumBlocks(c) for c in circuits[warmup:])
     moved = [fused_bytes(qe, c, n) for c in circuits[warmup:]]
-    nbytes, sweeps = sum(m[0] for m in moved), sum(m[1] for m in moved)
+    nbytes, sweeps, flops = (sum(m[i] for m in moved) for i in range(3))
     for s in range(warmup):
         qe.qmxCircuitApply(q, circuits[s], 1)
     qe.qmxSync()
@@ -172,7 +188,7 @@ def run_fp32_fused(qe, n, plans, warmup, steps, k):
         qe.qmxCircuitDestroy(c)
     log(f"fp32 fused timed {steps} steps: wall {wall:.3f}s blocks {blocks} ({sweeps} full sweeps) "
         f"norm^2 before renorm {norm2:.12f}")
-    return q, wall, blocks, norm2, nbytes, sweeps
+    return q, wall, blocks, norm2, nbytes, sweeps, flops
 
 
 def run_fp32_large(qe, n, seed, k):
@@ -190,7 +206,7 @@ def run_fp32_large(qe, n, seed, k):
     c = W.build_circuit(qe, n, gates)
     qe.qmxCircuitFuse(c, k)
     blocks = qe.qmxCircuitNumBlocks(c)
-    nbytes, sweeps = fused_bytes(qe, c, n)
+    nbytes, sweeps, flops = fused_bytes(qe, c, n)
     qe.qmxSync()
     t0 = time.perf_counter()
     qe.qmxCircuitApply(q32, c, 1)
@@ -227,9 +243,9 @@ def run_fp32_large(qe, n, seed, k):
             "fp64_per_gate_gb_per_s": round(W.gate_bytes(gates, n, 16) / wall64 / 1e9, 1),
             "speedup_vs_fp64_per_gate": round(wall64 / wall, 3),
             "fidelity_error": float(1 - fid), "max_abs_amp_error": float(maxabs),
-            "roofline": {"bound": "hbm", "kernel": "kFused5Tile", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS,
+            "roofline": {"bound": "hbm", "kernel": "kTileSweep", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS,
                          "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None,
-                         "mfma_tflops": round(sweeps * N * 192 / wall / 1e12, 2)}}
+                         "mfma_tflops": round(flops * N / wall / 1e12, 2)}}
 
 
 # CPUs this process may use, read before any OpenMP runtime starts (with
@@ -848,8 +864,8 @@ def main():
                   "config": {"workload": "state-vector leg skipped (--steps 0 or --only)", "qubits": n}}
 
     if not args.no_fused and q64 is not None and not getattr(args, "fused_large_only", False):
-        q32, wall32, blocks, norm2, fbytes, fsweeps = run_fp32_fused(qe, n, plans, args.warmup, args.steps,
-                                                                     args.fuse_qubits)
+        q32, wall32, blocks, norm2, fbytes, fsweeps, fflops = run_fp32_fused(qe, n, plans, args.warmup, args.steps,
+                                                                             args.fuse_qubits)
         ip = qe.calcInnerProduct(q64, q32)
         # normalised fidelity: norms from FP64 reductions (the FP32-stored vector
         # re-rounds its norm^2 by ~1e-9 even right after renormalisation)
@@ -865,16 +881,16 @@ def main():
         fgbs = fbytes / wall32 / 1e9
         result["fused_fp32"]["full_sweeps_per_step"] = fsweeps / args.steps
         result["fused_fp32"]["roofline"] = {
-            "bound": "hbm", "kernel": "kFused5Tile (5-qubit blocks on LDS tiles, v_mfma_f32_16x16x4f32, "
-                                      "three real products per complex product)", "achieved": round(fgbs, 1),
+            "bound": "hbm", "kernel": "kTileSweep (sweeps of 4- and 5-qubit blocks on LDS tiles, "
+                                      "v_mfma_f32_16x16x4f32, three real products per complex product)", "achieved": round(fgbs, 1),
             "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(fgbs / HBM_PEAK_GBS, 4),
-            "traffic": profiled_traffic("fused32_fp32", "kFused5Tile", n)[0],
-            "traffic_source": profiled_traffic("fused32_fp32", "kFused5Tile", n)[1],
-            "bytes_per_block": 2.0 * N * 8,
-            "mfma_tflops": round(fsweeps * N * 192 / wall32 / 1e12, 2),
-            "note": "a block of several gates (padded to 5 qubits) reads and writes the FP32 register once, with "
-                    "192 MFMA flops per amplitude; a lone gate on fewer qubits runs its per-gate kernel and counts "
-                    "what that moves; over the fused steps' wall time (launch gaps included)"}
+            "traffic": profiled_traffic("fused32_fp32", "kTileSweep", n)[0],
+            "traffic_source": profiled_traffic("fused32_fp32", "kTileSweep", n)[1],
+            "bytes_per_sweep": 2.0 * N * 8,
+            "mfma_tflops": round(fflops * N / wall32 / 1e12, 2),
+            "note": "a sweep reads and writes the FP32 register once for all its blocks, with 96 (4 qubits) or 192 "
+                    "(5) MFMA flops per amplitude and block; a lone gate runs its per-gate kernel and counts what "
+                    "that moves; over the fused steps' wall time (launch gaps included)"}
         log(f"fused fp32: {wall / wall32:.2f}x vs fp64 per-gate, 1-F={1 - fid:.3e}, max|da|={maxabs:.3e}")
         qe.destroy(q32)
     if q64 is not None:
@@ -886,8 +902,8 @@ def main():
         result["stream"] = run_stream(qe, n)
     if args.only == "fused-kernel":
         plans = [period_gates(n, s, args.seed) for s in range(args.warmup + args.fused_steps)]
-        q32, wall32, blocks, _, fbytes, fsweeps = run_fp32_fused(qe, n, plans, args.warmup, args.fused_steps,
-                                                                 args.fuse_qubits)
+        q32, wall32, blocks, _, fbytes, fsweeps, _ = run_fp32_fused(qe, n, plans, args.warmup, args.fused_steps,
+                                                                    args.fuse_qubits)
         qe.destroy(q32)
         gbs = fbytes / wall32 / 1e9
         result["fused_kernel"] = {"qubits": n, "periods": args.fused_steps, "blocks": blocks,

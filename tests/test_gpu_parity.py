@@ -538,6 +538,36 @@ def test_trotter_many_large_angle_rotations_fp32(gpu, cpuref, density, n, with_x
     assert np.max(np.abs(outs[0] - outs[1])) < 2e-5
 
 
+@pytest.mark.parametrize("n,precision", [(11, None), (12, None), (14, None), (12, QMX_PREC_FP32),
+                                         (13, QMX_PREC_FP32), (14, QMX_PREC_FP32)])
+@pytest.mark.parametrize("scale", [0.1, 2.0])
+def test_trotter_strings_of_every_sign_form(gpu, cpuref, n, precision, scale):
+    """Random X/Y/Z strings of one to four qubits on registers of one tile and a few: the
+    masks and signs of every form of a rotation in full tiles, at angles of the
+    tangent form (scale 0.1) and with large ones of the plain form among them."""
+    rng = np.random.default_rng(n)
+    T = 70
+    codes = np.zeros((T, n), dtype=np.int32)
+    for row in codes:
+        qs = rng.choice(n, size=int(rng.integers(1, 5)), replace=False)
+        row[qs] = rng.integers(1, 4, size=len(qs))
+    coeffs = scale * rng.standard_normal(T)
+    outs = []
+    for lib, prec in ((gpu, precision), (cpuref, None)):
+        q = lib.qureg(n, precision=prec) if prec is not None else lib.qureg(n)
+        for j in range(n):
+            lib.lib.rotateY(q, j, 0.3 + 0.1 * j)
+            lib.lib.rotateZ(q, j, 0.2 + 0.3 * j)
+        h = lib.hamil(coeffs, codes)
+        lib.call("applyTrotterCircuit", q, h, 1.0, 2, 2)
+        lib.lib.destroyPauliHamil(h)
+        outs.append(lib.state(q))
+        lib.destroy(q)
+    # 4 x 70 rotations, each unitary: a few ulps of an amplitude (at most 1) each
+    tol = 1e-12 if precision is None else 2.0 ** -22 * np.sqrt(4 * T)
+    assert np.max(np.abs(outs[0] - outs[1])) < tol
+
+
 @pytest.mark.parametrize("density,n", [(False, 3), (False, 7), (False, 13), (True, 3), (True, 6)])
 def test_prob_of_all_outcomes_matches_oracle(gpu, cpuref, density, n):
     """Subsets of every size and order, low and high qubits, one pass each."""
