@@ -13,7 +13,8 @@ namespace qmx {
 // conjugate one on its column bits. CHANNEL is a one-qubit channel with real maps of
 // its qubit's diagonal entries, (x00, x11) -> (d00 x00 + d01 x11, d10 x00 + d11 x11),
 // and off-diagonal ones, (x01, x10) -> (f x01 + g x10, g x01 + f x10): target = the
-// row bit, k = the column bit, u = {(f, g), (d00, d01), (d10, d11), unused}.
+// row bit, k = the column bit, u = {(f, g), (d00, d01), (d10, d11), (fLo, d00Lo)}, lo =
+// d11Lo: what rounding f, d00 and d11 left over, where channels were joined into one.
 struct FlatGate {
     enum Kind { MATRIX2 = 0, NOT = 1, MATRIXN = 2, CHANNEL = 3 };
     int kind = MATRIX2;
@@ -23,6 +24,7 @@ struct FlatGate {
     int k = 0;                     // MATRIXN: targets (targs[0] = least significant bit), 2^k x 2^k
     const int *targs = nullptr;
     const Cplx *uN = nullptr;
+    float lo = 0;                  // CHANNEL
     uint64_t mask() const {
         uint64_t m = ctrl;
         if (kind == MATRIXN)

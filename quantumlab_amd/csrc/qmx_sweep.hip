@@ -65,8 +65,9 @@ struct GateDev {
     unsigned ctrl;       // controls, bits of the block's index
     int k;               // MATRIXN
     int mat;             // MATRIXN: its matrix (entry offset)
-    int pad[3];
-    alignas(16) double u[8];  // the matrix, (re, im) by rows; CHANNEL: f, g, d00, d01, d10, d11
+    float lo;            // CHANNEL: d11Lo
+    int pad[2];
+    alignas(16) double u[8];  // the matrix, (re, im) by rows; CHANNEL: f, g, d00, d01, d10, d11, fLo, d00Lo
 };
 
 // gates staged in LDS at a time (whole coalesced loads; one entry more is read)
@@ -103,6 +104,12 @@ __device__ __forceinline__ GateDev uniformGate(const GateDev &g) {
 __device__ __forceinline__ Amp<double> rowTimes(double a, double b, double c, double d, const Amp<double> &p,
                                                 const Amp<double> &q) {
     return Amp<double>{a * p.x - b * p.y + c * q.x - d * q.y, a * p.y + b * p.x + c * q.y + d * q.x};
+}
+// (a + aLo) p + b q, b small beside a where aLo counts; the low part goes in before the
+// sum is rounded to the size of a p, beside which it would be lost
+__device__ __forceinline__ Amp<double> realTimes(double a, double aLo, double b, const Amp<double> &p,
+                                                 const Amp<double> &q) {
+    return Amp<double>{fma(a, p.x, fma(b, q.x, aLo * p.x)), fma(a, p.y, fma(b, q.y, aLo * p.y))};
 }
 // what a tile sweep needs of a block besides its vectors
 struct BlockDev {
@@ -174,10 +181,10 @@ __global__ void __launch_bounds__(kBlock) kBuildBlocks(const BuildDev *__restric
                 Amp<double> *p00 = M + (r << k) + col, *p11 = p00 + ((b0 | b1) << k);
                 Amp<double> *p01 = p00 + (b0 << k), *p10 = p00 + (b1 << k);
                 const Amp<double> x = *p00, y = *p11, v = *p01, w = *p10;
-                *p00 = Amp<double>{G.u[2] * x.x + G.u[3] * y.x, G.u[2] * x.y + G.u[3] * y.y};
-                *p11 = Amp<double>{G.u[4] * x.x + G.u[5] * y.x, G.u[4] * x.y + G.u[5] * y.y};
-                *p01 = Amp<double>{G.u[0] * v.x + G.u[1] * w.x, G.u[0] * v.y + G.u[1] * w.y};
-                *p10 = Amp<double>{G.u[1] * v.x + G.u[0] * w.x, G.u[1] * v.y + G.u[0] * w.y};
+                *p00 = realTimes(G.u[2], G.u[7], G.u[3], x, y);
+                *p11 = realTimes(G.u[5], G.lo, G.u[4], y, x);
+                *p01 = realTimes(G.u[0], G.u[6], G.u[1], v, w);
+                *p10 = realTimes(G.u[0], G.u[6], G.u[1], w, v);
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
@@ -494,8 +501,8 @@ struct SmallGate {
     unsigned what;               // SG_*
     unsigned bit;                // the target's bit, as a byte offset of the LDS register (16 B an amplitude)
     unsigned ctrl;               // the controls' bits, likewise; SG_CHANNEL: the column bit
-    unsigned pad;
-    alignas(16) double u[8];     // the matrix, (re, im) by rows
+    float lo;                    // SG_CHANNEL: d11Lo
+    alignas(16) double u[8];     // the matrix, (re, im) by rows; SG_CHANNEL: f, g, d00, d01, d10, d11, fLo, d00Lo
 };
 enum { SG_GENERAL = 0, SG_NOT = 1, SG_PHASE = 2, SG_REAL = 3, SG_CHANNEL = 4 };  // SG_PHASE: diag(1, u)
 constexpr int kSmallStage = 256;
@@ -521,6 +528,7 @@ __global__ void __launch_bounds__(kSmallThreads) kSmallCircuit(Amp<T> *__restric
         }
         const unsigned what = uniform(nextHead.x), bit = uniform(nextHead.y), ctrl = uniform(nextHead.z);
         const unsigned high = ~(bit - 1u);
+        const double lo11 = __uint_as_float(nextHead.w);
         const d8 u = nextU;
         // past a stage's last one: unused
         nextHead = *reinterpret_cast<const uint4 *>(stage + g % kSmallStage + 1);
@@ -532,10 +540,10 @@ __global__ void __launch_bounds__(kSmallThreads) kSmallCircuit(Amp<T> *__restric
                 i += i & hi;
                 Amp<double> &A = at(i), &B = at(i + bit), &C = at(i + ctrl), &D = at(i + bit + ctrl);
                 const Amp<double> x = A, y = D, v = B, z = C;
-                A = Amp<double>{u[2] * x.x + u[3] * y.x, u[2] * x.y + u[3] * y.y};
-                D = Amp<double>{u[4] * x.x + u[5] * y.x, u[4] * x.y + u[5] * y.y};
-                B = Amp<double>{u[0] * v.x + u[1] * z.x, u[0] * v.y + u[1] * z.y};
-                C = Amp<double>{u[1] * v.x + u[0] * z.x, u[1] * v.y + u[0] * z.y};
+                A = realTimes(u[2], u[7], u[3], x, y);
+                D = realTimes(u[5], lo11, u[4], y, x);
+                B = realTimes(u[0], u[6], u[1], v, z);
+                C = realTimes(u[0], u[6], u[1], z, v);
             }
             __syncthreads();
             continue;
@@ -641,6 +649,7 @@ void fillBuild(const SweepPlan &plan, const FlatGate *gates, int firstBlock, int
                     d.u[2 * e] = f.u[e].re;
                     d.u[2 * e + 1] = f.u[e].im;
                 }
+                d.lo = f.lo;
             } else {
                 d.t = (unsigned)local(f.target);
                 for (int e = 0; e < 4; ++e) {
@@ -953,7 +962,7 @@ void smallCircuit(QuregDev *q, const FlatGate *gates, int count) {
             d.what = (unsigned)smallKind(f);
             d.bit = 16u << f.target;
             d.ctrl = f.kind == FlatGate::CHANNEL ? 16u << f.k : 16u * (unsigned)f.ctrl;
-            d.pad = 0;
+            d.lo = f.lo;
             for (int e = 0; e < 4; ++e) {
                 d.u[2 * e] = f.u[e].re;
                 d.u[2 * e + 1] = f.u[e].im;
