@@ -131,7 +131,9 @@ long long qmxLoadStateCSV(Qureg qureg, const char *path);
  * unfused, each operation is the QuEST call that loop makes; fused (state
  * vectors), the unitaries between collapses run as dense blocks of at most k
  * qubits, several blocks to a sweep where k is 5. State vectors of at most 12
- * qubits take either form gate by gate, in one launch. */
+ * qubits stay in one compute unit's memory between collapses and gates too wide
+ * for it: fused circuits in blocks of 4 and 5 qubits whatever k is, unfused ones
+ * and lists applied once (qmxApplyOperations) gate by gate. */
 typedef struct qmxCircuit qmxCircuit;
 
 /* QuantumLab's basic operations: the codes of EBasicOperation
@@ -193,7 +195,7 @@ int qmxCircuitNumBlocks(const qmxCircuit *c);
  * matrix index) and its 2^k x 2^k matrix (row-major; any pointer may be NULL),
  * returning k; 0 for a collapse; -1 past the end. */
 int qmxCircuitStep(const qmxCircuit *c, int step, int *targs, qreal *re, qreal *im);
-/* How a circuit fused into blocks of 5 runs on registers of more than 12 qubits:
+/* How a circuit fused into blocks of 5 (registers of at most 12 qubits: of any size) runs:
  * sweep `sweep` (one read and write of a register of this storage precision)
  * applies its blocks of 4 or 5 qubits one after another; a gate that shares its
  * sweep with no other is one block of its own qubits (targets and controls). Gives

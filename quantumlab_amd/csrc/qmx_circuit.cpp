@@ -20,8 +20,9 @@
 // qubits on registers of more than 12 qubits share sweeps (qmx_plan.cpp plans
 // them, qmx_sweep.hip builds and applies them: many gates to a read and write of
 // the register); other block sizes take one sweep a block (qmx::applyMatrixN).
-// State vectors of at most 12 qubits take every list, fused or not, gate by gate
-// in one workgroup's LDS, one launch for the list. On density registers, fused
+// State vectors of at most 12 qubits lie in one workgroup's LDS: a fused circuit
+// runs there in blocks of 4 and 5 qubits, a list applied once or unfused gate by
+// gate, in one launch between collapses and gates too wide for it. On density registers, fused
 // application is the unfused sequence: a recorded circuit's operations are the QuEST
 // calls, which compose into superoperator sweeps two qubits at a time, and
 // qmxApplyOperations plans its list as gates on the row and column bits.
@@ -696,12 +697,12 @@ void runSmall(qmx::QuregDev *d, const GateList &l, F stop) {
 }
 
 // sweeps for the list's gates, segment by segment: no sweep crosses a stop
-void planList(int numQubits, int prec, const GateList &l, qmx::SweepPlan &plan,
+void planList(const qmx::SweepShape &shape, const GateList &l, qmx::SweepPlan &plan,
               std::vector<std::pair<int, int>> &stops) {
     int i = 0;
     for (size_t s = 0; s <= l.stops.size(); ++s) {
         const int until = s < l.stops.size() ? l.stops[s].first : (int)l.gates.size();
-        if (until > i) qmx::planSweeps(qmx::sweepShape(numQubits, prec, false), l.gates.data() + i, until - i, i, plan);
+        if (until > i) qmx::planSweeps(shape, l.gates.data() + i, until - i, i, plan);
         i = until;
         if (s < l.stops.size()) stops.push_back({(int)plan.sweeps.size(), l.stops[s].second});
     }
@@ -725,13 +726,25 @@ void runSweepsOnce(qmx::QuregDev *d, const GateList &l, F stop) {
     }
 }
 
+// The fused circuit's sweeps; nullptr where it does not run in sweeps. Small registers
+// have one plan for both precisions, whatever the blocks' size: at 9 to 12 qubits and
+// 20 brick layers it takes 19, 26, 35 and 63 us, where blocks of 5 at a launch each took
+// 64, 104, 81 and 96 (FP32) or 780, 1070, 190 and 256 (FP64) and the gates one by one
+// 123, 159, 221 and 347; 4 gates on 4 qubits 4 us, 10 one by one. A gate too wide for a
+// block is a launch of its own there (4 to 9 us) and a step of 0.3 to 0.9 us one by one:
+// a plan that cuts the list for fewer than 16 gates a launch is not taken.
 CircuitSweeps *sweepsOf(qmxCircuit *c, int prec) {
-    CircuitSweeps *&s = c->sweeps[prec];
+    const bool small = c->numQubits <= qmx::kSmallCircuitQubits;
+    if (c->blocks.empty() || (!small && c->fusedQubits != qmx::kSweepBlockQubits)) return nullptr;
+    CircuitSweeps *&s = c->sweeps[small ? qmx::FP64 : prec];
     if (!s) {
         s = new CircuitSweeps;
         s->list = gateList(c, c->fusedOps, false);
-        planList(c->numQubits, prec, s->list, s->plan, s->stops);
+        planList(small ? qmx::smallShape(c->numQubits) : qmx::sweepShape(c->numQubits, prec, false), s->list, s->plan,
+                 s->stops);
     }
+    const int cuts = (int)s->plan.sweeps.size() - (int)s->list.stops.size() - 1;
+    if (small && cuts > 0 && 16 * cuts > (int)s->list.gates.size()) return nullptr;
     return s;
 }
 
@@ -740,7 +753,20 @@ double applyCircuit(const Qureg &q, qmxCircuit *c, int fused) {
     const bool noisy = q.isDensityMatrix && hasNoise(c->noise);
     qmx::QuregDev *d = qmx::dev(q);
     const bool asBlocks = fused && !c->blocks.empty() && !q.isDensityMatrix;
-    if (!q.isDensityMatrix && qmx::smallCircuitSupported(d)) {
+    if (CircuitSweeps *s = asBlocks ? sweepsOf(c, d->prec) : nullptr) {
+        if (!s->program)
+            s->program = qmx::sweepProgramCreate(qmx::smallStateVector(d) ? qmx::FP64 : d->prec, s->plan,
+                                                 s->list.gates.data());
+        int at = 0;
+        for (size_t i = 0; i <= s->stops.size(); ++i) {
+            const int until = i < s->stops.size() ? s->stops[i].first : (int)s->plan.sweeps.size();
+            qmx::sweepProgramRun(d, s->program, s->plan, s->list.gates.data(), at, until);
+            at = until;
+            if (i < s->stops.size()) prob *= runOp(q, c->ops[s->stops[i].second]);
+        }
+        return prob;
+    }
+    if (qmx::smallStateVector(d)) {
         runSmall(d, asBlocks ? gateList(c, c->fusedOps, false) : gateList(c, (int)c->ops.size(), true),
                  [&](int op) { prob *= runOp(q, c->ops[op]); });
         return prob;
@@ -749,18 +775,6 @@ double applyCircuit(const Qureg &q, qmxCircuit *c, int fused) {
         for (Op &o : c->ops) {
             prob *= runOp(q, o);
             if (noisy) noiseAfterGate(q, o, c->noise);
-        }
-        return prob;
-    }
-    if (c->fusedQubits == qmx::kSweepBlockQubits && qmx::sweepSupported(d->numQubits)) {
-        CircuitSweeps *s = sweepsOf(c, d->prec);
-        if (!s->program) s->program = qmx::sweepProgramCreate(d->prec, s->plan, s->list.gates.data());
-        int at = 0;
-        for (size_t i = 0; i <= s->stops.size(); ++i) {
-            const int until = i < s->stops.size() ? s->stops[i].first : (int)s->plan.sweeps.size();
-            qmx::sweepProgramRun(d, s->program, s->plan, s->list.gates.data(), at, until);
-            at = until;
-            if (i < s->stops.size()) prob *= runOp(q, c->ops[s->stops[i].second]);
         }
         return prob;
     }
@@ -1055,10 +1069,9 @@ int qmxCircuitStep(const qmxCircuit *c, int step, int *targs, qreal *re, qreal *
 
 int qmxCircuitSweepBlock(qmxCircuit *c, int precision, int sweep, int block, int *targs, qreal *re, qreal *im) {
     CIRCUIT_TRY
-    if (c->blocks.empty() || c->fusedQubits != qmx::kSweepBlockQubits || !qmx::sweepSupported(c->numQubits) ||
-        (precision != QMX_PREC_FP64 && precision != QMX_PREC_FP32))
-        return -1;
+    if (precision != QMX_PREC_FP64 && precision != QMX_PREC_FP32) return -1;
     const CircuitSweeps *s = sweepsOf(c, precision == QMX_PREC_FP64 ? qmx::FP64 : qmx::FP32);
+    if (!s) return -1;
     if (sweep < 0 || sweep >= (int)s->plan.sweeps.size()) return -1;
     const qmx::Sweep &w = s->plan.sweeps[sweep];
     if (block < 0 || block >= (w.lone >= 0 ? 1 : w.numBlocks)) return 0;
@@ -1069,7 +1082,8 @@ int qmxCircuitSweepBlock(qmxCircuit *c, int precision, int sweep, int block, int
     } else {
         const qmx::SweepBlock &sb = s->plan.blocks[w.firstBlock + block];
         for (int g = 0; g < sb.numGates; ++g) b.gates.push_back(s->list.op[s->plan.order[sb.firstGate + g]]);
-        for (int j = 0; j < sb.k; ++j) b.mask |= 1ull << sb.targs[j];
+        for (int j = 0; j < sb.k; ++j)
+            if (sb.targs[j] < c->numQubits) b.mask |= 1ull << sb.targs[j];
     }
     buildBlockMatrix(*c, b);
     const int k = (int)b.targs.size();

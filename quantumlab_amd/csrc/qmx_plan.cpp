@@ -226,9 +226,10 @@ void planSweeps(const SweepShape &shape, const FlatGate *gates, int count, int b
             int j = 0;
             for (uint64_t x = m; x; x &= x - 1) b.targs[j++] = __builtin_ctzll(x);
         }
-        for (int b = firstBlock; b < (int)plan.blocks.size(); b += kSweepMaxBlocks)
-            plan.sweeps.push_back(
-                Sweep{fromOrder(shape, tile), b, std::min(kSweepMaxBlocks, (int)plan.blocks.size() - b), -1});
+        for (int b = firstBlock, n = 0; b < (int)plan.blocks.size(); b += n) {
+            n = std::min(shape.maxBlocks, (int)plan.blocks.size() - b);
+            plan.sweeps.push_back(Sweep{fromOrder(shape, tile), b, n, -1});
+        }
     }
 }
 

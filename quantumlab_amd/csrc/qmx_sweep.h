@@ -74,10 +74,12 @@ struct SweepPlan {
 struct SweepShape {
     int bits, lowBits, tileBits;
     bool density;
+    int maxBlocks;                     // of one sweep
 };
 inline SweepShape sweepShape(int numBits, int prec, bool density) {
     // density tiles: a qubit is two bits, so 12 hold twice the pairs of 8
-    return SweepShape{numBits, sweepLowBits(prec), density ? kSweepTileBits : sweepTileBits(numBits), density};
+    return SweepShape{numBits, sweepLowBits(prec), density ? kSweepTileBits : sweepTileBits(numBits), density,
+                      kSweepMaxBlocks};
 }
 // Appends the sweeps of gates[0 .. count) to `plan` (gate indices offset by `base`).
 void planSweeps(const SweepShape &shape, const FlatGate *gates, int count, int base, SweepPlan &plan);
@@ -96,6 +98,16 @@ void sweepRunOnce(QuregDev *q, const SweepPlan &plan, const FlatGate *gates);
 void applyFlatGate(QuregDev *q, const FlatGate &g);
 
 // ---- small registers: the whole register in one workgroup's LDS -----------------
+// A state vector of at most kSmallCircuitQubits is one tile, of at least 9 bits (16
+// groups of a 5-qubit block; bits past the register are zeros), in FP64 for both
+// storage precisions; sweeps of any number of blocks.
+inline SweepShape smallShape(int numQubits) {
+    const int bits = numQubits < 9 ? 9 : numQubits;
+    return SweepShape{bits, sweepLowBits(FP64), bits, false, 1 << 30};
+}
+inline bool smallStateVector(const QuregDev *q) { return !q->isDensity && q->numQubits <= kSmallCircuitQubits; }
+
+// Gate lists applied once run gate by gate.
 // A density operation is three or four steps of the LDS kernel (rows, columns,
 // channels; 0.8 us each), where a tile of 12 bits takes whole blocks of them: 6
 // qubits, 82 operations with their noise and reads, FP64 379 us there and 216 in

@@ -306,6 +306,10 @@ __device__ __forceinline__ f4 mfma(float a, float b, f4 c) {
 __device__ __forceinline__ d4 mfma(double a, double b, d4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
+// waves of a small register's workgroup: one chunk of a 4-qubit block each, two at 12
+// bits (16 waves would leave a lane 128 registers, and two a SIMD keep it busy)
+constexpr int smallWaves(int tileBits) { return tileBits >= 11 ? 8 : 1 << (tileBits - 8); }
+
 template <typename T> struct Acc4;
 template <> struct Acc4<float> { typedef f4 type; };
 template <> struct Acc4<double> { typedef d4 type; };
@@ -316,8 +320,8 @@ template <typename T, int K, int WAVES, int TB>
 __device__ __forceinline__ void blockChunks(char *tile, const typename Frag<T>::V *v, const BlockDev &B, int wave) {
     typedef typename Acc4<T>::type A;
     constexpr int S = 1 << (K - 2), H = K == 5 ? 2 : 1, PV = 16 / sizeof(T), NV = H * S / PV, SV = S / 4;
-    constexpr int CH = (1 << (TB - 4 - K)) / WAVES, IL = K == 5 ? 1 : 2;
-    static_assert(CH % IL == 0, "every wave has whole runs of chunks");
+    constexpr int CH = (1 << (TB - 4 - K)) / WAVES, IL = K == 5 || CH < 2 ? 1 : 2;
+    static_assert(CH > 0 && CH % IL == 0, "every wave has whole runs of chunks");
     unsigned slot[S];
 #pragma unroll
     for (int i = 0; i < SV; ++i) {
@@ -411,6 +415,42 @@ __device__ __forceinline__ void blockChunks(char *tile, const typename Frag<T>::
     }
 }
 
+// The blocks on a tile in LDS, one after another; a barrier behind each.
+template <typename T, int WAVES, int TB>
+__device__ __forceinline__ void tileBlocks(char *tile, const BlockDev *__restrict__ blocks, int numBlocks,
+                                           const char *__restrict__ frags, int lane, int wave) {
+    typedef typename Frag<T>::V V;
+    // a 4-qubit block's vectors are loaded while the block before it multiplies
+    constexpr int V4 = blockVecs<T>(4), V5 = blockVecs<T>(5);
+    // waves of a 5-qubit block: small tiles have fewer chunks of it than waves
+    constexpr int W5 = (1 << (TB - 9)) < WAVES ? 1 << (TB - 9) : WAVES;
+    const V *next = reinterpret_cast<const V *>(frags) + lane;
+    BlockDev B = blocks[0], nB = B;
+    V v[V5], pre[V4];
+#pragma unroll
+    for (int i = 0; i < V4; ++i) pre[i] = next[i * 64];
+    for (int b = 0; b < numBlocks; ++b) {
+        const V *mineB = next;
+        next += kBlockBytes / sizeof(V);
+#pragma unroll
+        for (int i = 0; i < V4; ++i) v[i] = pre[i];
+        if (b + 1 < numBlocks) {  // the same for the whole workgroup
+            nB = blocks[b + 1];
+#pragma unroll
+            for (int i = 0; i < V4; ++i) pre[i] = next[i * 64];
+        }
+        if (B.k == 5) {
+#pragma unroll
+            for (int i = V4; i < V5; ++i) v[i] = mineB[i * 64];
+            if (W5 == WAVES || wave < W5) blockChunks<T, 5, W5, TB>(tile, v, B, wave);
+        } else {
+            blockChunks<T, 4, WAVES, TB>(tile, v, B, wave);
+        }
+        B = nB;
+        __syncthreads();
+    }
+}
+
 template <typename T, bool NT, int WAVES, int TB>
 __global__ void __launch_bounds__(64 * WAVES, sizeof(T) == 4 ? 4 : 2)
     kTileSweep(Amp<T> *__restrict__ a, TileGeom geo, const BlockDev *__restrict__ blocks, int numBlocks,
@@ -443,33 +483,7 @@ __global__ void __launch_bounds__(64 * WAVES, sizeof(T) == 4 ? 4 : 2)
         }
     }
     __syncthreads();
-    // a 4-qubit block's vectors are loaded while the block before it multiplies
-    constexpr int V4 = blockVecs<T>(4), V5 = blockVecs<T>(5);
-    const V *next = reinterpret_cast<const V *>(frags) + lane;
-    BlockDev B = blocks[0], nB = B;
-    V v[V5], pre[V4];
-#pragma unroll
-    for (int i = 0; i < V4; ++i) pre[i] = next[i * 64];
-    for (int b = 0; b < numBlocks; ++b) {
-        const V *mineB = next;
-        next += kBlockBytes / sizeof(V);
-#pragma unroll
-        for (int i = 0; i < V4; ++i) v[i] = pre[i];
-        if (b + 1 < numBlocks) {  // the same for the whole workgroup
-            nB = blocks[b + 1];
-#pragma unroll
-            for (int i = 0; i < V4; ++i) pre[i] = next[i * 64];
-        }
-        if (B.k == 5) {
-#pragma unroll
-            for (int i = V4; i < V5; ++i) v[i] = mineB[i * 64];
-            blockChunks<T, 5, WAVES, TB>(tile, v, B, wave);
-        } else {
-            blockChunks<T, 4, WAVES, TB>(tile, v, B, wave);
-        }
-        B = nB;
-        __syncthreads();
-    }
+    tileBlocks<T, WAVES, TB>(tile, blocks, numBlocks, frags, lane, wave);
 #pragma unroll
     for (int j = 0; j < J; ++j) {
         V r;
@@ -574,6 +588,29 @@ __global__ void __launch_bounds__(kSmallThreads) kSmallCircuit(Amp<T> *__restric
     for (unsigned i = tid; i < dim; i += step) a[i] = Amp<T>{(T)at(16u * i).x, (T)at(16u * i).y};
 }
 
+// A planned list on a small register: the whole register is one workgroup's tile, in
+// FP64 for both storage precisions (FP32 results are rounded once: 1.4e-7 from the
+// 64-bit state after 400 gates on 12 qubits, 6.1e-7 with FP32 blocks). Up to 10 qubits a
+// 4-qubit block is one chain of LDS reads, 12 products and writes, 0.35 us; at 12 the
+// products of 16 chunks on one CU bound it, 1.1 us. A block stands for five or six gates.
+template <typename S, int TB>
+__global__ void __launch_bounds__(64 * smallWaves(TB)) kSmallBlocks(Amp<S> *__restrict__ a, int n,
+                                                                   const BlockDev *__restrict__ blocks, int numBlocks,
+                                                                   const char *__restrict__ frags) {
+    constexpr int WAVES = smallWaves(TB);
+    __shared__ __attribute__((aligned(16))) char tile[sizeof(Amp<double>) << TB];
+    const unsigned tid = threadIdx.x, dim = 1u << n;
+    auto at = [&](unsigned i) -> Amp<double> & {
+        return *reinterpret_cast<Amp<double> *>(tile + tileSlot<double>(i) * sizeof(Amp<double>));
+    };
+    for (unsigned i = tid; i < 1u << TB; i += 64 * WAVES)
+        at(i) = i < dim ? Amp<double>{(double)a[i].x, (double)a[i].y} : Amp<double>{0.0, 0.0};
+    __syncthreads();
+    tileBlocks<double, WAVES, TB>(tile, blocks, numBlocks, frags, tid & 63,
+                                  __builtin_amdgcn_readfirstlane((int)tid >> 6));
+    for (unsigned i = tid; i < dim; i += 64 * WAVES) a[i] = Amp<S>{(S)at(i).x, (S)at(i).y};
+}
+
 // ---- host side -----------------------------------------------------------------------
 size_t align16(size_t x) { return (x + 15) & ~(size_t)15; }
 
@@ -664,7 +701,7 @@ void fillBuild(const SweepPlan &plan, const FlatGate *gates, int firstBlock, int
 // the tile's qubits, ascending; returns how many
 int tilePositions(uint64_t tile, int pos[kMaxTB]) {
     const int bits = __builtin_popcountll(tile);
-    if (bits != kMaxTB && bits != kMaxTB - 1) {
+    if (bits > kMaxTB || bits < 9) {
         std::fprintf(stderr, "libquest_mi355x: a planned tile has %d qubits\n", bits);
         std::abort();
     }
@@ -774,17 +811,36 @@ void launchSweep(QuregDev *q, const Sweep &w, const BlockDev *blocks, const char
         launchTiles<T, false, 4, kSweepTileBits>(q, w, blocks, frags);
 }
 
+void launchSmallBlocks(QuregDev *q, const Sweep &w, const BlockDev *blocks, const char *frags) {
+    QMX_DISPATCH(q->prec, S, {
+        auto launch = [&](auto kernel, int tb) {
+            hipLaunchKernelGGL(kernel, dim3(1), dim3(64 * smallWaves(tb)), 0, hstream(), (Amp<S> *)q->amps,
+                               q->numQubits, blocks, w.numBlocks, frags);
+        };
+        switch (__builtin_popcountll(w.tile)) {
+            case 9: launch(kSmallBlocks<S, 9>, 9); break;
+            case 10: launch(kSmallBlocks<S, 10>, 10); break;
+            case 11: launch(kSmallBlocks<S, 11>, 11); break;
+            default: launch(kSmallBlocks<S, 12>, 12); break;
+        }
+    });
+    checkLaunch("small register's blocks");
+}
+
 void runSweeps(QuregDev *q, const SweepPlan &plan, const FlatGate *gates, int first, int last, int firstBlock,
                const BlockDev *blocks, const char *frags) {
     for (int s = first; s < last; ++s) {
         const Sweep &w = plan.sweeps[s];
+        const bool small = smallStateVector(q);
         if (w.lone >= 0) {
-            applyFlatGate(q, gates[w.lone]);
+            if (small && gates[w.lone].kind != FlatGate::MATRIXN) smallCircuit(q, gates + w.lone, 1);
+            else applyFlatGate(q, gates[w.lone]);
             continue;
         }
         const BlockDev *b = blocks + (w.firstBlock - firstBlock);
         const char *f = frags + (size_t)(w.firstBlock - firstBlock) * kBlockBytes;
-        QMX_DISPATCH(q->prec, T, { launchSweep<T>(q, w, b, f); });
+        if (small) launchSmallBlocks(q, w, b, f);
+        else QMX_DISPATCH(q->prec, T, { launchSweep<T>(q, w, b, f); });
     }
 }
 

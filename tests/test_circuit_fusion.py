@@ -285,3 +285,45 @@ def test_a_sweep_stays_in_its_tile(host, precision, low):
             at += k
     finally:
         host.lib.qmxCircuitDestroy(c)
+
+
+@pytest.mark.parametrize("n,k", [(1, 5), (2, 2), (4, 4), (5, 5), (8, 3), (8, 8), (9, 5), (10, 5), (12, 5)])
+def test_small_registers_run_fused_in_one_sweep(host, n, k):
+    """Up to 12 qubits, a fused circuit is one sweep of blocks that stand for four gates
+    each or more, and its operator is the gate list's; blocks name the register's own
+    qubits."""
+    gates = W.brick_circuit(n, 20, seed=n, extra_every=5 if n >= 6 else 0) if n > 1 else random_circuit(1, 40, 1)
+    c = W.build_circuit(host, n, gates)
+    try:
+        host.lib.qmxCircuitFuse(c, k)
+        blocks, counts = sweeps_of(host, c, Q.QMX_PREC_FP32)
+        assert len(counts) == 1 and 4 * counts[0] <= len(gates)
+        rng = np.random.default_rng(n)
+        psi = rng.standard_normal(1 << n) + 1j * rng.standard_normal(1 << n)
+        want, got = psi.copy(), psi.copy()
+        for g in gates:
+            qs, u = local_gate(g)
+            want = apply_local(want, n, qs, u)
+        for qs, u in blocks:
+            assert qs == sorted(set(qs)) and qs[-1] < n
+            got = apply_local(got, n, qs, u)
+        assert np.max(np.abs(got - want)) < 1e-11 * np.max(np.abs(want))
+    finally:
+        host.lib.qmxCircuitDestroy(c)
+
+
+def test_wide_gates_leave_a_small_register_gate_by_gate(host):
+    """A gate too wide for a block cuts the sweep: a few of them among hundreds do, one
+    to every eight gates leaves the list without sweeps."""
+    rng = np.random.default_rng(3)
+    for every, planned in ((100, True), (8, False)):
+        gates = W.brick_circuit(9, 20, seed=2)
+        for i in range(every, len(gates), every):
+            gates.insert(i, ("mcu", [0, 2, 4, 6, 8], 5, W.haar_unitary(rng, 2)))
+        c = W.build_circuit(host, 9, gates)
+        try:
+            host.lib.qmxCircuitFuse(c, 5)
+            _, counts = sweeps_of(host, c, Q.QMX_PREC_FP64)
+            assert (len(counts) > 1) == planned
+        finally:
+            host.lib.qmxCircuitDestroy(c)

@@ -441,3 +441,45 @@ def test_repeated_noise_does_not_drift(gpu, n):
         v[:, 0, :, 1], v[:, 1, :, 0] = f * x01, f * x10
     err = float(np.sqrt(np.sum(np.abs(got - rho) ** 2) / np.sum(np.abs(rho) ** 2)))
     assert err < 4 * 2.0 ** -53 * np.sqrt(len(ops))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 8, 9, 10, 11, 12])
+@pytest.mark.parametrize("precision", [None, QMX_PREC_FP32])
+def test_small_registers_in_blocks(gpu, cpuref, n, precision):
+    """Fused circuits on registers of one workgroup's LDS: 4-qubit blocks, 5-qubit ones
+    (of which tiles of 9 to 11 bits have fewer chunks than waves), more than 64 in a
+    sweep, collapses and a gate too wide for a block between sweeps; applied twice."""
+    rng = np.random.default_rng(50 + n)
+    gates = W.brick_circuit(n, 12, seed=n, extra_every=4 if n >= 6 else 0) if n > 1 else []
+    for i in range(100):
+        qs = [int(x) for x in rng.permutation(n)]
+        if n >= 5 and i % 5 == 0:
+            gates.append(("mqu", qs[:5], W.haar_unitary(rng, 32)))
+        elif n >= 2 and i % 3 == 0:
+            gates.append(("cnot", qs[0], qs[1]))
+        else:
+            gates.append(("cu", qs[0], *W.compact_pair(rng)))
+    if n >= 6:
+        gates.insert(40, ("mcu", qs[:5], qs[5], W.haar_unitary(rng, 2)))
+    c = W.build_circuit(gpu, n, gates)
+    gpu.qmxCircuitAddOperation(c, O.CC, ints([0]), 1, 1.0)
+    gpu.qmxCircuitAddOperation(c, O.H, ints([0]), 1, 0.0)
+    assert gpu.qmxCircuitFuse(c, 5) >= 1
+    q, qc = gpu.qureg(n, precision=precision), cpuref.qureg(n)
+    for lib, r in ((gpu, q), (cpuref, qc)):
+        for j in range(n):
+            lib.lib.rotateY(r, j, 0.3 + 0.1 * j)
+    # FP32: each launch (4 an application) and the n rotations round an amplitude once, by
+    # 2^-24; a collapse divides what came before by the root of its probability (> 0.05)
+    tol = 1e-12 if precision is None else 2.0 ** -24 * (n + 8) / 0.05
+    for _ in range(2):
+        W.apply_gates(cpuref, qc, gates)
+        want = cpuref.call("collapseToOutcome", qc, 0, 1)
+        cpuref.call("hadamard", qc, 0)
+        got = gpu.qmxCircuitApply(q, c, 1)
+        assert want > 0.05 and abs(got - want) < tol
+        assert np.max(np.abs(gpu.state(q) - cpuref.state(qc))) < tol
+    gpu.destroy(q)
+    cpuref.destroy(qc)
+    gpu.qmxCircuitDestroy(c)
