@@ -483,3 +483,35 @@ def test_small_registers_in_blocks(gpu, cpuref, n, precision):
     gpu.destroy(q)
     cpuref.destroy(qc)
     gpu.qmxCircuitDestroy(c)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count", [32, 33, 400])
+@pytest.mark.parametrize("precision", [None, QMX_PREC_FP32])
+def test_long_lists_on_two_qubits(gpu, cpuref, count, precision):
+    """Runs of more than 32 gates (none joined: two-qubit ones between one-qubit ones)
+    become one matrix each; a collapse ends a run."""
+    rng = np.random.default_rng(count)
+    two = [O.CX, O.CY, O.CZ, O.CP, O.CRX, O.CRY, O.CRZ]
+    run = []
+    for i in range(count):
+        a = int(rng.integers(2))
+        run.append((int(rng.choice(two)), [a, 1 - a], float(rng.uniform(0, 6))) if i % 2 else
+                   (int(rng.choice([O.H, O.X, O.Y, O.P, O.RX, O.RY, O.RZ])), [a], float(rng.uniform(0, 6))))
+    ops = run + [(O.CC, [0], 1.0), (O.H, [0], 0.0)] + run
+    qc = cpuref.qureg(2)
+    cpuref.lib.rotateY(qc, 0, 0.4)
+    cpuref.lib.rotateX(qc, 1, 1.1)
+    want = O.run_ops(cpuref, qc, ops)
+    ref = cpuref.state(qc)
+    cpuref.destroy(qc)
+    assert want > 0.04
+    # each run and each operation beside it rounds an amplitude once by 2^-24
+    tol = TOL if precision is None else 2.0 ** -24 * 8 / 0.04
+    q = gpu.qureg(2, precision=precision)
+    gpu.lib.rotateY(q, 0, 0.4)
+    gpu.lib.rotateX(q, 1, 1.1)
+    got = gpu.qmxApplyOperations(q, _operation_array(ops), len(ops), None, 2)
+    assert abs(got - want) < tol
+    assert np.max(np.abs(gpu.state(q) - ref)) < tol
+    gpu.destroy(q)
