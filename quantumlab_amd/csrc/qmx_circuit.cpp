@@ -93,6 +93,7 @@ struct Block {
     std::vector<int> gates;     // indices into the operation list, in order
     std::vector<int> targs;     // ascending qubits (targs[0] = LSB of the block matrix)
     std::vector<Cplx> u;        // dense block matrix, row-major
+    void *prepared5 = nullptr;  // its device form for FP32 registers (5 qubits)
     int barrierOp = -1;         // >= 0: this step is the collapse ops[barrierOp]
 };
 
@@ -391,6 +392,7 @@ struct qmxCircuit {
     CircuitSweeps *sweeps[2] = {nullptr, nullptr};  // by storage precision, planned when first needed
     qmxNoiseAfterGate noise{};
     void releaseBlocks() {
+        for (Block &b : blocks) qmx::fused5Free(b.prepared5);
         blocks.clear();
         for (CircuitSweeps *&s : sweeps) {
             if (s) qmx::sweepProgramFree(s->program);
@@ -828,6 +830,11 @@ double applyCircuit(const Qureg &q, qmxCircuit *c, int fused) {
         }
         if (b.gates.size() == 1) {
             runOp(q, c->ops[b.gates[0]]);  // a lone gate keeps its cheaper kernel
+            continue;
+        }
+        if (d->prec == qmx::FP32 && b.targs.size() == 5) {  // more than 12 qubits here
+            if (!b.prepared5) b.prepared5 = qmx::fused5Prepare(b.targs.data(), b.u.data());
+            qmx::fused5Apply(d, b.prepared5);
             continue;
         }
         qmx::applyMatrixN(d, 0, b.targs.data(), (int)b.targs.size(), b.u.data());

@@ -117,8 +117,13 @@ void applyMultiRotateZ(QuregDev *q, uint64_t ctrlMask, uint64_t targMask, double
 void applyMatrixN(QuregDev *q, uint64_t ctrlMask, const int *targs, int k, const Cplx *u);
 // uniformly controlled 2x2: matrix k (4 entries, row-major) where the controls read k
 void applyUniform2(QuregDev *q, const int *controls, int numControls, int target, const Cplx *u);
-// uncontrolled 5-qubit matrix on an FP32 register of >= 9 qubits via MFMA
-// (qmx_fused.hip; staged per call, no allocation)
+// dense 5-qubit block on an FP32 register of >= 11 qubits via MFMA (qmx_fused.hip),
+// prepared once for blocks applied many times
+void *fused5Prepare(const int *targs, const Cplx *u);
+void fused5Free(void *prepared);
+void fused5Apply(QuregDev *q, const void *prepared);
+// uncontrolled 5-qubit matrix on an FP32 register of >= 9 qubits, staged per call, no
+// allocation
 void fused5ApplyOnce(QuregDev *q, const int *targs, const Cplx *u);
 // uncontrolled 5-qubit matrix on an FP64 register of >= 11 qubits (MFMA tiles)
 void fused5ApplyOnce64(QuregDev *q, const int *targs, const Cplx *u);

@@ -515,3 +515,30 @@ def test_long_lists_on_two_qubits(gpu, cpuref, count, precision):
     assert abs(got - want) < tol
     assert np.max(np.abs(gpu.state(q) - ref)) < tol
     gpu.destroy(q)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k", [(13, 6), (14, 7), (16, 6)])
+def test_five_qubit_blocks_of_wider_circuits(gpu, cpuref, n, k):
+    """FP32 circuits fused into blocks of more than 5 qubits keep the device form of the
+    blocks that have exactly 5: applied twice, fused again, applied again."""
+    gates = _edge_gates(n, 60, 70 + n)
+    qc = cpuref.qureg(n)
+    c = W.build_circuit(gpu, n, gates)
+    q = gpu.qureg(n, precision=QMX_PREC_FP32)
+    for lib, r in ((gpu, q), (cpuref, qc)):
+        for j in range(n):
+            lib.lib.rotateY(r, j, 0.3 + 0.1 * j)
+    sizes = []
+    for i in range(3):
+        if i != 1:
+            blocks = gpu.qmxCircuitFuse(c, k)
+            sizes = [gpu.qmxCircuitStep(c, s, None, None, None) for s in range(blocks)]
+        assert 5 in sizes
+        W.apply_gates(cpuref, qc, gates)
+        gpu.qmxCircuitApply(q, c, 1)
+        # as in test_circuits_at_the_edges_of_their_kernels, for i + 1 applications
+        assert np.max(np.abs(gpu.state(q) - cpuref.state(qc))) < 2.0 ** -22 * np.sqrt((i + 1) * len(gates))
+    gpu.destroy(q)
+    cpuref.destroy(qc)
+    gpu.qmxCircuitDestroy(c)
