@@ -92,7 +92,7 @@ struct Block {
     uint64_t mask = 0;          // qubits of the block
     std::vector<int> gates;     // indices into the operation list, in order
     std::vector<int> targs;     // ascending qubits (targs[0] = LSB of the block matrix)
-    std::vector<Cplx> u;        // dense block matrix, row-major
+    std::vector<Cplx> u;        // dense block matrix, row-major; empty until something wants it
     void *prepared5 = nullptr;  // its device form for FP32 registers (5 qubits)
     int barrierOp = -1;         // >= 0: this step is the collapse ops[barrierOp]
 };
@@ -409,10 +409,12 @@ struct qmxCircuit {
 
 namespace {
 
-void buildBlockMatrix(const qmxCircuit &c, Block &b) {
+void listTargets(Block &b) {
     b.targs.clear();
-    for (int q = 0; q < 64; ++q)
-        if ((b.mask >> q) & 1ull) b.targs.push_back(q);
+    for (uint64_t m = b.mask; m; m &= m - 1) b.targs.push_back(__builtin_ctzll(m));
+}
+
+void buildBlockMatrix(const qmxCircuit &c, Block &b) {
     const size_t dim = 1ull << b.targs.size();
     b.u.assign(dim * dim, Cplx{0, 0});
     std::vector<Cplx> col(dim);
@@ -944,9 +946,9 @@ int fuseCircuit(qmxCircuit *c, int maxQubits) {
         seg.push_back(gi);
     }
     fuseSegment(c, seg, maxQubits);
-    // The MFMA kernel applies exactly-5-qubit blocks: pad smaller multi-gate
-    // blocks with identity on extra qubits, taken from the top so the low
-    // qubits stay non-targets (consecutive groups = consecutive addresses).
+    // Blocks of at most 5 qubits are the steps qmxCircuitStep reports; on registers of
+    // 9 qubits and more those of several gates name exactly 5, the extra ones (identity)
+    // from the top. What runs is planned anew (sweepsOf).
     if (maxQubits == 5 && c->numQubits >= 9) {
         for (Block &b : c->blocks) {
             if (b.barrierOp >= 0 || b.gates.size() < 2) continue;
@@ -954,8 +956,14 @@ int fuseCircuit(qmxCircuit *c, int maxQubits) {
                 b.mask |= 1ull << qb;
         }
     }
-    for (Block &b : c->blocks)
-        if (b.barrierOp < 0) buildBlockMatrix(*c, b);
+    // the matrices of blocks that applications read (a lone gate keeps its own kernel);
+    // a step's is formed when it is asked for (qmxCircuitStep)
+    const bool applied = maxQubits != qmx::kSweepBlockQubits && qmx::sweepSupported(c->numQubits);
+    for (Block &b : c->blocks) {
+        if (b.barrierOp >= 0) continue;
+        listTargets(b);
+        if (applied && b.gates.size() > 1) buildBlockMatrix(*c, b);
+    }
     return (int)c->blocks.size();
 }
 
@@ -1109,11 +1117,19 @@ int qmxCircuitStep(const qmxCircuit *c, int step, int *targs, qreal *re, qreal *
     const size_t dim = 1ull << k;
     if (targs)
         for (int j = 0; j < k; ++j) targs[j] = b.targs[j];
-    if (re && im)
-        for (size_t e = 0; e < dim * dim; ++e) {
-            re[e] = (qreal)b.u[e].re;
-            im[e] = (qreal)b.u[e].im;
+    if (re && im) {
+        Block formed;  // of the same gates; a step that runs has its matrix already
+        if (b.u.empty()) {
+            formed.targs = b.targs;
+            formed.gates = b.gates;
+            buildBlockMatrix(*c, formed);
         }
+        const std::vector<Cplx> &u = b.u.empty() ? formed.u : b.u;
+        for (size_t e = 0; e < dim * dim; ++e) {
+            re[e] = (qreal)u[e].re;
+            im[e] = (qreal)u[e].im;
+        }
+    }
     return k;
 }
 
@@ -1135,11 +1151,12 @@ int qmxCircuitSweepBlock(qmxCircuit *c, int precision, int sweep, int block, int
         for (int j = 0; j < sb.k; ++j)
             if (sb.targs[j] < c->numQubits) b.mask |= 1ull << sb.targs[j];
     }
-    buildBlockMatrix(*c, b);
+    listTargets(b);
     const int k = (int)b.targs.size();
     const size_t dim = 1ull << k;
     if (targs)
         for (int j = 0; j < k; ++j) targs[j] = b.targs[j];
+    if (re && im) buildBlockMatrix(*c, b);
     if (re && im)
         for (size_t e = 0; e < dim * dim; ++e) {
             re[e] = (qreal)b.u[e].re;
