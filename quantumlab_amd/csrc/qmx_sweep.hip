@@ -117,7 +117,8 @@ struct BlockDev {
     unsigned rest[4];    // slots of the tile's bits beyond columns and targets: 16-group chunks
 };
 struct BuildDev {
-    int firstGate, numGates, k, pad;
+    int firstGate, numGates, k;
+    unsigned at;         // its vectors' place, in KiB
     // byte offsets of the LDS slots: column bits, combination bits 0 and 1,
     // combinations 4 st
     unsigned col[4], kq[2], st[8];
@@ -126,10 +127,10 @@ struct BuildDev {
 
 // What a lane needs of a block, in 16 B vectors (vector i of all lanes, then i + 1):
 // its operands' LDS slots, one for each step (1 vector for k = 4, 2 for k = 5), then
-// its 3 x 4 or 3 x 16 matrix fragments. Every block has the room of the largest.
-constexpr size_t kBlockBytes = (2 * 16 + 3 * 16 * sizeof(double)) * 64;
+// its 3 x 4 or 3 x 16 matrix fragments; the next block's follow. A vector of all lanes
+// is 1 KiB: a block takes 4 (4 qubits, FP32) to 26 of them.
 template <typename T> constexpr int blockVecs(int k) { return (k == 5 ? 2 : 1) + 3 * (k == 5 ? 16 : 4) * (int)sizeof(T) / 16; }
-static_assert(blockVecs<double>(5) * 1024 <= (int)kBlockBytes, "a block's vectors fit its room");
+constexpr size_t kMaxBlockBytes = (size_t)blockVecs<double>(5) * 1024;
 
 template <typename T> struct Frag;
 template <> struct Frag<float> { typedef f4 V; };
@@ -139,10 +140,11 @@ template <> struct Frag<double> { typedef d2 V; };
 // block's vectors. The gates arrive as the host recorded them, so a list of any
 // length costs one small copy instead of a matrix per block (on the host a block
 // of ten gates took ~25 us). A wave owns a quarter of the matrix's columns, which no
-// other wave touches, so gates follow one another without barriers; each gate is
-// read from LDS while the one before it is applied (scalar loads straight from
-// memory arrive a line at a time, 0.65 us a gate). todo and gates may lie in pinned host
-// memory: each is read once, whole, into LDS.
+// other wave touches, so gates follow one another without barriers (but for those with a
+// matrix of their own, which is staged first); each gate is read from LDS while the one
+// before it is applied (scalar loads straight from memory arrive a line at a time, 0.65
+// us a gate). todo, gates and mats lie in pinned host memory: each is read once, whole,
+// into LDS.
 template <typename T>
 __global__ void __launch_bounds__(kBlock) kBuildBlocks(const BuildDev *__restrict__ todo,
                                                        const GateDev *__restrict__ gates,
@@ -150,6 +152,7 @@ __global__ void __launch_bounds__(kBlock) kBuildBlocks(const BuildDev *__restric
                                                        BlockDev *__restrict__ blocks) {
     __shared__ Amp<double> buf[2][32 * 32];
     __shared__ GateDev stage[kStage + 1];
+    __shared__ Amp<double> U[32 * 32];
     __shared__ BuildDev b;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     static_assert(sizeof(BuildDev) / 4 <= 64, "one load a lane");
@@ -212,7 +215,9 @@ __global__ void __launch_bounds__(kBlock) kBuildBlocks(const BuildDev *__restric
             continue;
         }
         const int gk = G.k, gd = 1 << gk;
-        const Amp<double> *U = mats + G.mat;
+        __syncthreads();  // the last matrix has been read
+        for (int i = tid; i < gd * gd; i += kBlock) U[i] = mats[G.mat + i];
+        __syncthreads();
         for (int r = lane >> cb; r < dim; r += 64 >> cb) {
             Amp<double> s = M[r * dim + col];
             if (((unsigned)r & G.ctrl) == G.ctrl) {
@@ -243,7 +248,7 @@ __global__ void __launch_bounds__(kBlock) kBuildBlocks(const BuildDev *__restric
     __syncthreads();
     // fragment (h steps + st) of each of the three matrices: Ur, Ui, Ur + Ui in FP32,
     // Ur, -(Ur + Ui), Ui - Ur in FP64
-    char *dst = out + (size_t)blockIdx.x * kBlockBytes;
+    char *dst = out + ((size_t)b.at << 10);
     const int steps = dim / 4, frags = (k == 5 ? 2 : 1) * steps;
     unsigned *slots = reinterpret_cast<unsigned *>(dst);
     for (int i = tid; i < steps * 64; i += kBlock) {
@@ -431,7 +436,7 @@ __device__ __forceinline__ void tileBlocks(char *tile, const BlockDev *__restric
     for (int i = 0; i < V4; ++i) pre[i] = next[i * 64];
     for (int b = 0; b < numBlocks; ++b) {
         const V *mineB = next;
-        next += kBlockBytes / sizeof(V);
+        next += (B.k == 5 ? V5 : V4) * 64;
 #pragma unroll
         for (int i = 0; i < V4; ++i) v[i] = pre[i];
         if (b + 1 < numBlocks) {  // the same for the whole workgroup
@@ -650,7 +655,7 @@ Upload layoutOf(const SweepPlan &plan, const FlatGate *gates, int firstBlock, in
 }
 
 void fillBuild(const SweepPlan &plan, const FlatGate *gates, int firstBlock, int numBlocks, const Upload &u,
-               char *host) {
+               const unsigned *place, char *host) {
     BuildDev *todo = reinterpret_cast<BuildDev *>(host + u.todo);
     GateDev *gd = reinterpret_cast<GateDev *>(host + u.gates);
     Amp<double> *mats = reinterpret_cast<Amp<double> *>(host + u.mats);
@@ -661,6 +666,7 @@ void fillBuild(const SweepPlan &plan, const FlatGate *gates, int firstBlock, int
         todo[i].firstGate = at;
         todo[i].numGates = b.numGates;
         todo[i].k = b.k;
+        todo[i].at = place[i];
         auto local = [&](int qubit) {
             for (int j = 0; j < b.k; ++j)
                 if (b.targs[j] == qubit) return j;
@@ -749,17 +755,27 @@ void blockSlots(const SweepBlock &b, const int *pos, int tb, BuildDev &todo) {
         if (!used[i]) todo.tile.rest[r++] = slot(i);
 }
 
-// LDS slots of the blocks that sweeps [first, last) hold
-void fillBlocks(int prec, const SweepPlan &plan, int first, int last, int firstBlock, const Upload &u, char *host) {
+// LDS slots of blocks [firstBlock, firstBlock + num)
+void fillBlocks(int prec, const SweepPlan &plan, int firstBlock, int num, const Upload &u, char *host) {
     BuildDev *todo = reinterpret_cast<BuildDev *>(host + u.todo);
-    for (int s = first; s < last; ++s) {
-        const Sweep &w = plan.sweeps[s];
-        if (w.lone >= 0) continue;
+    for (const Sweep &w : plan.sweeps) {
+        const int from = std::max(w.firstBlock, firstBlock);
+        const int to = std::min(w.firstBlock + w.numBlocks, firstBlock + num);
+        if (w.lone >= 0 || from >= to) continue;
         int pos[kMaxTB];
         const int tb = tilePositions(w.tile, pos);
-        for (int b = w.firstBlock; b < w.firstBlock + w.numBlocks; ++b)
+        for (int b = from; b < to; ++b)
             QMX_DISPATCH(prec, T, { blockSlots<T>(plan.blocks[b], pos, tb, todo[b - firstBlock]); });
     }
+}
+
+// where the vectors of blocks [firstBlock, firstBlock + num) lie, in KiB, and their end
+void placeBlocks(int prec, const SweepPlan &plan, int firstBlock, int num, std::vector<unsigned> &at) {
+    at.resize(num + 1);
+    at[0] = 0;
+    QMX_DISPATCH(prec, T, {
+        for (int i = 0; i < num; ++i) at[i + 1] = at[i] + (unsigned)blockVecs<T>(plan.blocks[firstBlock + i].k);
+    });
 }
 
 // from `src`, an upload that the device can read
@@ -828,7 +844,7 @@ void launchSmallBlocks(QuregDev *q, const Sweep &w, const BlockDev *blocks, cons
 }
 
 void runSweeps(QuregDev *q, const SweepPlan &plan, const FlatGate *gates, int first, int last, int firstBlock,
-               const BlockDev *blocks, const char *frags) {
+               const BlockDev *blocks, const std::vector<unsigned> &place, const char *frags) {
     for (int s = first; s < last; ++s) {
         const Sweep &w = plan.sweeps[s];
         const bool small = smallStateVector(q);
@@ -838,7 +854,7 @@ void runSweeps(QuregDev *q, const SweepPlan &plan, const FlatGate *gates, int fi
             continue;
         }
         const BlockDev *b = blocks + (w.firstBlock - firstBlock);
-        const char *f = frags + (size_t)(w.firstBlock - firstBlock) * kBlockBytes;
+        const char *f = frags + ((size_t)place[w.firstBlock - firstBlock] << 10);
         if (small) launchSmallBlocks(q, w, b, f);
         else QMX_DISPATCH(q->prec, T, { launchSweep<T>(q, w, b, f); });
     }
@@ -861,6 +877,7 @@ struct Workspace {
     int at = 0;
     char *frags = nullptr;
     int fragBlocks = 0;
+    std::vector<unsigned> place;
 
     char *hostRoom(size_t need) {
         at ^= 1;
@@ -884,19 +901,33 @@ struct Workspace {
         if (blocks > fragBlocks) {
             if (frags) devFree(frags);
             fragBlocks = std::max(blocks, 32);
-            frags = static_cast<char *>(devAlloc((size_t)fragBlocks * (kBlockBytes + sizeof(BlockDev))));
+            frags = static_cast<char *>(devAlloc((size_t)fragBlocks * (kMaxBlockBytes + sizeof(BlockDev))));
         }
         return frags;
     }
-    BlockDev *blocks() const { return reinterpret_cast<BlockDev *>(frags + (size_t)fragBlocks * kBlockBytes); }
+    BlockDev *blocks() const { return reinterpret_cast<BlockDev *>(frags + (size_t)fragBlocks * kMaxBlockBytes); }
 } g_ws;
+
+// Blocks [firstBlock, firstBlock + num) on the device: their vectors where `place` says,
+// their descriptions at blocks.
+void buildBatch(int prec, const SweepPlan &plan, const FlatGate *gates, int firstBlock, int num,
+                const unsigned *place, char *frags, BlockDev *blocks) {
+    const Upload u = layoutOf(plan, gates, firstBlock, num);
+    char *host = g_ws.hostRoom(u.bytes);
+    fillBuild(plan, gates, firstBlock, num, u, place, host);
+    fillBlocks(prec, plan, firstBlock, num, u, host);
+    launchBuild(prec, num, u, host, frags, blocks);
+    g_ws.launched();
+}
 
 }  // namespace
 
 struct SweepProgram {
     int prec;
-    char *upload = nullptr, *frags = nullptr;
+    char *frags = nullptr;
+    size_t bytes = 0;
     BlockDev *blocks = nullptr;
+    std::vector<unsigned> place;
 };
 
 SweepProgram *sweepProgramCreate(int prec, const SweepPlan &plan, const FlatGate *gates) {
@@ -904,28 +935,30 @@ SweepProgram *sweepProgramCreate(int prec, const SweepPlan &plan, const FlatGate
     p->prec = prec;
     const int n = (int)plan.blocks.size();
     if (n == 0) return p;
-    const Upload u = layoutOf(plan, gates, 0, n);
-    std::vector<char> host(u.bytes);
-    fillBuild(plan, gates, 0, n, u, host.data());
-    fillBlocks(prec, plan, 0, (int)plan.sweeps.size(), 0, u, host.data());
-    p->upload = static_cast<char *>(devAlloc(u.bytes));
-    hostToDevice(p->upload, host.data(), u.bytes);
-    p->frags = static_cast<char *>(devAlloc((size_t)n * (kBlockBytes + sizeof(BlockDev))));
-    p->blocks = reinterpret_cast<BlockDev *>(p->frags + (size_t)n * kBlockBytes);
-    launchBuild(prec, n, u, p->upload, p->frags, p->blocks);
+    runtimeInit();
+    placeBlocks(prec, plan, 0, n, p->place);
+    const size_t fragBytes = (size_t)p->place[n] << 10;
+    p->bytes = fragBytes + (size_t)n * sizeof(BlockDev);
+    p->frags = static_cast<char *>(poolAlloc(p->bytes));
+    if (!p->frags) {
+        std::fprintf(stderr, "libquest_mi355x: no device memory for a circuit's blocks (%zu bytes)\n", p->bytes);
+        std::abort();
+    }
+    p->blocks = reinterpret_cast<BlockDev *>(p->frags + fragBytes);
+    for (int b = 0; b < n; b += kBatchBlocks)
+        buildBatch(prec, plan, gates, b, std::min(kBatchBlocks, n - b), p->place.data() + b, p->frags, p->blocks + b);
     return p;
 }
 
 void sweepProgramFree(SweepProgram *p) {
     if (!p) return;
-    devFree(p->upload);
-    devFree(p->frags);
+    poolFree(p->frags, p->bytes);
     delete p;
 }
 
 void sweepProgramRun(QuregDev *q, const SweepProgram *p, const SweepPlan &plan, const FlatGate *gates, int first,
                      int last) {
-    runSweeps(q, plan, gates, first, last, 0, p->blocks, p->frags);
+    runSweeps(q, plan, gates, first, last, 0, p->blocks, p->place, p->frags);
 }
 
 void sweepRunOnce(QuregDev *q, const SweepPlan &plan, const FlatGate *gates) {
@@ -944,18 +977,14 @@ void sweepRunOnce(QuregDev *q, const SweepPlan &plan, const FlatGate *gates) {
             ++last;
         }
         if (n == 0) {
-            runSweeps(q, plan, gates, first, last, 0, nullptr, nullptr);
+            runSweeps(q, plan, gates, first, last, 0, nullptr, g_ws.place, nullptr);
             first = last;
             continue;
         }
-        const Upload u = layoutOf(plan, gates, firstBlock, n);
-        char *host = g_ws.hostRoom(u.bytes);
-        fillBuild(plan, gates, firstBlock, n, u, host);
-        fillBlocks(q->prec, plan, first, last, firstBlock, u, host);
         char *frags = g_ws.fragRoom(n);
-        launchBuild(q->prec, n, u, host, frags, g_ws.blocks());
-        g_ws.launched();
-        runSweeps(q, plan, gates, first, last, firstBlock, g_ws.blocks(), frags);
+        placeBlocks(q->prec, plan, firstBlock, n, g_ws.place);
+        buildBatch(q->prec, plan, gates, firstBlock, n, g_ws.place.data(), frags, g_ws.blocks());
+        runSweeps(q, plan, gates, first, last, firstBlock, g_ws.blocks(), g_ws.place, frags);
         first = last;
     }
 }

@@ -542,3 +542,47 @@ def test_five_qubit_blocks_of_wider_circuits(gpu, cpuref, n, k):
     gpu.destroy(q)
     cpuref.destroy(qc)
     gpu.qmxCircuitDestroy(c)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision,most", [(None, 7), (QMX_PREC_FP32, 4)])
+def test_a_planned_circuit_holds_its_blocks_only(gpu, precision, most):
+    """Device memory that a circuit's first application takes and keeps: a 4-qubit block's
+    vectors are 4 KiB in FP32 and 7 in FP64 and its description 20 bytes; the gates are
+    needed while the blocks are built. 2000 blocks and more, and two allocations' slack."""
+    with open("/proc/self/maps") as f:  # the HIP runtime that the library runs on
+        hip = C.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+
+    def free():
+        gpu.qmxSync()
+        f, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(total)) == 0
+        return f.value
+
+    n = 14
+    rng = np.random.default_rng(14)
+    gates = []
+    for i in range(9000):
+        qs = [int(x) for x in rng.choice(n, 2, replace=False)]
+        gates += [("cnot", qs[0], qs[1]), ("cu", qs[0], *W.compact_pair(rng))]
+    c = W.build_circuit(gpu, n, gates)
+    gpu.qmxCircuitFuse(c, 5)
+    small = large = sweep = 0
+    while True:
+        k = gpu.lib.qmxCircuitSweepBlock(c, 0 if precision is None else 1, sweep, 0, None, None, None)
+        if k < 0:
+            break
+        block = 0
+        while k > 0:
+            small, large, block = small + (k <= 4), large + (k == 5), block + 1
+            k = gpu.lib.qmxCircuitSweepBlock(c, 0 if precision is None else 1, sweep, block, None, None, None)
+        sweep += 1
+    assert small > 2000
+    q = gpu.qureg(n, precision=precision)
+    gpu.lib.hadamard(q, 0)
+    before = free()
+    gpu.qmxCircuitApply(q, c, 1)
+    kept = before - free()
+    gpu.destroy(q)
+    gpu.qmxCircuitDestroy(c)
+    assert kept <= small * (most * 1024 + 20) + large * (26 * 1024 + 20) + 2 * (4 << 20)
