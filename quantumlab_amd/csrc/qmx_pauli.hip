@@ -458,6 +458,7 @@ __global__ void __launch_bounds__(kBlock) kPauliCoset(Amp<T> *__restrict__ a, Co
     }
 }
 
+constexpr size_t kStagedRecords = (size_t)16 << 20;
 constexpr int kMaxBlockOps = 1 << 16;  // rotations per block (bounds the host's records only)
 
 // host records of the coset form, before slots and thread bits are known
@@ -822,8 +823,10 @@ void applyPauliSequence(QuregDev *q, const PauliExp *seqIn, int countIn, int rep
         i = j;
     }
     if (blocks.empty()) return;
-    // one upload, through the library's growable staging pair: nothing is
-    // allocated or waited for per call
+    // One upload. Through the library's staging pair a call allocates nothing unless its
+    // records outgrow the pair, and waits for the upload of the call before, which is
+    // queued behind the work before that. The pair is kept, so long sequences (16 MiB are
+    // 350000 FP64 rotations) take an allocation of their own and return it.
     auto align = [](size_t x) { return (x + 63) & ~(size_t)63; };
     const size_t opBytes = coset ? (cops.size() + 1) * (q->prec == FP64 ? sizeof(CosetExpDev<double>)
                                                                         : sizeof(CosetExpDev<float>))
@@ -843,7 +846,12 @@ void applyPauliSequence(QuregDev *q, const PauliExp *seqIn, int countIn, int rep
         if (!ops.empty()) std::memcpy(image.data(), ops.data(), opBytes);
         if (!passes.empty()) std::memcpy(image.data() + groupAt, passes.data(), passes.size() * sizeof(PassDev));
     }
-    const char *dev = static_cast<const char *>(stageLarge(image.data(), bytes, hstream()));
+    char *own = nullptr;
+    if (bytes > kStagedRecords) {
+        own = static_cast<char *>(devAlloc(bytes));
+        hostToDevice(own, image.data(), bytes);
+    }
+    const char *dev = own ? own : static_cast<const char *>(stageLarge(image.data(), bytes, hstream()));
     const PauliExpDev *dOps = reinterpret_cast<const PauliExpDev *>(dev);
     const PassDev *dPasses = reinterpret_cast<const PassDev *>(dev + groupAt);
     const CosetGroupDev *dGroups = reinterpret_cast<const CosetGroupDev *>(dev + groupAt);
@@ -877,6 +885,7 @@ void applyPauliSequence(QuregDev *q, const PauliExp *seqIn, int countIn, int rep
         }
         checkLaunch("applyPauliSequence");
     }
+    devFree(own);  // waits for the launches that read it
 }
 
 int pauliSequenceBlocks(int n, int prec, const PauliExp *seqIn, int countIn) {

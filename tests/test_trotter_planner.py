@@ -394,3 +394,38 @@ def test_fused_trotter_fp32_amplitudes(gpu, n):
             outs.append(gpu.state(q))
             gpu.destroy(q)
         assert np.max(np.abs(outs[0] - outs[1])) < 2e-6, (n, order)
+
+
+@pytest.mark.gpu
+def test_long_sequences_give_their_records_back(gpu):
+    """More than 16 MiB of records (48 B a rotation): the same rotations as a list of one
+    long repetition and as many short ones, and no device memory kept for them."""
+    with open("/proc/self/maps") as f:  # the HIP runtime that the library runs on
+        hip = C.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+
+    def free():
+        gpu.qmxSync()
+        f, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(total)) == 0
+        return f.value
+
+    n = 13
+    inst = H.trotter_instance(n, seed=3, index=0)
+    reps = 380000 // inst.terms
+    states, kept = [], 0
+    for whole in (False, True):
+        if whole:
+            inst.codes = np.tile(inst.codes, (reps, 1))
+            inst.coeffs = np.tile(inst.coeffs, reps)
+        hb = H.HamilBatch([inst])
+        q = gpu.qureg(n)
+        gpu.lib.initPlusState(q)
+        gpu.lib.rotateY(q, 3, 0.7)
+        before = free()
+        gpu.lib.applyTrotterCircuit(q, hb[0], 2.0 / reps if whole else 2.0, 1, 1 if whole else reps)
+        kept = before - free()
+        states.append(gpu.state(q))
+        gpu.destroy(q)
+    # a rotation rounds an amplitude by 2^-53 at most a few times, here in any direction
+    assert np.max(np.abs(states[0] - states[1])) < len(inst.coeffs) * 2.0 ** -53
+    assert kept < 8 << 20
