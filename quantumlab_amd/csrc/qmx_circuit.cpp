@@ -581,9 +581,10 @@ void checkRegister(const qmxCircuit *c, const Qureg &q, const char *f) {
         qv::raise("The circuit and the register have different numbers of qubits.", f);
 }
 
-// the first numOps operations as a gate list; `everyOp`: operations without a
-// matrix form stop the list (they run as the QuEST calls they are), else only
-// collapses do and the others are skipped, as fused application has it
+// the first numOps operations as a state vector's gate list; `everyOp`: operations
+// without a matrix form stop the list (they run as the QuEST calls they are), but for
+// noise, which does nothing there; else only collapses do and the others are skipped,
+// as fused application has it
 GateList gateList(const qmxCircuit *c, int numOps, bool everyOp) {
     GateList l;
     l.gates.reserve(numOps);
@@ -593,7 +594,7 @@ GateList gateList(const qmxCircuit *c, int numOps, bool everyOp) {
         if (o.gate.kind != G_NONE) {
             l.gates.push_back(flatGate(o.gate));
             l.op.push_back(i);
-        } else if (everyOp || o.barrier) {
+        } else if ((everyOp && !isNoise(o.code)) || o.barrier) {
             l.stops.push_back({(int)l.gates.size(), i});
         }
     }

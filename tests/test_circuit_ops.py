@@ -586,3 +586,26 @@ def test_a_planned_circuit_holds_its_blocks_only(gpu, precision, most):
     gpu.destroy(q)
     gpu.qmxCircuitDestroy(c)
     assert kept <= small * (most * 1024 + 20) + large * (26 * 1024 + 20) + 2 * (4 << 20)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [2, 10])
+def test_noise_does_not_cut_a_state_vectors_list(gpu, n):
+    """Noise is ignored on state vectors: an unfused circuit with noise after every gate
+    gives the bits of the circuit without it (FP32 is rounded once a launch, so a list
+    that noise cuts into launches gives others)."""
+    rng = np.random.default_rng(n)
+    states = []
+    gates = [(O.RY if i % 2 else O.RX, int(rng.integers(n)), float(rng.uniform(0, 6))) for i in range(60)]
+    for noisy in (False, True):
+        c = gpu.qmxCircuitCreate(n)
+        for code, target, angle in gates:
+            gpu.qmxCircuitAddOperation(c, code, ints([target]), 1, angle)
+            if noisy:
+                gpu.qmxCircuitAddOperation(c, O.NOISE_DAMPING, ints([target]), 1, 0.1)
+        q = gpu.qureg(n, precision=QMX_PREC_FP32)
+        gpu.qmxCircuitApply(q, c, 0)
+        states.append(gpu.state(q))
+        gpu.destroy(q)
+        gpu.qmxCircuitDestroy(c)
+    assert np.array_equal(states[0], states[1])
