@@ -1247,13 +1247,17 @@ qreal qmxApplyOperations(Qureg qureg, const qmxBasicOperation *ops, int numOps, 
             }
         }
         if (fuseQubits < 0 || fuseQubits > 10) qv::raise(badFuse, __func__);
-        std::vector<Cplx> room;
-        if (c.numQubits == 2 && fuseQubits >= 2) composePairs(l, room);
-        if (small)
-            runSmall(d, l, stop);
-        else
-            runSweepsOnce(d, l, stop);
-        return (qreal)prob;
+        // a fused list without gates and collapses goes on unfused below, where each
+        // undispatched operation says so
+        if (!l.gates.empty() || !l.stops.empty()) {
+            std::vector<Cplx> room;
+            if (c.numQubits == 2 && fuseQubits >= 2) composePairs(l, room);
+            if (small)
+                runSmall(d, l, stop);
+            else
+                runSweepsOnce(d, l, stop);
+            return (qreal)prob;
+        }
     }
     for (int i = 0; i < numOps; ++i)
         recordBasic(&c, ops[i].operation, ops[i].qubits, ops[i].numQubits, (double)ops[i].param, __func__);

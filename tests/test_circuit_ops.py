@@ -609,3 +609,21 @@ def test_noise_does_not_cut_a_state_vectors_list(gpu, n):
         gpu.destroy(q)
         gpu.qmxCircuitDestroy(c)
     assert np.array_equal(states[0], states[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [3, 13])
+@pytest.mark.parametrize("fuse", [0, 3, 5])
+def test_undispatched_operations_say_so(gpu, capfd, n, fuse):
+    """Lists of operations that QuantumLab's loop does not dispatch report each of them,
+    fused or not (QLGate.cpp:652-803); among gates that are fused they are passed over."""
+    libc = C.CDLL(None)
+    q = gpu.qureg(n)
+    for ops, said in (([(O.PHASE, [0], 0.2), (O.PHASE, [1], 0.3)], 2),
+                      ([(O.H, [0], 0.0), (O.PHASE, [0], 0.2)], 0 if fuse else 1)):
+        libc.fflush(None)
+        capfd.readouterr()
+        assert gpu.qmxApplyOperations(q, _operation_array(ops), len(ops), None, fuse) == 1.0
+        libc.fflush(None)
+        assert capfd.readouterr().out.count("not supported type!") == said
+    gpu.destroy(q)
