@@ -627,3 +627,113 @@ def test_undispatched_operations_say_so(gpu, capfd, n, fuse):
         libc.fflush(None)
         assert capfd.readouterr().out.count("not supported type!") == said
     gpu.destroy(q)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,precision", [(21, None), (25, None), (22, QMX_PREC_FP32), (26, QMX_PREC_FP32)])
+def test_tile_sweeps_of_large_registers(gpu, n, precision):
+    """The tile kernel's forms for registers that fill the CUs with four-wave workgroups:
+    the smallest such register, and the smallest that outgrows the last-level cache (whose
+    accesses are nontemporal); a recorded circuit against its gates one by one."""
+    gates = W.brick_circuit(n, 4, seed=n, extra_every=2)
+    a, b = gpu.qureg(n, precision=precision), gpu.qureg(n, precision=precision)
+    for q in (a, b):
+        for j in range(n):
+            gpu.lib.rotateY(q, j, 0.9 + 0.05 * j)
+            gpu.lib.rotateZ(q, j, 0.2 * j)
+    c = W.build_circuit(gpu, n, gates)
+    gpu.qmxCircuitFuse(c, 5)
+    gpu.qmxCircuitApply(a, c, 1)
+    W.apply_gates(gpu, b, gates)
+    # as in test_circuits_at_the_edges_of_their_kernels, for the two paths
+    assert gpu.lib.qmxMaxAbsDiff(a, b) < (1e-12 if precision is None else 2.0 ** -22 * np.sqrt(2 * len(gates)))
+    assert abs(gpu.calcTotalProb(a) - 1) < (1e-12 if precision is None else 2.0 ** -22 * np.sqrt(2 * len(gates)))
+    gpu.destroy(a)
+    gpu.destroy(b)
+    gpu.qmxCircuitDestroy(c)
+
+
+def _mixed_ops(rng, n, count, qubits=None):
+    pool = np.arange(n) if qubits is None else np.array(qubits)
+    ops = []
+    for i in range(count):
+        qs = [int(x) for x in rng.choice(pool, 2, replace=False)]
+        two = i % 3 == 2
+        code = int(rng.choice([O.CX, O.CY, O.CZ, O.CP, O.CRX, O.CRY, O.CRZ] if two else
+                              [O.H, O.X, O.Y, O.Z, O.P, O.RX, O.RY, O.RZ]))
+        ops.append((code, qs if two else qs[:1], float(rng.uniform(0, 6))))
+    return ops
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,precision", [(11, None), (13, None), (12, QMX_PREC_FP32), (13, QMX_PREC_FP32)])
+def test_density_lists_of_large_registers(gpu, n, precision):
+    """The same kernel forms on density registers (22 to 26 row and column bits): a list
+    with noise against the recorded circuit, which composes superoperators call by call."""
+    ops = _mixed_ops(np.random.default_rng(n), n, 40)
+    noise = NoiseAfterGate(damping=0.01, dephasing=0.02, depolarising=0.015)
+    c = gpu.qmxCircuitCreate(n)
+    for code, qs, t in ops:
+        gpu.qmxCircuitAddOperation(c, code, ints(qs), len(qs), t)
+    gpu.qmxCircuitSetNoiseAfterGate(c, noise)
+    a, b = gpu.qureg(n, density=True, precision=precision), gpu.qureg(n, density=True, precision=precision)
+    for q in (a, b):
+        gpu.lib.initPlusState(q)
+        for j in range(n):
+            gpu.lib.rotateX(q, j, 0.3 + 0.1 * j)
+    gpu.qmxApplyOperations(a, _operation_array(ops), len(ops), C.byref(noise), 5)
+    gpu.qmxCircuitApply(b, c, 0)
+    gpu.qmxCircuitDestroy(c)
+    # as in test_density_lists_match_oracle, whose entries reach 1 where these are near 2^-n
+    assert gpu.lib.qmxMaxAbsDiff(a, b) < (TOL if precision is None else 2.0 ** -21 * np.sqrt(len(ops))) * 1e-2
+    assert abs(gpu.calcTotalProb(a) - 1) < (TOL if precision is None else 2.0 ** -21 * np.sqrt(len(ops)))
+    gpu.destroy(a)
+    gpu.destroy(b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,count,qubits,fuse", [
+    (13, 9000, None, 5),                  # more blocks than a batch of the workspace holds (256)
+    (13, 2000, [0, 5, 8, 12], 5),         # one set of 4 qubits: more gates than a block may hold (512) or stages at a time (64)
+    (10, 12000, None, 5), (3, 12000, None, 0)])  # more gates than a launch takes (4096 after joins)
+@pytest.mark.parametrize("precision", [None, QMX_PREC_FP32])
+def test_lists_longer_than_a_launch(gpu, cpuref, n, count, qubits, fuse, precision):
+    ops = _mixed_ops(np.random.default_rng(n + count), n, count, qubits)
+    qc = cpuref.qureg(n)
+    O.run_ops(cpuref, qc, ops)
+    ref = cpuref.state(qc)
+    cpuref.destroy(qc)
+    # every operation rounds an amplitude by a few ulps, in random directions
+    tol = 2.0 ** -51 * np.sqrt(count) * 8 if precision is None else 2.0 ** -22 * np.sqrt(count)
+    q = gpu.qureg(n, precision=precision)
+    gpu.qmxApplyOperations(q, _operation_array(ops), len(ops), None, fuse)
+    assert np.max(np.abs(gpu.state(q) - ref)) < tol
+    gpu.destroy(q)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [12, 13])
+@pytest.mark.parametrize("precision", [None, QMX_PREC_FP32])
+def test_recorded_circuits_of_many_blocks(gpu, cpuref, n, precision):
+    """More blocks than are built at a time (256), some with matrices of their own, in one
+    sweep on 12 qubits and in many on 13."""
+    rng = np.random.default_rng(n)
+    gates = []
+    for i in range(2400):
+        qs = [int(x) for x in rng.permutation(n)]
+        if i % 50 == 0:
+            gates.append(("mqu", qs[:5], W.haar_unitary(rng, 32)))
+        elif i % 3:
+            gates.append(("cu", qs[0], *W.compact_pair(rng)))
+        else:
+            gates.append(("cnot", qs[0], qs[1]))
+    c = W.build_circuit(gpu, n, gates)
+    gpu.qmxCircuitFuse(c, 5)
+    q, qc = gpu.qureg(n, precision=precision), cpuref.qureg(n)
+    W.apply_gates(cpuref, qc, gates)
+    gpu.qmxCircuitApply(q, c, 1)
+    tol = 1e-12 if precision is None else 2.0 ** -22 * np.sqrt(2 * len(gates))
+    assert np.max(np.abs(gpu.state(q) - cpuref.state(qc))) < tol
+    gpu.destroy(q)
+    cpuref.destroy(qc)
+    gpu.qmxCircuitDestroy(c)
