@@ -205,9 +205,10 @@ int qmxCircuitStep(const qmxCircuit *c, int step, int *targs, qreal *re, qreal *
 int qmxCircuitSweepBlock(qmxCircuit *c, int precision, int sweep, int block, int *targs, qreal *re, qreal *im);
 /* Apply to a register of the circuit's width; returns the product of the
  * collapse probabilities (1 without collapses). fused != 0 on a state vector
- * uses the fused blocks (after qmxCircuitFuse), otherwise each operation is the
- * QuEST call PerformBasicOperation makes; density registers always run the
- * operations in order, each followed by the circuit's after-gate noise. */
+ * runs fused (after qmxCircuitFuse), otherwise each operation is the QuEST call
+ * PerformBasicOperation makes, or its gate in the one launch that a state vector
+ * of at most 12 qubits takes; density registers always run the operations in
+ * order, each followed by the circuit's after-gate noise. */
 qreal qmxCircuitApply(Qureg qureg, qmxCircuit *c, int fused);
 /* The simulators' loop over an SBasicOperation list in one call: records ops
  * (validated), fuses into blocks of at most fuseQubits qubits when that is

@@ -6,8 +6,8 @@
 // of others) that absorbs the most gates; inside it, the gates become blocks of 4
 // or 5 qubits, each the window with the most gates for its cost on the matrix
 // cores (a 5-qubit block costs twice a 4-qubit one). On the 30-qubit brick period
-// of five layers (224 gates) this makes 7 sweeps of 24 blocks, worth 12.5 5-qubit
-// blocks of arithmetic, where one sweep per 5-qubit block takes 16 of each.
+// of five layers (230 gates) this makes 6 to 8 sweeps of 24 to 26 blocks, worth 12.5 to
+// 15 5-qubit blocks of arithmetic, where one sweep per 5-qubit block takes 16 of each.
 #include <algorithm>
 
 #include "qmx_sweep.h"
@@ -91,7 +91,7 @@ uint64_t growth(const std::vector<Item> &rem, uint64_t touched, int maxQubits, i
     return best;
 }
 
-// add the lowest (or highest) qubits below n to `mask` until it has k
+// add the lowest qubits below n to `mask` until it has k
 uint64_t padLow(uint64_t mask, int n, int k) {
     for (int b = 0; b < n && popcount(mask) < k; ++b) mask |= 1ull << b;
     return mask;

@@ -1,5 +1,5 @@
 // Batched swap tests for quantum k-means (QKMeans): thousands of registers of
-// uneven size in one persistent launch.
+// uneven size in one launch.
 //
 // Reference construction (QuantumLab): a point v1 and a centroid v2 of length
 // 2^q are amplitude-encoded into q-qubit registers by a tree of uniformly

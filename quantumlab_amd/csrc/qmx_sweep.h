@@ -117,7 +117,7 @@ inline bool smallStateVector(const QuregDev *q) { return !q->isDensity && q->num
 inline bool smallCircuitSupported(const QuregDev *q) {
     return q->numQubits <= (q->isDensity && q->prec == FP64 ? 10 : kSmallCircuitQubits);
 }
-// gates[0 .. count) in order, one launch per few hundred of them; no MATRIXN
+// gates[0 .. count) in order, one launch per 4096 of them; no MATRIXN
 void smallCircuit(QuregDev *q, const FlatGate *gates, int count);
 
 }  // namespace qmx

@@ -20,8 +20,8 @@
 // do; two or three blocks a sweep bring the two to the same time. 4-qubit blocks
 // take half a 5-qubit block's arithmetic and absorb two thirds of its gates, so
 // the planner prefers them. Five-layer brick period, one block a sweep before and
-// now: 30 qubits FP32 50.9 -> 30.2 ms (16 sweeps -> 7, of 25 4-qubit blocks), 27 qubits
-// FP64 12.4 -> 7.2 ms. Seven blocks a sweep keep the matrix cores busy 70 % of the
+// now: 30 qubits FP32 50.7 -> 30.1 ms (16 sweeps -> 6 to 8, of 24 to 26 blocks), 27
+// qubits FP64 12.6 -> 7.0 ms. Seven blocks a sweep keep the matrix cores busy 70 % of the
 // time, two leave it to HBM (3.1 ms for 16 GiB).
 //
 // Operand placement (16x16x4, wave64; lane = 16 kq + col):
@@ -513,9 +513,10 @@ __global__ void __launch_bounds__(64 * WAVES, sizeof(T) == 4 ? 4 : 2)
 // at 12 qubits), one barrier a gate. Nothing but a gate's own chain bounds it (one
 // workgroup): its constants, read from LDS while the gate before it runs, the
 // pair's LDS reads, the products, the writes, the barrier; so the code of a gate is
-// kept short: 0.3 us a gate up to 9 qubits, 0.4 at 10, 0.8 at 12. 80 operations on
-// 10 qubits take 34 us here; as 10 fused blocks of a launch each they took 45 us on
-// the device and 340 us with the host's part of each block.
+// kept short: 0.4 us a gate up to 9 qubits, 0.45 at 10, 0.6 at 11, 0.9 at 12 (2x2s and
+// CNOTs). 80 operations on 10 qubits, 53 gates after joins, take 26 us here; as 10 fused
+// blocks of a launch each they took 45 us on the device and 340 us with the host's part
+// of each block.
 struct SmallGate {
     unsigned what;               // SG_*
     unsigned bit;                // the target's bit, as a byte offset of the LDS register (16 B an amplitude)
