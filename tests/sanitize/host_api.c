@@ -64,7 +64,8 @@ static ComplexMatrix2 hadamardMatrix(void) {
     return u;
 }
 
-/* fusion at every block width, each step read back in full and with NULL outputs */
+/* fusion at every block width, each step and each planned block read back in full and
+ * with NULL outputs */
 static void fuseAtEveryWidth(qmxCircuit *c, int n, int recorded) {
     static qreal bre[1 << 20], bim[1 << 20];
     int targs[64];
@@ -87,6 +88,15 @@ static void fuseAtEveryWidth(qmxCircuit *c, int n, int recorded) {
         }
         CHECK(qmxCircuitStep(c, steps, targs, bre, bim) == -1);
         CHECK(qmxCircuitNumBlocks(c) <= steps);
+        for (int precision = 0; precision < 2; ++precision)
+            for (int sweep = 0, w = 1; w >= 0; ++sweep)
+                for (int block = 0; (w = qmxCircuitSweepBlock(c, precision, sweep, block, targs, bre, bim)) > 0;
+                     ++block) {
+                    CHECK(w <= 5 && w <= n);
+                    for (int i = 1; i < w; ++i) CHECK(targs[i - 1] < targs[i]);
+                    CHECK(targs[0] >= 0 && targs[w - 1] < n);
+                    CHECK(qmxCircuitSweepBlock(c, precision, sweep, block, NULL, NULL, NULL) == w);
+                }
     }
 }
 
