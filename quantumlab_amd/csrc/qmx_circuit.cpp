@@ -22,8 +22,8 @@
 // the register); other block sizes take one sweep a block (qmx::applyMatrixN).
 // State vectors of at most 12 qubits lie in one workgroup's LDS: a fused circuit
 // runs there in blocks of 4 and 5 qubits, a list applied once or unfused gate by
-// gate, in one launch between collapses and gates too wide for it. On density registers, fused
-// application is the unfused sequence: a recorded circuit's operations are the QuEST
+// gate, in one launch between collapses and gates too wide for it. On density
+// registers, fused application is the unfused sequence: a recorded circuit's operations are the QuEST
 // calls, which compose into superoperator sweeps two qubits at a time, and
 // qmxApplyOperations plans its list as gates on the row and column bits.
 //
@@ -681,10 +681,9 @@ struct DensityList {
     }
 };
 
-// On two qubits, every run of more than 32 gates as one matrix, formed here (40 ns a
-// gate where the LDS kernel takes 0.35 us: lists of 60, 400 and 2000 operations, FP32, 25,
-// 35 and 81 us, and 39, 136 and 590 gate by gate); `room`
-// holds the matrices.
+// On two qubits, every run of more than 32 gates as one matrix, formed here and kept in
+// `room`: 40 ns a gate where the LDS kernel takes 0.35 us (FP32 lists of 60, 400 and 2000
+// operations: 25, 35 and 81 us, gate by gate 39, 136 and 590).
 void composePairs(GateList &l, std::vector<Cplx> &room) {
     static const int targs[2] = {0, 1};
     std::vector<FlatGate> out;
